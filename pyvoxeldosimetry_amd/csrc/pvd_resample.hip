@@ -1,10 +1,11 @@
 // Grid-to-grid resampling (nearest / trilinear / cubic B-spline) for the activity
-// <-> kernel resolution round trip of the dose path.  A workgroup writes one output
-// row along z (coalesced stores); the input neighbours of consecutive outputs share
-// cache lines, so the pass is bound by HBM (4 B written per output voxel, input read
-// about once).  Coordinates are formed in FP64 so that equal spacings map every
-// output voxel exactly onto an input voxel.  The cubic B-spline coefficients come
-// from a separable mirror-boundary FIR prefilter (three passes, one per axis).
+// <-> kernel resolution round trip of the dose path.  Linear and cubic interpolation
+// are separable: a workgroup interpolates the input along x once into LDS and writes a
+// tile of output rows from it (resample_staged); nearest, and outputs much coarser than
+// the input, gather each output's neighbours (resample_kernel).  Coordinates are formed
+// in FP64 so that equal spacings map every output voxel exactly onto an input voxel.
+// The cubic B-spline coefficients come from a separable mirror-boundary FIR prefilter
+// (two launches: x, then y and z).
 #include "pvd_internal.h"
 #include "../../include/pvd_resample.h"
 
@@ -142,6 +143,191 @@ __global__ __launch_bounds__(256) void resample_kernel(ResampleArgs a) {
     }
 }
 
+// ---------------------------------------------------------------------------------
+// Separable form of the linear and cubic interpolation.  A workgroup writes a tile of
+// TJ output rows (i, j0 .. j0 + TJ - 1) times KT outputs along z:
+//   1. S[y][z] = the input interpolated along x, for the input rows and columns that
+//      the tile reads (coalesced loads, W per element, shared by the whole tile);
+//   2. cubic only: T[j][z] = S interpolated along y;
+//   3. every output from 2 x 2 values of S (linear) or 4 of T (cubic) in LDS.
+// The gather form above issues 8 (linear) or 64 (cubic) loads per output and is bound
+// by them; here a tile costs W loads per input element it spans, so the cost follows
+// the input samples per output and the pass goes to the HBM stores.  Gather -> staged:
+// 251x251x196 -> 512x512x400 linear 321 -> 155 us (94 at the copy rate), cubic 2139 ->
+// 209; 301x301x233 -> 206x206x160 linear 51 -> 25 us, cubic 283 -> 41 (22).
+constexpr int kRsBlock = 256;      // threads
+constexpr int kRsSpan = 256;       // input columns of a tile (at most)
+constexpr int kRsRows = 8;         // output rows of a tile (at most)
+constexpr int kRsU = 4;            // columns per lane in flight in step 1
+
+struct StagedArgs {
+    ResampleArgs a;
+    int tj, kt;                    // output rows and columns of a tile
+    int njt, nkc;                  // tiles along y and z
+    int span, rows;                // LDS extents: input columns, input rows
+    long long tiles;
+};
+
+template <int W>
+__global__ __launch_bounds__(kRsBlock) void resample_staged(StagedArgs q) {
+    extern __shared__ float rs_lds[];
+    __shared__ float s_wy[kRsRows][4];
+    __shared__ int s_ry[kRsRows][4];     // input rows of an output row (relative to ylo); < 0: outside
+    const ResampleArgs &a = q.a;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    // XCD-contiguous bands of tiles (neighbouring tiles share input rows in one L2)
+    const long long G = gridDim.x;
+    const long long t = (long long)(blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
+    if (t >= q.tiles) return;
+    const int kc = (int)(t % q.nkc);
+    const long long ij = t / q.nkc;
+    const int jt = (int)(ij % q.njt), i = (int)(ij / q.njt);
+    const int j0 = jt * q.tj, nj = min(q.tj, a.m[1] - j0);
+    const int k0 = kc * q.kt, nk = min(q.kt, a.m[2] - k0);
+    float *orow = a.out + ((long long)i * a.m[1] + j0) * a.m[2] + k0;
+    int bx;
+    float fx;
+    // first and last input row and column the tile can touch (mirrored and clamped
+    // neighbours lie within 3 of the base index), 0-filled tiles aside
+    const double cy1 = (j0 + nj - 1) * a.ratio[1], cz1 = (k0 + nk - 1) * a.ratio[2];
+    constexpr int B = W == 4 ? 3 : 1;
+    const int ylo = min(max((int)floor(fmin(j0 * a.ratio[1], 2.0e9)) - (B - 1), 0), a.n[1] - 1);
+    const int yb1 = (int)fmin(floor(cy1), (double)(a.n[1] - 1));
+    const int yhi = min(yb1 + B, a.n[1] - 1);
+    const int zlo = min(max((int)floor(fmin(k0 * a.ratio[2], 2.0e9)) - (B - 1), 0), a.n[2] - 1);
+    const int zhi = min((int)fmin(floor(cz1), (double)(a.n[2] - 1)) + B, a.n[2] - 1);
+    const int ny = min(yhi - ylo + 1, q.rows), nz = min(zhi - zlo + 1, q.span);
+    if (!axis_pos(i * a.ratio[0], a.n[0], bx, fx) || !(j0 * a.ratio[1] < a.n[1] - 0.5)) {
+        for (int jj = 0; jj < nj; ++jj)
+            for (int k = tid; k < nk; k += kRsBlock) orow[(long long)jj * a.m[2] + k] = 0.0f;
+        return;
+    }
+    if (tid < nj) {
+        int b = 0;
+        float f = 0.0f;
+        const bool in = axis_pos((j0 + tid) * a.ratio[1], a.n[1], b, f);
+        float w[4] = {f, 0.0f, 0.0f, 0.0f};
+        if (W == 4) bspline3_weights(f, w);
+#pragma unroll
+        for (int v = 0; v < W; ++v) {
+            const int y = W == 4 ? mirror_index(b - 1 + v, a.n[1]) : min(max(b + v, 0), a.n[1] - 1);
+            s_ry[tid][v] = in ? y - ylo : -1;
+            s_wy[tid][v] = w[v];
+        }
+    }
+    // 1. x: the planes and weights are uniform over the workgroup
+    const float *plane[W];
+    float wx[4];
+    if (W == 4) bspline3_weights(fx, wx);
+#pragma unroll
+    for (int u = 0; u < W; ++u) {
+        const int x = W == 4 ? mirror_index(bx - 1 + u, a.n[0]) : min(max(bx + u, 0), a.n[0] - 1);
+        plane[u] = a.in + (long long)x * a.n[1] * a.n[2];
+    }
+    float *S = rs_lds, *T = rs_lds + (size_t)q.rows * q.span;
+    for (int y = wave; y < ny; y += kRsBlock / 64) {
+        const long long r0 = (long long)(ylo + y) * a.n[2] + zlo;
+        for (int z0 = lane; z0 < nz; z0 += 64 * kRsU) {
+            float v[kRsU][W];
+#pragma unroll
+            for (int c = 0; c < kRsU; ++c)
+#pragma unroll
+                for (int u = 0; u < W; ++u) v[c][u] = plane[u][r0 + min(z0 + 64 * c, nz - 1)];
+#pragma unroll
+            for (int c = 0; c < kRsU; ++c) {
+                float x;
+                if (W == 4) x = fmaf(wx[3], v[c][W - 1], fmaf(wx[2], v[c][W - 2], fmaf(wx[1], v[c][1], wx[0] * v[c][0])));
+                else x = fmaf(fx, v[c][1] - v[c][0], v[c][0]);
+                if (z0 + 64 * c < nz) S[y * q.span + z0 + 64 * c] = x;
+            }
+        }
+    }
+    __syncthreads();
+    // 2. y (cubic)
+    if (W == 4) {
+        for (int jj = wave; jj < nj; jj += kRsBlock / 64) {
+            if (s_ry[jj][0] < 0) continue;
+            const float *s0 = S + s_ry[jj][0] * q.span, *s1 = S + s_ry[jj][1] * q.span;
+            const float *s2 = S + s_ry[jj][2] * q.span, *s3 = S + s_ry[jj][3] * q.span;
+            const float w0 = s_wy[jj][0], w1 = s_wy[jj][1], w2 = s_wy[jj][2], w3 = s_wy[jj][3];
+            for (int z = lane; z < nz; z += 64)
+                T[jj * q.span + z] = fmaf(w3, s3[z], fmaf(w2, s2[z], fmaf(w1, s1[z], w0 * s0[z])));
+        }
+        __syncthreads();
+    }
+    // 3. z, and the stores
+    for (int k = tid; k < nk; k += kRsBlock) {
+        int b = 0;
+        float f = 0.0f;
+        const bool inz = axis_pos((k0 + k) * a.ratio[2], a.n[2], b, f);
+        float wz[4];
+        int z[W];
+        if (W == 4) bspline3_weights(f, wz);
+#pragma unroll
+        for (int v = 0; v < W; ++v) {
+            const int zz = W == 4 ? mirror_index(b - 1 + v, a.n[2]) : min(max(b + v, 0), a.n[2] - 1);
+            z[v] = inz ? zz - zlo : 0;
+        }
+        for (int jj = 0; jj < nj; ++jj) {
+            const int r0 = s_ry[jj][0];
+            float x = 0.0f;
+            if (inz && r0 >= 0) {
+                if (W == 4) {
+                    const float *p = T + jj * q.span;
+                    x = fmaf(wz[3], p[z[W - 1]], fmaf(wz[2], p[z[W - 2]], fmaf(wz[1], p[z[1]], wz[0] * p[z[0]])));
+                } else {
+                    const float *p = S + r0 * q.span, *p1 = S + s_ry[jj][1] * q.span;
+                    const float fy = s_wy[jj][0];
+                    const float e0 = fmaf(fy, p1[z[0]] - p[z[0]], p[z[0]]);
+                    const float e1 = fmaf(fy, p1[z[1]] - p[z[1]], p[z[1]]);
+                    x = fmaf(f, e1 - e0, e0);
+                }
+            }
+            orow[(long long)jj * a.m[2] + k] = a.scale * x;
+        }
+    }
+}
+
+// Largest extent of input indices that `cnt` consecutive outputs touch on an axis of n
+// samples (any start): the kernel's lo .. hi range.
+int staged_extent(double ratio, int cnt, int n, int W) {
+    // (one more than the real numbers need: the products are rounded)
+    const double e = std::floor((cnt - 1) * ratio) + 3.0 + (W == 4 ? 5 : 1);
+    return e < (double)n ? (int)e : n;
+}
+
+// Coarsest output / input spacing (along y and z) that takes the staged form: beyond it
+// a tile spans more input than its outputs use and the gather is faster.  512x512x400
+// inputs, gather / staged us: linear 102 / 97 at 2.04, 38 / 52 at 3.0; cubic 225 / 110 at
+// 3.0, 99 / 72 at 4.5, 32 / 34 at 8.3.
+constexpr double kStagedLinear = 2.5, kStagedCubic = 8.0;
+
+template <int W>
+hipError_t launch_staged(const ResampleArgs &a, hipStream_t st) {
+    StagedArgs q{};
+    q.a = a;
+    // outputs along z whose input columns fit a tile
+    q.kt = a.m[2];
+    if (staged_extent(a.ratio[2], q.kt, a.n[2], W) > kRsSpan) {
+        q.kt = std::max(1, std::min(a.m[2], (int)((kRsSpan - 9) / a.ratio[2])));
+        const int nt = (a.m[2] + q.kt - 1) / q.kt;     // equal tiles
+        q.kt = (a.m[2] + nt - 1) / nt;
+    }
+    q.kt = std::min(q.kt, 2048);
+    q.span = staged_extent(a.ratio[2], q.kt, a.n[2], W);
+    q.tj = kRsRows;
+    while (q.tj > 1 && staged_extent(a.ratio[1], q.tj, a.n[1], W) > 32) q.tj /= 2;
+    q.rows = staged_extent(a.ratio[1], q.tj, a.n[1], W);
+    q.njt = (a.m[1] + q.tj - 1) / q.tj;
+    q.nkc = (a.m[2] + q.kt - 1) / q.kt;
+    q.tiles = (long long)a.m[0] * q.njt * q.nkc;
+    const size_t lds = sizeof(float) * q.span * (size_t)(q.rows + (W == 4 ? q.tj : 0));
+    const long long grid = (q.tiles + 7) / 8 * 8;
+    if (grid > 0x7fffffffLL || q.span > kRsSpan || lds > 48 * 1024) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(resample_staged<W>, dim3((unsigned)grid), dim3(kRsBlock), lds, st, q);
+    return hipGetLastError();
+}
+
 // Cubic B-spline prefilter taps h[k] = sqrt(3) z^k, z = sqrt(3) - 2, k = 0..14 (FP64-built).
 constexpr int kBsK = 14;
 struct BsTaps { float h[kBsK + 1]; };
@@ -153,28 +339,94 @@ constexpr BsTaps bs_taps() {
     return t;
 }
 
-// One axis of the prefilter: dst[i] = sum_{|k| <= 14} h[|k|] src[mirror(i_axis + k)];
-// a thread per element, consecutive threads along z (coalesced on every axis).
-template <int AXIS>
-__global__ __launch_bounds__(256) void bspline_axis_kernel(const float *__restrict__ src, float *__restrict__ dst,
-                                                           int n0, int n1, int n2) {
+// One output of the prefilter, sum_{|k| <= 14} h[|k|] w[k], from a window centred on c.
+template <typename Window>
+__device__ __forceinline__ float bs_fir(const Window &w, int c) {
     constexpr BsTaps T = bs_taps();
-    const long long total = (long long)n0 * n1 * n2;
-    const int n = AXIS == 0 ? n0 : AXIS == 1 ? n1 : n2;
-    const long long stride = AXIS == 0 ? (long long)n1 * n2 : AXIS == 1 ? n2 : 1;
-    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += (long long)gridDim.x * blockDim.x) {
-        const int z = (int)(e % n2);
-        const long long xy = e / n2;
-        const int y = (int)(xy % n1), x = (int)(xy / n1);
-        const int i = AXIS == 0 ? x : AXIS == 1 ? y : z;
-        const float *line = src + (e - (long long)i * stride);
-        float acc = T.h[0] * line[(long long)i * stride];
+    float acc = T.h[0] * w[c];
 #pragma unroll
-        for (int k = 1; k <= kBsK; ++k)
-            acc = fmaf(T.h[k], line[(long long)mirror_index(i - k, n) * stride] +
-                                   line[(long long)mirror_index(i + k, n) * stride], acc);
-        dst[e] = acc;
+    for (int k = 1; k <= kBsK; ++k) acc = fmaf(T.h[k], w[c - k] + w[c + k], acc);
+    return acc;
+}
+
+// The prefilter runs along x in one launch and along y and z in a second (the FIR of
+// each axis is 29 taps, 43 operations: compute stays under the memory time).  A thread
+// owns one column of R consecutive outputs along the filtered axis: R + 28 loads, all
+// issued before the first is used, instead of 29 per output with an index division each
+// in three launches: 301x301x233 1288 -> 146 us (x 49, yz 94), 68 at the copy rate; the
+// yz launch is bound by its FIRs and the LDS round trip.  Same sums in the same order.
+constexpr int kBsX = 48;           // outputs per thread along x
+constexpr int kBsY = 24;           // outputs per thread along y (rows of the z tile)
+constexpr int kBsZ = 14;           // outputs per unit along z
+constexpr int kBsCols = 34 * kBsZ + 2 * kBsK;      // columns of a z tile (at most): 504
+
+__global__ __launch_bounds__(256) void bspline_x(const float *__restrict__ src, float *__restrict__ dst, int n0,
+                                                 long long plane, long long gx) {
+    const long long p = blockIdx.x % gx * 256LL + threadIdx.x;
+    const int x0 = (int)(blockIdx.x / gx) * kBsX;
+    const long long pc = p < plane ? p : plane - 1;
+    float w[kBsX + 2 * kBsK];
+#pragma unroll
+    for (int i = 0; i < kBsX + 2 * kBsK; ++i)
+        w[i] = src[(long long)mirror_index(min(x0 + i - kBsK, n0 - 1 + kBsK), n0) * plane + pc];
+    if (p >= plane) return;
+#pragma unroll
+    for (int i = 0; i < kBsX; ++i)
+        if (x0 + i < n0) dst[(long long)(x0 + i) * plane + p] = bs_fir(w, i + kBsK);
+}
+
+// y in registers, then z through LDS: column c of a tile holds z = mirror(z0 - 14 + c),
+// kBsY rows; phase 2 takes units of 14 consecutive outputs of a row (42 LDS words), puts
+// the results back into the tile and stores whole rows.
+__global__ __launch_bounds__(512) void bspline_yz(const float *__restrict__ src, float *__restrict__ dst, int n1,
+                                                  int n2, int zt, int ld, int nzt, int nyt, long long tiles) {
+    extern __shared__ float tile[];
+    const int tid = threadIdx.x;
+    const int cols = zt + 2 * kBsK;
+    const int upr = zt / kBsZ;                       // units per row
+    const int units = kBsY * upr;                    // at most 2 * blockDim (host)
+    for (long long t = blockIdx.x; t < tiles; t += gridDim.x) {
+        const int z0 = (int)(t % nzt) * zt, y0 = (int)(t / nzt % nyt) * kBsY;
+        const long long base = t / nzt / nyt * n1 * n2;
+        if (tid < cols) {
+            const int z = mirror_index(min(z0 + tid - kBsK, n2 - 1 + kBsK), n2);
+            const float *col = src + base + z;
+            float w[kBsY + 2 * kBsK];
+#pragma unroll
+            for (int i = 0; i < kBsY + 2 * kBsK; ++i)
+                w[i] = col[(long long)mirror_index(min(y0 + i - kBsK, n1 - 1 + kBsK), n1) * n2];
+#pragma unroll
+            for (int i = 0; i < kBsY; ++i) tile[i * ld + tid] = bs_fir(w, i + kBsK);
+        }
+        __syncthreads();
+        float r[2][kBsZ];
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+            const int u = tid + it * (int)blockDim.x;
+            if (u < units) {
+                const float *p = tile + (u / upr) * ld + (u % upr) * kBsZ;
+                float w[3 * kBsZ];
+#pragma unroll
+                for (int i = 0; i < 3 * kBsZ; ++i) w[i] = p[i];
+#pragma unroll
+                for (int i = 0; i < kBsZ; ++i) r[it][i] = bs_fir(w, i + kBsK);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+            const int u = tid + it * (int)blockDim.x;
+            if (u < units) {
+                float *p = tile + (u / upr) * ld + (u % upr) * kBsZ;
+#pragma unroll
+                for (int i = 0; i < kBsZ; ++i) p[i] = r[it][i];
+            }
+        }
+        __syncthreads();
+        const int nz = min(zt, n2 - z0), rows = min(kBsY, n1 - y0);
+        for (int i = 0; i < rows; ++i)
+            for (int c = tid; c < nz; c += blockDim.x) dst[base + (long long)(y0 + i) * n2 + z0 + c] = tile[i * ld + c];
+        __syncthreads();
     }
 }
 
@@ -185,13 +437,24 @@ extern "C" int pvd_bspline_prefilter(const float *in, int n0, int n1, int n2, fl
     if (!in || !coef || !tmp) return pvd_set_error(PVD_EINVAL, "null argument");
     if (n0 < 1 || n1 < 1 || n2 < 1) return pvd_set_error(PVD_EINVAL, "grid extents must be >= 1");
     if (coef == in || tmp == in || coef == tmp) return pvd_set_error(PVD_EINVAL, "coef, tmp and in must differ");
-    const long long total = (long long)n0 * n1 * n2;
-    const unsigned grid = (unsigned)std::min<long long>((total + 255) / 256, 65536);
+    const long long plane = (long long)n1 * n2;
+    const long long gx = (plane + 255) / 256, blocks_x = gx * ((n0 + (long long)kBsX - 1) / kBsX);
+    if (blocks_x > 0x7fffffffLL) return pvd_set_error(PVD_ENOTSUP, "grid too large");
+    const int nyt = (n1 + kBsY - 1) / kBsY;
+    // z tiles of equal width, a multiple of the unit; a thread per column
+    const int nt = (n2 + kBsCols - 2 * kBsK - 1) / (kBsCols - 2 * kBsK);
+    const int zt = ((n2 + nt - 1) / nt + kBsZ - 1) / kBsZ * kBsZ;
+    const int block = (std::max(zt + 2 * kBsK, kBsY * (zt / kBsZ) / 2) + 63) / 64 * 64;
+    const int ld = zt + 2 * kBsK + 1;
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(bspline_axis_kernel<0>, dim3(grid), dim3(256), 0, st, in, coef, n0, n1, n2);
-    hipLaunchKernelGGL(bspline_axis_kernel<1>, dim3(grid), dim3(256), 0, st, (const float *)coef, tmp, n0, n1, n2);
-    hipLaunchKernelGGL(bspline_axis_kernel<2>, dim3(grid), dim3(256), 0, st, (const float *)tmp, coef, n0, n1, n2);
-    const hipError_t e = hipGetLastError();
+    hipLaunchKernelGGL(bspline_x, dim3((unsigned)blocks_x), dim3(256), 0, st, in, tmp, n0, plane, gx);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return pvd_hip_error(e, "launch B-spline prefilter");
+    const int nzt = (n2 + zt - 1) / zt;
+    const long long tiles = (long long)n0 * nyt * nzt;
+    hipLaunchKernelGGL(bspline_yz, dim3((unsigned)std::min<long long>(tiles, 0x7fffffffLL)), dim3(block),
+                       sizeof(float) * kBsY * ld, st, (const float *)tmp, coef, n1, n2, zt, ld, nzt, nyt, tiles);
+    e = hipGetLastError();
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch B-spline prefilter");
 }
 
@@ -217,7 +480,14 @@ extern "C" int pvd_resample(const float *in, int n0, int n1, int n2, const doubl
     if ((long long)m0 * m1 > 0x7fffffffLL) return pvd_set_error(PVD_ENOTSUP, "too many output rows");
     long long g = (long long)m0 * m1;
     if (g > 65536) g = 65536;
-    hipLaunchKernelGGL(resample_kernel, dim3((unsigned)g), dim3(256), 0, (hipStream_t)stream, a);
-    const hipError_t e = hipGetLastError();
+    hipError_t e;
+    if (interp == PVD_INTERP_LINEAR && a.ratio[2] <= kStagedLinear && a.ratio[1] <= kStagedLinear) {
+        e = launch_staged<2>(a, (hipStream_t)stream);
+    } else if (interp == PVD_INTERP_CUBIC && a.ratio[2] <= kStagedCubic && a.ratio[1] <= kStagedCubic) {
+        e = launch_staged<4>(a, (hipStream_t)stream);
+    } else {
+        hipLaunchKernelGGL(resample_kernel, dim3((unsigned)g), dim3(256), 0, (hipStream_t)stream, a);
+        e = hipGetLastError();
+    }
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch resample");
 }

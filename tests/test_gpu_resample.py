@@ -96,3 +96,30 @@ def test_resample_dose_map_shape_affine_and_values():
     np.testing.assert_array_equal(aff, np.diag([0.98, 1.5, 2.0, 1.0]))
     exp = ors.resample(dose, (2.0, 2.0, 2.5), (0.98, 1.5, 2.0), "cubic", shape=shape)
     np.testing.assert_allclose(out, exp, rtol=0, atol=2e-6)
+
+
+@pytest.mark.parametrize("shape,ratio", [
+    ((3, 9, 300), (1.0, 1.0, 1.0)),          # more input columns than one tile
+    ((5, 17, 64), (0.7, 0.31, 0.11)),        # many outputs per input row
+    ((9, 40, 33), (1.3, 2.5, 2.5)),          # the coarsest linear ratio of the staged form
+    ((9, 40, 70), (1.3, 2.51, 2.51)),        # just past it
+    ((6, 64, 90), (1.0, 8.0, 8.0)),          # the coarsest cubic ratio of the staged form
+    ((6, 64, 90), (1.0, 8.01, 8.01)),
+    ((2, 49, 477), (0.9, 1.1, 0.8)),         # prefilter: y tile of 24 + 1, two z tiles
+    ((49, 3, 14), (1.2, 0.5, 1.0)),          # prefilter: x chunk of 48 + 1, one z unit
+    ((97, 25, 15), (0.6, 0.9, 0.77)),
+    ((1, 1, 1), (0.4, 1.0, 3.0)),
+])
+def test_staged_interpolation_edges(shape, ratio):
+    """Tile edges of the staged linear / cubic interpolation and of the B-spline prefilter,
+    and both sides of the rules that choose it.  FP32 sums of at most 29 + 4 terms per axis
+    with FP64 coordinates: linear 1e-6, cubic 2e-6 of max|image|."""
+    from pyvoxeldosimetry_amd.resample import resample
+    _say("staged", shape, ratio)
+    rng = np.random.default_rng(sum(shape))
+    img = rng.normal(size=shape).astype(np.float32)
+    out_shape = tuple(max(1, int(np.ceil(n / r)) + 1) for n, r in zip(shape, ratio))     # past the far edge: zeros
+    for mode, tol in (("linear", 1e-6), ("cubic", 2e-6)):
+        got = resample(img, (1.0, 1.0, 1.0), ratio, mode, output_shape=out_shape, scale=1.0)
+        exp = ors.resample(img, (1.0, 1.0, 1.0), ratio, mode, shape=out_shape)
+        np.testing.assert_allclose(got, exp, rtol=0, atol=tol * np.abs(img).max())

@@ -568,3 +568,26 @@ def test_plain_dose_matches_monte_carlo_in_water():
          f"signed bias {bias:+.4f}")
     assert abs(bias) < 0.005
     assert rel.mean().item() < 0.85 * floor.mean().item()     # noise-limited: ~1/sqrt(2) of the MC-MC spread
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (31, 3), (32, 32), (33, 33), (255, 31), (257, 65), (2049, 32), (256, 1000)])
+def test_reduce_rows_edges(rows, cols):
+    """Column sums around the kernel's 32-column, 32-row-group and 8-load steps; FP32 sums of
+    at most rows terms: |err| <= rows 2^-24 sum|x| (and the accumulate form)."""
+    import ctypes
+
+    import torch
+
+    from pyvoxeldosimetry_amd import _native as nat
+    _say("reduce_rows", rows, cols)
+    lib = nat.load()
+    g = torch.Generator().manual_seed(rows * 1000 + cols)
+    part = torch.randn((rows, cols), generator=g).cuda()
+    out = torch.full((cols,), 2.0, device="cuda")
+    st = ctypes.c_void_p(nat.current_stream_handle())
+    for acc in (0, 1):
+        nat.check(lib.pvd_reduce_rows(ctypes.c_void_p(part.data_ptr()), rows, cols, ctypes.c_void_p(out.data_ptr()), acc,
+                                      st), "pvd_reduce_rows")
+        exp = part.double().sum(0) * (1 + acc)
+        tol = (rows + 2) * 2.0 ** -24 * part.double().abs().sum(0) * (1 + acc)
+        assert bool(((out.double() - exp).abs() <= tol).all())

@@ -591,3 +591,32 @@ def test_reduce_rows_edges(rows, cols):
         exp = part.double().sum(0) * (1 + acc)
         tol = (rows + 2) * 2.0 ** -24 * part.double().abs().sum(0) * (1 + acc)
         assert bool(((out.double() - exp).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("cin", [16, 32])
+@pytest.mark.parametrize("shape", [(1, 1, 32), (2, 4, 32), (3, 5, 96), (5, 9, 32), (34, 35, 64)])
+def test_wgrad_block_edges(cin, shape):
+    """Weight gradient at the edges of its 2 x 4-row blocks (one row, whole blocks, one row
+    past, more blocks than workgroups).  FP32 sums of n products of BF16 values:
+    |err| <= n 2^-24 sum|x||dz|, checked with the products' actual magnitudes."""
+    import ctypes
+
+    import torch
+
+    from pyvoxeldosimetry_amd import _native as nat
+    _say("wgrad edges", cin, shape)
+    lib = nat.load()
+    rng = np.random.default_rng(cin + sum(shape))
+    x = ocnn.bf16_round(rng.normal(size=shape + (cin,)).astype(np.float32))
+    dz = ocnn.bf16_round(rng.normal(size=shape + (32,)).astype(np.float32))
+    work = torch.empty(int(lib.pvd_cnn_wgrad_work_floats(*shape)), dtype=torch.float32, device="cuda")
+    dw = torch.empty(27 * 32 * cin, dtype=torch.float32, device="cuda")
+    xt, dzt = bf(x), bf(dz)
+    nat.check(lib.pvd_cnn_wgrad(ctypes.c_void_p(xt.data_ptr()), cin, ctypes.c_void_p(dzt.data_ptr()),
+                                ctypes.c_void_p(dw.data_ptr()), ctypes.c_void_p(work.data_ptr()), *shape,
+                                ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "wgrad")
+    got = dw.cpu().numpy().reshape(27, 32, cin)
+    exp = ocnn.conv3_weight_grad(x, dz)
+    mag = ocnn.conv3_weight_grad(np.abs(x), np.abs(dz))
+    n = int(np.prod(shape))
+    assert (np.abs(got - exp) <= min(n, 4096) * 2.0 ** -24 * mag + 1e-30).all()

@@ -3,6 +3,8 @@
 // Layout: activations channels-last BF16 [n0][n1][n2][C] (n2 % 32 == 0), weights
 // BF16 [27][32 cout][cin] with tap = (dx+1)*9 + (dy+1)*3 + (dz+1).
 //
+// conv_march residual layers on whole volumes (see there); conv_fwd the other layers and
+//           region lists:
 // conv_fwd  implicit GEMM per output row of 32 voxels along z:
 //           D[32 voxels][32 cout] += A[32 voxels][16 cin] * B[16 cin][32 cout]
 //           with v_mfma_f32_32x32x16_bf16, K-loop over 27 taps x cin/16.
@@ -226,6 +228,202 @@ __global__ __launch_bounds__(FWD_THREADS) void cnn_conv_fwd(ConvArgs a) {
                 } else {
                     a.y32[v * 32 + co] += acc[i];
                 }
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------
+// Residual layer (32 -> 32, y = x + relu(conv(x) + b)) on whole volumes.  A workgroup owns
+// a column of 8 y-rows x 32 z-voxels and marches along x, one plane of outputs per step (a
+// row per wave), over a ring of four input planes in LDS: planes p - 1, p, p + 1 are read
+// while p + 2 arrives, so a step costs one barrier and the waves may drift by a step (one
+// wave's epilogue beside another's MFMAs), and each input plane is read once per column
+// (1.33 times over the volume, against 3.2 for 2 x 4-row blocks).  The weights of MR_REG
+// of the 27 taps stay in registers (two waves per SIMD leave room for them), the others in
+// LDS: MFMAs take fewer LDS reads than the two fragments each would need.
+// Operands are swapped against the kernel above: the weights are A and the voxels B, so a
+// lane holds one voxel's channels in groups of four and the epilogue moves 8 bytes at a
+// time; the accumulation order is the same (same bits).
+// LDS: 16-byte chunk c of weight row R sits in slot c ^ (R >> 2) & 3 of its 64 bytes, of
+// halo voxel (row, hz) in slot c ^ (hz >> 2) & 3: 8 consecutive lanes hit distinct banks
+// without padding, and a fragment address is a lane constant plus an immediate.
+// 128^3 layer 176 -> 115-125 us, 256x256x224 1090 -> 790 us (812 GFLOP at 1.03 PFLOP/s; the
+// one-row kernel above waits at its two barriers a block and for its LDS reads).  Measured
+// at 256x256x224: no tap in registers 842, 9 taps 809, 21 taps 816, 18 taps 790 (reading
+// one or three taps ahead the same); 4 x 4-row blocks, two rows per wave sharing fragments,
+// all weights in LDS 863.
+constexpr int MR_Y = 8, MR_HY = MR_Y + 2;                            // rows of a column, with halo
+constexpr int MR_PITCH = HZ * 64, MR_PLANE = MR_HY * MR_PITCH;       // bytes of a halo row, a plane
+constexpr int MR_WBYTES = 27 * 32 * 64;
+constexpr size_t MR_LDS = (size_t)MR_WBYTES + 4 * MR_PLANE + 8 * FWD_STAGE + 128;
+constexpr int MR_REG = 18, MR_DEPTH = 2;    // taps held in registers; taps read ahead
+constexpr bool mr_in_reg(int t) { return t * MR_REG / 27 != (t + 1) * MR_REG / 27; }
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ u32x4 g_zero_row[64];        // what a halo row outside the volume reads
+
+// two floats to BF16, round to nearest even, in one word
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, bf16x2{(__bf16)lo, (__bf16)hi});
+}
+
+struct MarchArgs {
+    ConvArgs c;
+    int nby, nbz, seg;        // columns along y and z, planes per segment
+    int nseg;
+};
+
+__global__ __launch_bounds__(FWD_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void cnn_conv_march(MarchArgs q) {
+    extern __shared__ uint4 lds_u4[];
+    const ConvArgs &a = q.c;
+    char *lds = reinterpret_cast<char *>(lds_u4);
+    char *wl = lds, *ring = lds + MR_WBYTES;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    char *stg = ring + 4 * MR_PLANE + wave * FWD_STAGE;
+    float *bl = reinterpret_cast<float *>(ring + 4 * MR_PLANE + 8 * FWD_STAGE);
+    for (int i = tid; i < 27 * 32 * 4; i += FWD_THREADS) {
+        const int row = i >> 2, c = i & 3;
+        reinterpret_cast<uint4 *>(wl)[row * 4 + (c ^ ((row >> 2) & 3))] = reinterpret_cast<const uint4 *>(a.w)[i];
+    }
+    if (tid < 32) bl[tid] = a.bias ? a.bias[tid] : 0.0f;
+    const int m = lane & 31, kh = lane >> 5;
+    // Columns: XCD x (workgroups x, x + 8, ...) takes the x-th eighth of them in (segment,
+    // y, z) order, so neighbouring columns share their halo rows in one L2.
+    const int cols = q.nby * q.nbz * q.nseg, per = gridDim.x / 8;
+    const int col = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (col >= cols) return;
+    const int bz = col % q.nbz, by = col / q.nbz % q.nby, x0 = col / (q.nbz * q.nby) * q.seg;
+    const int x1 = min(x0 + q.seg, a.n0), y0 = by * MR_Y, z0 = bz * 32;
+    // A plane's halo: 20 units of 16 voxels (half rows, wave-uniform), waves 0..7 units w and
+    // w + 8, waves 0..3 also 16 + w; then 80 lanes of waves 4 and 5 the rows' end voxels.
+    u32x4 pf[3];
+    const long long plane = (long long)a.n1 * a.n2 * 4;           // 16-byte chunks
+    const u32x4 *xb = reinterpret_cast<const u32x4 *>(a.x);
+    auto unit_off = [&](int u, bool &in) -> long long {
+        const int gy = y0 - 1 + (u >> 1);
+        in = gy >= 0 && gy < a.n1;
+        return ((long long)gy * a.n2 + z0 + (u & 1) * 16) * 4;
+    };
+    auto fetch = [&](int p) {
+        const bool px = p >= 0 && p < a.n0;
+        const u32x4 *xp = xb + p * plane;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            bool in;
+            const long long o = unit_off(wave + 8 * j, in);
+            const u32x4 *s = px && in ? xp + o : g_zero_row;
+            pf[j] = s[lane];
+        }
+        if (wave < 4) {
+            bool in;
+            const long long o = unit_off(wave + 16, in);
+            const u32x4 *s = px && in ? xp + o : g_zero_row;
+            pf[2] = s[lane];
+        } else {
+            const int e = tid - 256, gy = y0 - 1 + (e >> 3), gz = z0 + (e & 4 ? 32 : -1);
+            const bool in = px && e < MR_HY * 8 && gy >= 0 && gy < a.n1 && gz >= 0 && gz < a.n2;
+            const u32x4 *s = in ? xp + ((long long)gy * a.n2 + gz) * 4 + (e & 3) : g_zero_row;
+            pf[2] = *s;
+        }
+    };
+    const int hzp = 1 + (wave & 1) * 16 + (lane >> 2);
+    const int put0 = (wave >> 1) * MR_PITCH + hzp * 64 + (((lane & 3) ^ ((hzp >> 2) & 3)) << 4);
+    int put2;
+    if (wave < 4) {
+        put2 = put0 + 8 * MR_PITCH;
+    } else {
+        const int e = tid - 256, he = e & 4 ? 33 : 0;
+        put2 = (e >> 3) * MR_PITCH + he * 64 + (((e & 3) ^ ((he >> 2) & 3)) << 4);
+    }
+    auto put = [&](int slot) {
+        char *d = ring + slot * MR_PLANE;
+        *reinterpret_cast<u32x4 *>(d + put0) = pf[0];
+        *reinterpret_cast<u32x4 *>(d + put0 + 4 * MR_PITCH) = pf[1];
+        if (wave < 4 || tid < 256 + MR_HY * 8) *reinterpret_cast<u32x4 *>(d + put2) = pf[2];
+    };
+    for (int p = x0 - 1; p <= x0 + 1; ++p) {
+        fetch(p);
+        put(p & 3);
+    }
+    lds_barrier();
+    // lane constants of the fragment addresses, and the register-resident weights
+    int wa[2], xa[3][2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        wa[c] = m * 64 + (((c * 2 + kh) ^ ((m >> 2) & 3)) << 4);
+#pragma unroll
+        for (int dz = 0; dz < 3; ++dz) {
+            const int hz = m + dz;
+            xa[dz][c] = wave * MR_PITCH + hz * 64 + (((c * 2 + kh) ^ ((hz >> 2) & 3)) << 4);
+        }
+    }
+    bf16x8 WR[MR_REG ? MR_REG : 1][2];
+#pragma unroll
+    for (int t = 0; t < 27; ++t)
+        if (mr_in_reg(t)) {
+            WR[t * MR_REG / 27][0] = lds_frag(wl + wa[0] + t * 2048);
+            WR[t * MR_REG / 27][1] = lds_frag(wl + wa[1] + t * 2048);
+        }
+    const int oy = y0 + wave;
+    const bool live = oy < a.n1;         // wave-uniform
+    u32x4 *yb = reinterpret_cast<u32x4 *>(a.y) + ((long long)min(oy, a.n1 - 1) * a.n2 + z0) * 4;
+    for (int p = x0; p < x1; ++p) {
+        // plane p + 1 written by every wave; slot (p + 2) & 3 (plane p - 2) read by every wave
+        if (p > x0) lds_barrier();
+        if (p + 1 < x1) fetch(p + 2);
+        f32x16 acc = {};
+        uint2 rs[4];
+        {
+            constexpr int NS = MR_DEPTH + 1;
+            bf16x8 X[NS][2], W[NS][2];
+            const char *pl[3] = {ring + ((p - 1) & 3) * MR_PLANE, ring + (p & 3) * MR_PLANE, ring + ((p + 1) & 3) * MR_PLANE};
+            auto read = [&](int t) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    X[t % NS][c] = lds_frag(pl[t / 9] + xa[t % 3][c] + t / 3 % 3 * MR_PITCH);
+                    if (!mr_in_reg(t)) W[t % NS][c] = lds_frag(wl + wa[c] + t * 2048);
+                }
+            };
+#pragma unroll
+            for (int t = 0; t < MR_DEPTH; ++t) read(t);
+#pragma unroll
+            for (int t = 0; t < 27; ++t) {
+                if (t + MR_DEPTH < 27) read(t + MR_DEPTH);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(mr_in_reg(t) ? WR[t * MR_REG / 27][c] : W[t % NS][c],
+                                                                  X[t % NS][c], acc, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // skip values: the centre voxel, 4 channels at a time
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int hz = m + 1;
+                rs[g] = *reinterpret_cast<const uint2 *>(pl[1] + (wave + 1) * MR_PITCH + hz * 64 +
+                                                         ((g ^ ((hz >> 2) & 3)) << 4) + kh * 8);
+            }
+        }
+        put((p + 2) & 3);      // (after the last plane it rewrites values that nothing reads)
+        // the row's 32 voxels x 32 channels through the wave's staging, stored as 2 KB
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const float4 bb = *reinterpret_cast<const float4 *>(bl + 8 * g + 4 * kh);
+            const float v0 = bf2f((uint16_t)rs[g].x) + fmaxf(acc[4 * g] + bb.x, 0.0f);
+            const float v1 = bf2f((uint16_t)(rs[g].x >> 16)) + fmaxf(acc[4 * g + 1] + bb.y, 0.0f);
+            const float v2 = bf2f((uint16_t)rs[g].y) + fmaxf(acc[4 * g + 2] + bb.z, 0.0f);
+            const float v3 = bf2f((uint16_t)(rs[g].y >> 16)) + fmaxf(acc[4 * g + 3] + bb.w, 0.0f);
+            *reinterpret_cast<uint2 *>(stg + m * 64 + ((g ^ ((m >> 2) & 3)) << 4) + kh * 8) =
+                make_uint2(pack_bf16(v0, v1), pack_bf16(v2, v3));
+        }
+        if (live) {
+            u32x4 *dst = yb + p * plane;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int v = h * 16 + (lane >> 2);
+                dst[h * 64 + lane] = *reinterpret_cast<const u32x4 *>(stg + v * 64 + (((lane & 3) ^ ((v >> 2) & 3)) << 4));
             }
         }
     }
@@ -886,6 +1084,38 @@ hipError_t launch_fwd(const ConvArgs &a, int blocks, hipStream_t st) {
     return hipGetLastError();
 }
 
+// Segments along x of the marching kernel: the count that minimises the rounds of
+// workgroups times a segment's steps (its planes and about two for the start).
+hipError_t launch_march(const ConvArgs &a, hipStream_t st) {
+    static bool attr = false;
+    if (!attr) {
+        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_march, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)MR_LDS);
+        if (e != hipSuccess) return e;
+        attr = true;
+    }
+    MarchArgs q{};
+    q.c = a;
+    q.nby = (a.n1 + MR_Y - 1) / MR_Y;
+    q.nbz = a.n2 >> 5;
+    const long long cols = (long long)q.nby * q.nbz;
+    long long best = -1;
+    for (int s = 1; s <= a.n0 && s <= 1024; ++s) {
+        const int seg = (a.n0 + s - 1) / s;
+        const long long n = cols * ((a.n0 + seg - 1) / seg);
+        const long long cost = (n + num_cus() - 1) / num_cus() * (seg + 2);
+        if (best < 0 || cost < best) {
+            best = cost;
+            q.seg = seg;
+            q.nseg = (a.n0 + seg - 1) / seg;
+        }
+    }
+    const long long grid = (cols * q.nseg + 7) / 8 * 8;
+    if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(cnn_conv_march, dim3((unsigned)grid), dim3(FWD_THREADS), MR_LDS, st, q);
+    return hipGetLastError();
+}
+
 template <int BX, int BY>
 hipError_t launch_in(const ConvArgs &a, int blocks, hipStream_t st) {
     static bool attr = false;
@@ -997,7 +1227,9 @@ int pvd_cnn_conv_fwd(const void *x, int cin, const void *w, const float *bias, i
     } else {
         switch (epi) {
             case 0: e = launch_fwd<32, 0>(a, grid, st); break;
-            case 1: e = launch_fwd<32, 1>(a, grid, st); break;
+            case 1:
+                e = !blocks && !act && resid == x ? launch_march(a, st) : launch_fwd<32, 1>(a, grid, st);
+                break;
             case 2: e = launch_io<false>(a, grid, blocks == nullptr, st); break;
             default: e = launch_fwd<32, 3>(a, grid, st); break;
         }

@@ -620,3 +620,32 @@ def test_wgrad_block_edges(cin, shape):
     mag = ocnn.conv3_weight_grad(np.abs(x), np.abs(dz))
     n = int(np.prod(shape))
     assert (np.abs(got - exp) <= min(n, 4096) * 2.0 ** -24 * mag + 1e-30).all()
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 32), (2, 8, 32), (3, 9, 64), (5, 17, 96), (33, 7, 32), (300, 8, 32), (70, 41, 64)])
+def test_residual_layer_marching_matches_block_kernel(shape):
+    """Residual layer of a whole volume (columns marching along x) against the block kernel
+    that region lists take, on a list of every block: the same bits (both accumulate in
+    tap order in FP32), at column and segment edges."""
+    import ctypes
+
+    import torch
+
+    from pyvoxeldosimetry_amd import _native as nat
+    _say("residual march", shape)
+    lib = nat.load()
+    n = int(np.prod(shape))
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn((n, 32), generator=g).relu().to(torch.bfloat16).cuda()
+    w = (torch.randn(27 * 32 * 32, generator=g) * 0.05).to(torch.bfloat16).cuda()
+    b = (torch.randn(32, generator=g) * 0.1).cuda()
+    nb = int(lib.pvd_cnn_region_block_count(*shape))
+    blocks = torch.arange(nb, dtype=torch.int32, device="cuda")
+    count = torch.tensor([nb], dtype=torch.int32, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)  # noqa: E731
+    ys = [torch.full((n, 32), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for y, bl, bn in ((ys[0], blocks, count), (ys[1], None, None)):
+        nat.check(lib.pvd_cnn_conv_fwd(p(x), 32, p(w), p(b), nat.PVD_CNN_EPI_RESID_RELU, p(x), p(y), p(None), p(None),
+                                       *shape, p(bl), p(bn), st), "conv")
+    assert torch.equal(ys[0].view(torch.int16), ys[1].view(torch.int16))

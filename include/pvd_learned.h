@@ -85,6 +85,13 @@ int pvd_cnn_conv_fwd(const void *x, int cin, const void *w, const float *bias, i
                      void *y, void *act, float *y32, int n0, int n1, int n2, const int *blocks, const int *nblocks,
                      void *stream);
 
+/* Training forward of a whole volume: the ReLU input layer (cin 4) or a residual layer
+ * y = x + relu(conv(x) + b) (cin 32) as in pvd_cnn_conv_fwd, and mask[v], whose bit c is
+ * set where the BF16 of relu(...) of channel c is not 0 (the activations themselves are
+ * not needed by pvd_cnn_layer_grad).  x and y 16-byte aligned, y not x. */
+int pvd_cnn_train_layer(const void *x, int cin, const void *w, const float *bias, void *y, unsigned *mask, int n0,
+                        int n1, int n2, void *stream);
+
 /* The blocks within the network's 6-voxel receptive field of the region dp >= frac *
  * (*dose_max): block_list receives their indices (in no fixed order) and *nblocks their
  * number, both on the device (no host synchronisation).  flags: int scratch of
@@ -102,6 +109,17 @@ int pvd_cnn_flip_weights(const void *w, void *wt, void *stream);
  * receives per-block channel sums of dz (nblocks = ceil(n / 1024)). */
 int pvd_cnn_relu_grad(const float *dh, const void *act, void *dz, float *dbias_part, long long n_voxels,
                       void *stream);
+
+/* Input gradient of a residual layer and the ReLU gradient of the layer below in one pass:
+ *   dh' = dh_in + conv(dz, w_flipped)   (FP32 [n][32]; dh_in NULL: 0; dh' to dh_out unless
+ *                                        that is NULL; dh_in == dh_out is fine)
+ *   dz_out = bf16(dh' where bit c of mask[v] is set, else 0)
+ *   dbias_part[k][c] = partial channel sums of dz_out before rounding, for
+ *                      k < pvd_cnn_grad_parts(n0, n1, n2) (pvd_reduce_rows sums them)
+ * dz and dz_out must differ. */
+size_t pvd_cnn_grad_parts(int n0, int n1, int n2);
+int pvd_cnn_layer_grad(const void *dz, const void *w_flipped, const float *dh_in, float *dh_out, const unsigned *mask,
+                       void *dz_out, float *dbias_part, int n0, int n1, int n2, void *stream);
 
 /* Weight gradient dw[tap][co][ci] = sum_v x[v + d(tap)][ci] dz[v][co] (FP32),
  * accumulated over voxels in a fixed order (deterministic).  work: FP32 scratch

@@ -23,6 +23,7 @@
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
@@ -55,6 +56,7 @@ struct ConvArgs {
     int n0, n1, n2;
     const int *list;          // blocks to compute (NULL: every block)
     const int *list_n;        // number of entries of list (device)
+    uint32_t *mask;           // ReLU mask, one word per voxel (bit = channel), or NULL
 };
 
 constexpr int FWD_BX = 2, FWD_BY = 4, FWD_THREADS = 512;
@@ -257,8 +259,18 @@ constexpr int MR_Y = 8, MR_HY = MR_Y + 2;                            // rows of 
 constexpr int MR_PITCH = HZ * 64, MR_PLANE = MR_HY * MR_PITCH;       // bytes of a halo row, a plane
 constexpr int MR_WBYTES = 27 * 32 * 64;
 constexpr size_t MR_LDS = (size_t)MR_WBYTES + 4 * MR_PLANE + 8 * FWD_STAGE + 128;
-constexpr int MR_REG = 18, MR_DEPTH = 2;    // taps held in registers; taps read ahead
-constexpr bool mr_in_reg(int t) { return t * MR_REG / 27 != (t + 1) * MR_REG / 27; }
+// The same march runs the input gradient (MR_GRAD*: x is dz, the weights are flipped):
+//   dh' = dh + conv(dz),  dz' = bf16(dh' where the ReLU mask is set),  sum of dz' before
+// rounding per channel, so the ReLU gradient of the layer below costs no pass of its own
+// over dh (128^3: accumulating convolution 360 us + ReLU gradient 165 us before, 128 us
+// now, 106 without a dh input).  Its epilogue needs registers for the dh tile: fewer taps'
+// weights stay there.  The forward writes the ReLU masks (4 bytes a voxel) in place of the
+// activations (64 bytes).
+enum { MR_FWD = 0, MR_MASK, MR_GRAD_FIRST, MR_GRAD, MR_GRAD_LAST };   // MASK: forward and mask;
+                                                                     // FIRST: dh = 0; LAST: dh' not stored
+constexpr int MR_DEPTH = 2;                                              // taps read ahead
+constexpr int mr_regs(int mode) { return mode == MR_FWD ? 18 : mode == MR_MASK ? 15 : 12; }   // taps in registers
+constexpr bool mr_in_reg(int t, int nr) { return t * nr / 27 != (t + 1) * nr / 27; }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 __device__ u32x4 g_zero_row[64];        // what a halo row outside the volume reads
@@ -273,9 +285,16 @@ struct MarchArgs {
     ConvArgs c;
     int nby, nbz, seg;        // columns along y and z, planes per segment
     int nseg;
+    const float *dh_in;       // gradient modes: c.x = dz, c.y = dz', c.mask = the mask
+    float *dh_out;
+    float *part;              // [column][32] sums of dz'
 };
 
+template <int MODE>
 __global__ __launch_bounds__(FWD_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void cnn_conv_march(MarchArgs q) {
+    constexpr int NR = mr_regs(MODE);
+    constexpr bool FWD = MODE == MR_FWD || MODE == MR_MASK;
+    constexpr bool IN = MODE == MR_GRAD || MODE == MR_GRAD_LAST, OUT = MODE == MR_GRAD_FIRST || MODE == MR_GRAD;
     extern __shared__ uint4 lds_u4[];
     const ConvArgs &a = q.c;
     char *lds = reinterpret_cast<char *>(lds_u4);
@@ -359,22 +378,33 @@ __global__ __launch_bounds__(FWD_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
             xa[dz][c] = wave * MR_PITCH + hz * 64 + (((c * 2 + kh) ^ ((hz >> 2) & 3)) << 4);
         }
     }
-    bf16x8 WR[MR_REG ? MR_REG : 1][2];
+    bf16x8 WR[NR][2];
 #pragma unroll
     for (int t = 0; t < 27; ++t)
-        if (mr_in_reg(t)) {
-            WR[t * MR_REG / 27][0] = lds_frag(wl + wa[0] + t * 2048);
-            WR[t * MR_REG / 27][1] = lds_frag(wl + wa[1] + t * 2048);
+        if (mr_in_reg(t, NR)) {
+            WR[t * NR / 27][0] = lds_frag(wl + wa[0] + t * 2048);
+            WR[t * NR / 27][1] = lds_frag(wl + wa[1] + t * 2048);
         }
     const int oy = y0 + wave;
     const bool live = oy < a.n1;         // wave-uniform
-    u32x4 *yb = reinterpret_cast<u32x4 *>(a.y) + ((long long)min(oy, a.n1 - 1) * a.n2 + z0) * 4;
+    const long long row0 = (long long)min(oy, a.n1 - 1) * a.n2 + z0, pvox = (long long)a.n1 * a.n2;
+    u32x4 *yb = reinterpret_cast<u32x4 *>(a.y) + row0 * 4;
+    float bs[FWD ? 1 : 16] = {};
     for (int p = x0; p < x1; ++p) {
         // plane p + 1 written by every wave; slot (p + 2) & 3 (plane p - 2) read by every wave
         if (p > x0) lds_barrier();
         if (p + 1 < x1) fetch(p + 2);
         f32x16 acc = {};
         uint2 rs[4];
+        f32x4 dh[4];                       // this lane's voxel: channels 8 g + 4 kh ..
+        const long long vox = p * pvox + row0 + m;
+        uint32_t mk = 0;
+        if constexpr (!FWD) {
+            mk = a.mask[vox];
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                dh[g] = IN ? reinterpret_cast<const f32x4 *>(q.dh_in)[vox * 8 + 2 * g + kh] : f32x4{};
+        }
         {
             constexpr int NS = MR_DEPTH + 1;
             bf16x8 X[NS][2], W[NS][2];
@@ -383,7 +413,7 @@ __global__ __launch_bounds__(FWD_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
                     X[t % NS][c] = lds_frag(pl[t / 9] + xa[t % 3][c] + t / 3 % 3 * MR_PITCH);
-                    if (!mr_in_reg(t)) W[t % NS][c] = lds_frag(wl + wa[c] + t * 2048);
+                    if (!mr_in_reg(t, NR)) W[t % NS][c] = lds_frag(wl + wa[c] + t * 2048);
                 }
             };
 #pragma unroll
@@ -394,29 +424,54 @@ __global__ __launch_bounds__(FWD_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int c = 0; c < 2; ++c)
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(mr_in_reg(t) ? WR[t * MR_REG / 27][c] : W[t % NS][c],
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(mr_in_reg(t, NR) ? WR[t * NR / 27][c] : W[t % NS][c],
                                                                   X[t % NS][c], acc, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            // skip values: the centre voxel, 4 channels at a time
+            if constexpr (FWD) {
+                // skip values: the centre voxel, 4 channels at a time
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int hz = m + 1;
-                rs[g] = *reinterpret_cast<const uint2 *>(pl[1] + (wave + 1) * MR_PITCH + hz * 64 +
-                                                         ((g ^ ((hz >> 2) & 3)) << 4) + kh * 8);
+                for (int g = 0; g < 4; ++g) {
+                    const int hz = m + 1;
+                    rs[g] = *reinterpret_cast<const uint2 *>(pl[1] + (wave + 1) * MR_PITCH + hz * 64 +
+                                                             ((g ^ ((hz >> 2) & 3)) << 4) + kh * 8);
+                }
             }
         }
         put((p + 2) & 3);      // (after the last plane it rewrites values that nothing reads)
         // the row's 32 voxels x 32 channels through the wave's staging, stored as 2 KB
+        uint32_t bits = 0;
+        if (!FWD) mk = live ? mk >> (4 * kh) : 0u;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const float4 bb = *reinterpret_cast<const float4 *>(bl + 8 * g + 4 * kh);
-            const float v0 = bf2f((uint16_t)rs[g].x) + fmaxf(acc[4 * g] + bb.x, 0.0f);
-            const float v1 = bf2f((uint16_t)(rs[g].x >> 16)) + fmaxf(acc[4 * g + 1] + bb.y, 0.0f);
-            const float v2 = bf2f((uint16_t)rs[g].y) + fmaxf(acc[4 * g + 2] + bb.z, 0.0f);
-            const float v3 = bf2f((uint16_t)(rs[g].y >> 16)) + fmaxf(acc[4 * g + 3] + bb.w, 0.0f);
+            float v[4];
+            if constexpr (FWD) {
+                const float4 bb = *reinterpret_cast<const float4 *>(bl + 8 * g + 4 * kh);
+                const float b4[4] = {bb.x, bb.y, bb.z, bb.w};
+                const uint32_t r2[2] = {rs[g].x, rs[g].y};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float av = fmaxf(acc[4 * g + j] + b4[j], 0.0f);
+                    v[j] = bf2f((uint16_t)(r2[j >> 1] >> (16 * (j & 1)))) + av;
+                    if (MODE == MR_MASK) bits |= av > 0x1p-134f ? 1u << (8 * g + j) : 0u;      // BF16 of av is not 0
+                }
+            } else {
+                f32x4 d = dh[g];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    d[j] += acc[4 * g + j];
+                    v[j] = (mk >> (8 * g + j)) & 1u ? d[j] : 0.0f;
+                    bs[4 * g + j] += v[j];
+                }
+                if (OUT && live) reinterpret_cast<f32x4 *>(q.dh_out)[vox * 8 + 2 * g + kh] = d;
+            }
             *reinterpret_cast<uint2 *>(stg + m * 64 + ((g ^ ((m >> 2) & 3)) << 4) + kh * 8) =
-                make_uint2(pack_bf16(v0, v1), pack_bf16(v2, v3));
+                make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+        }
+        if constexpr (MODE == MR_MASK) {
+            bits <<= 4 * kh;
+            bits |= __shfl_xor(bits, 32);
+            if (live && kh == 0) a.mask[vox] = bits;
         }
         if (live) {
             u32x4 *dst = yb + p * plane;
@@ -425,6 +480,25 @@ __global__ __launch_bounds__(FWD_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
                 const int v = h * 16 + (lane >> 2);
                 dst[h * 64 + lane] = *reinterpret_cast<const u32x4 *>(stg + v * 64 + (((lane & 3) ^ ((v >> 2) & 3)) << 4));
             }
+        }
+    }
+    if constexpr (!FWD) {
+        // channel sums: over the 32 voxels of a lane half, then over the waves in order
+        float *red = reinterpret_cast<float *>(ring + 4 * MR_PLANE);
+        lds_barrier();
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            float v = bs[i];
+#pragma unroll
+            for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o);
+            if (m == 0) red[wave * 32 + 8 * (i >> 2) + 4 * kh + (i & 3)] = v;
+        }
+        lds_barrier();
+        if (tid < 32) {
+            float v = 0.0f;
+#pragma unroll
+            for (int w = 0; w < 8; ++w) v += red[w * 32 + tid];
+            q.part[(size_t)col * 32 + tid] = v;
         }
     }
 }
@@ -469,7 +543,11 @@ __global__ __launch_bounds__(FWD_THREADS) void cnn_conv_in(ConvArgs a) {
     auto block_of = [&](int i) { return a.list ? a.list[i] : i; };
     const int wave = tid >> 6, lane = tid & 63;
     const int m = lane & 31, kh = lane >> 5;
-    const float bco = a.bias ? a.bias[m] : 0.0f;
+    float bias4[4][4];         // channels 8 g + 4 kh + j
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bias4[g][j] = a.bias ? a.bias[8 * g + 4 * kh + j] : 0.0f;
     constexpr int PER_T = (IN_HALO + FWD_THREADS - 1) / FWD_THREADS;
     uint2 pf[PER_T];
     auto fetch = [&](int b) {
@@ -519,19 +597,35 @@ __global__ __launch_bounds__(FWD_THREADS) void cnn_conv_in(ConvArgs a) {
             }
             const bf16x8 fa = __builtin_bit_cast(bf16x8, make_uint4(h[0].x, h[0].y, h[1].x, h[1].y));
             const bf16x8 fb = lds_frag(wl + (c * 32 + m) * IN_WS + kh * 16);
-            if ((c & 1) == 0) acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, fb, acc0, 0, 0, 0);
-            else acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, fb, acc1, 0, 0, 0);
+            // weights as A, voxels as B: a lane holds one voxel's channels in groups of four
+            if ((c & 1) == 0) acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb, fa, acc0, 0, 0, 0);
+            else acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb, fa, acc1, 0, 0, 0);
         }
         const f32x16 acc = acc0 + acc1;
-        // the output tile (32 voxels x 32 channels) staged in the wave's LDS slot as
-        // [row][channel], then written as two 16-byte stores per lane
-        uint16_t *sy = reinterpret_cast<uint16_t *>(stg);
-        const uint4 *src = reinterpret_cast<const uint4 *>(stg);
+        // the output tile (32 voxels x 32 channels) through the wave's LDS slot (16-byte
+        // chunk g of voxel v in slot g ^ (v >> 2) & 3), stored as two 16-byte pieces per lane
+        uint32_t bits = 0;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sy[mfma_row(i, lane) * 32 + m] = f2bf(fmaxf(acc[i] + bco, 0.0f));
+        for (int g = 0; g < 4; ++g) {
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = fmaxf(acc[4 * g + j] + bias4[g][j], 0.0f);
+            const uint32_t lo = pack_bf16(v[0], v[1]), hi = pack_bf16(v[2], v[3]);
+            bits |= ((lo & 0xffffu ? 1u : 0u) | (lo >> 16 ? 2u : 0u) | (hi & 0xffffu ? 4u : 0u) | (hi >> 16 ? 8u : 0u))
+                    << (8 * g);
+            *reinterpret_cast<uint2 *>(stg + m * 64 + ((g ^ ((m >> 2) & 3)) << 4) + kh * 8) = make_uint2(lo, hi);
+        }
+        if (a.mask) {
+            bits <<= 4 * kh;
+            bits |= __shfl_xor(bits, 32);
+            if (kh == 0) a.mask[vrow + m] = bits;
+        }
         uint4 *dst = reinterpret_cast<uint4 *>(a.y + vrow * 32);
-        dst[lane] = src[lane];
-        dst[lane + 64] = src[lane + 64];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int v = h * 16 + (lane >> 2);
+            dst[h * 64 + lane] = *reinterpret_cast<const uint4 *>(stg + v * 64 + (((lane & 3) ^ ((v >> 2) & 3)) << 4));
+        }
         }
     }
 }
@@ -1086,34 +1180,42 @@ hipError_t launch_fwd(const ConvArgs &a, int blocks, hipStream_t st) {
 
 // Segments along x of the marching kernel: the count that minimises the rounds of
 // workgroups times a segment's steps (its planes and about two for the start).
-hipError_t launch_march(const ConvArgs &a, hipStream_t st) {
+void march_plan(MarchArgs *q, int n0, int n1, int n2) {
+    q->nby = (n1 + MR_Y - 1) / MR_Y;
+    q->nbz = n2 >> 5;
+    const long long cols = (long long)q->nby * q->nbz;
+    long long best = -1;
+    for (int s = 1; s <= n0 && s <= 1024; ++s) {
+        const int seg = (n0 + s - 1) / s, nseg = (n0 + seg - 1) / seg;
+        const long long cost = (cols * nseg + num_cus() - 1) / num_cus() * (seg + 2);
+        if (best < 0 || cost < best) {
+            best = cost;
+            q->seg = seg;
+            q->nseg = nseg;
+        }
+    }
+}
+
+template <int MODE>
+hipError_t launch_march(MarchArgs &q, hipStream_t st) {
     static bool attr = false;
     if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_march, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)MR_LDS);
+        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_march<MODE>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)MR_LDS);
         if (e != hipSuccess) return e;
         attr = true;
     }
+    march_plan(&q, q.c.n0, q.c.n1, q.c.n2);
+    const long long grid = ((long long)q.nby * q.nbz * q.nseg + 7) / 8 * 8;
+    if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(cnn_conv_march<MODE>, dim3((unsigned)grid), dim3(FWD_THREADS), MR_LDS, st, q);
+    return hipGetLastError();
+}
+
+hipError_t launch_layer(const ConvArgs &a, hipStream_t st) {
     MarchArgs q{};
     q.c = a;
-    q.nby = (a.n1 + MR_Y - 1) / MR_Y;
-    q.nbz = a.n2 >> 5;
-    const long long cols = (long long)q.nby * q.nbz;
-    long long best = -1;
-    for (int s = 1; s <= a.n0 && s <= 1024; ++s) {
-        const int seg = (a.n0 + s - 1) / s;
-        const long long n = cols * ((a.n0 + seg - 1) / seg);
-        const long long cost = (n + num_cus() - 1) / num_cus() * (seg + 2);
-        if (best < 0 || cost < best) {
-            best = cost;
-            q.seg = seg;
-            q.nseg = (a.n0 + seg - 1) / seg;
-        }
-    }
-    const long long grid = (cols * q.nseg + 7) / 8 * 8;
-    if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(cnn_conv_march, dim3((unsigned)grid), dim3(FWD_THREADS), MR_LDS, st, q);
-    return hipGetLastError();
+    return a.mask ? launch_march<MR_MASK>(q, st) : launch_march<MR_FWD>(q, st);
 }
 
 template <int BX, int BY>
@@ -1210,7 +1312,7 @@ int pvd_cnn_conv_fwd(const void *x, int cin, const void *w, const float *bias, i
         ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(act)) & 15))
         return pvd_set_error(PVD_EINVAL, "y and act must be 16-byte aligned");
     ConvArgs a{(const uint16_t *)x, (const uint16_t *)w, bias, (const uint16_t *)resid, (uint16_t *)y,
-               (uint16_t *)act, y32, n0, n1, n2, blocks, nblocks};
+               (uint16_t *)act, y32, n0, n1, n2, blocks, nblocks, nullptr};
     const long long total = (long long)((n0 + FWD_BX - 1) / FWD_BX) * ((n1 + FWD_BY - 1) / FWD_BY) * (n2 >> 5);
     const int grid = (int)(total < num_cus() ? total : num_cus());
     hipStream_t st = (hipStream_t)stream;
@@ -1228,13 +1330,55 @@ int pvd_cnn_conv_fwd(const void *x, int cin, const void *w, const float *bias, i
         switch (epi) {
             case 0: e = launch_fwd<32, 0>(a, grid, st); break;
             case 1:
-                e = !blocks && !act && resid == x ? launch_march(a, st) : launch_fwd<32, 1>(a, grid, st);
+                e = !blocks && !act && resid == x ? launch_layer(a, st) : launch_fwd<32, 1>(a, grid, st);
                 break;
             case 2: e = launch_io<false>(a, grid, blocks == nullptr, st); break;
             default: e = launch_fwd<32, 3>(a, grid, st); break;
         }
     }
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch CNN convolution");
+}
+
+int pvd_cnn_train_layer(const void *x, int cin, const void *w, const float *bias, void *y, unsigned *mask, int n0,
+                        int n1, int n2, void *stream) {
+    if (int rc = check_grid(n0, n1, n2)) return rc;
+    if (!x || !w || !y || !mask) return pvd_set_error(PVD_EINVAL, "null argument");
+    if (cin != 4 && cin != 32) return pvd_set_error(PVD_EINVAL, "cin must be 4 or 32 (got %d)", cin);
+    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15)
+        return pvd_set_error(PVD_EINVAL, "x and y must be 16-byte aligned");
+    ConvArgs a{(const uint16_t *)x, (const uint16_t *)w, bias, (const uint16_t *)x, (uint16_t *)y, nullptr, nullptr,
+               n0, n1, n2, nullptr, nullptr, mask};
+    hipStream_t st = (hipStream_t)stream;
+    const hipError_t e = cin == 4 ? launch_io<true>(a, 0, true, st) : launch_layer(a, st);
+    return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch CNN training layer");
+}
+
+size_t pvd_cnn_grad_parts(int n0, int n1, int n2) {
+    if (n0 < 1 || n1 < 1 || n2 < 32) return 0;
+    MarchArgs q{};
+    march_plan(&q, n0, n1, n2);
+    return (size_t)q.nby * q.nbz * q.nseg;
+}
+
+int pvd_cnn_layer_grad(const void *dz, const void *w_flipped, const float *dh_in, float *dh_out, const unsigned *mask,
+                       void *dz_out, float *dbias_part, int n0, int n1, int n2, void *stream) {
+    if (int rc = check_grid(n0, n1, n2)) return rc;
+    if (!dz || !w_flipped || !mask || !dz_out || !dbias_part || (!dh_in && !dh_out))
+        return pvd_set_error(PVD_EINVAL, "null argument");
+    if (dz == dz_out) return pvd_set_error(PVD_EINVAL, "dz and dz_out must differ");
+    if ((reinterpret_cast<uintptr_t>(dz) | reinterpret_cast<uintptr_t>(dz_out) | reinterpret_cast<uintptr_t>(dh_in) |
+         reinterpret_cast<uintptr_t>(dh_out)) & 15)
+        return pvd_set_error(PVD_EINVAL, "dz, dz_out, dh_in and dh_out must be 16-byte aligned");
+    MarchArgs q{};
+    q.c = ConvArgs{(const uint16_t *)dz, (const uint16_t *)w_flipped, nullptr, nullptr, (uint16_t *)dz_out, nullptr,
+                   nullptr, n0, n1, n2, nullptr, nullptr, const_cast<unsigned *>(mask)};
+    q.dh_in = dh_in;
+    q.dh_out = dh_out;
+    q.part = dbias_part;
+    hipStream_t st = (hipStream_t)stream;
+    const hipError_t e = !dh_in ? launch_march<MR_GRAD_FIRST>(q, st)
+                         : dh_out ? launch_march<MR_GRAD>(q, st) : launch_march<MR_GRAD_LAST>(q, st);
+    return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch CNN layer gradient");
 }
 
 int pvd_cnn_flip_weights(const void *w, void *wt, void *stream) {

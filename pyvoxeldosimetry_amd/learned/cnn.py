@@ -122,12 +122,14 @@ class ResidualCNN:
             ws = {
                 # zeroed once: a region-restricted forward reads neighbours it did not write
                 "h": [torch.zeros((n, 32), **bf) for _ in range(5)],
-                "act": [None] + [torch.empty((n, 32), **bf) for _ in range(4)],
+                # ReLU masks of layers 0..4, one word of 32 channel bits per voxel
+                "mask": [torch.zeros(n, dtype=torch.int32, device=self.device) for _ in range(5)],
                 "r": torch.zeros(n, dtype=torch.float32, device=self.device),
-                "dz": torch.empty((n, 32), **bf),
+                "dz": [torch.empty((n, 32), **bf) for _ in range(2)],
                 "dr": torch.empty((n, 32), **bf),
                 "dh": torch.empty((n, 32), dtype=torch.float32, device=self.device),
-                "dbias_part": torch.empty(((n + 1023) // 1024, 32), dtype=torch.float32, device=self.device),
+                "dbias_part": torch.empty((int(self.lib.pvd_cnn_grad_parts(*shape)), 32), dtype=torch.float32,
+                                          device=self.device),
                 "wwork": torch.empty(int(self.lib.pvd_cnn_wgrad_work_floats(*shape)), dtype=torch.float32,
                                      device=self.device),
                 "loss_part": torch.empty((256, 3), dtype=torch.float32, device=self.device),
@@ -151,16 +153,23 @@ class ResidualCNN:
     # ------------------------------------------------------------------ forward / backward
     def forward(self, x, shape, keep_activations: bool = True, blocks=None):
         """x: BF16 [n, 16] inputs; returns the FP32 correction r [n] (workspace tensor).
-        ``keep_activations=False`` (inference) skips the ReLU outputs backward needs.
+        ``keep_activations=False`` (inference) skips the ReLU masks backward needs (a
+        whole-volume forward writes them).
         ``blocks``: (block list, count) device tensors from ``pvd_cnn_region_blocks``:
         every layer runs on those blocks only, and r is defined on the region they cover."""
         ws = self._workspace(shape)
         h = ws["h"]
         # the input's channels 4..15 are zero (pvd_cnn_pack): the four-channel input layer
-        self._conv(x, 4, 0, nat.PVD_CNN_EPI_RELU, shape, y=h[0], blocks=blocks)
-        for l in range(1, 5):
-            self._conv(h[l - 1], 32, l, nat.PVD_CNN_EPI_RESID_RELU, shape, y=h[l],
-                       act=ws["act"][l] if keep_activations else None, resid=h[l - 1], blocks=blocks)
+        if keep_activations and blocks is None:
+            for l in range(5):
+                nat.check(self.lib.pvd_cnn_train_layer(_p(x if l == 0 else h[l - 1]), 4 if l == 0 else 32,
+                                                       _p(self.w_bf16(l)), _p(self.bias(l)), _p(h[l]), _p(ws["mask"][l]),
+                                                       shape[0], shape[1], shape[2], self._stream()),
+                          "pvd_cnn_train_layer")
+        else:
+            self._conv(x, 4, 0, nat.PVD_CNN_EPI_RELU, shape, y=h[0], blocks=blocks)
+            for l in range(1, 5):
+                self._conv(h[l - 1], 32, l, nat.PVD_CNN_EPI_RESID_RELU, shape, y=h[l], resid=h[l - 1], blocks=blocks)
         self._conv(h[4], 32, 5, nat.PVD_CNN_EPI_LINEAR_F32, shape, y32=ws["r"], blocks=blocks)
         return ws["r"]
 
@@ -181,8 +190,7 @@ class ResidualCNN:
     def backward(self, x, shape):
         """Gradients of every parameter into self.grad (after forward + loss_and_grad)."""
         ws = self._workspace(shape)
-        n = ws["r"].numel()
-        h, act, dz, dh = ws["h"], ws["act"], ws["dz"], ws["dh"]
+        h, dh, parts = ws["h"], ws["dh"], ws["dbias_part"]
         st = self._stream()
         # layer 5
         nat.check(self.lib.pvd_cnn_wgrad(_p(h[4]), 32, _p(ws["dr"]), _p(self.grad_w(5)), _p(ws["wwork"]),
@@ -190,22 +198,20 @@ class ResidualCNN:
         gb5 = self.grad_b(5)
         gb5.zero_()
         gb5[0:1].copy_(ws["loss_sum"][2:3])
-        dh.zero_()
-        nat.check(self.lib.pvd_cnn_flip_weights(_p(self.w_bf16(5)), _p(self._flip), st), "pvd_cnn_flip_weights")
-        self._conv(ws["dr"], 32, 5, nat.PVD_CNN_EPI_ACCUM_F32, shape, y32=dh, weights=self._flip, bias=False)
+        dz = ws["dr"]
         for l in range(4, -1, -1):
-            a = act[l] if l > 0 else h[0]
-            nat.check(self.lib.pvd_cnn_relu_grad(_p(dh), _p(a), _p(dz), _p(ws["dbias_part"]), n, st),
-                      "pvd_cnn_relu_grad")
-            nat.check(self.lib.pvd_reduce_rows(_p(ws["dbias_part"]), ws["dbias_part"].shape[0], 32,
-                                               _p(self.grad_b(l)), 0, st), "pvd_reduce_rows")
-            xin = x if l == 0 else h[l - 1]
-            nat.check(self.lib.pvd_cnn_wgrad(_p(xin), CIN[l], _p(dz), _p(self.grad_w(l)), _p(ws["wwork"]),
-                                             shape[0], shape[1], shape[2], st), "pvd_cnn_wgrad")
-            if l > 0:
-                nat.check(self.lib.pvd_cnn_flip_weights(_p(self.w_bf16(l)), _p(self._flip), st),
-                          "pvd_cnn_flip_weights")
-                self._conv(dz, 32, l, nat.PVD_CNN_EPI_ACCUM_F32, shape, y32=dh, weights=self._flip, bias=False)
+            # through layer l + 1 to dL/dh_l (kept for the skip connection) and, past the
+            # ReLU of layer l, dz_l and its bias gradient
+            nat.check(self.lib.pvd_cnn_flip_weights(_p(self.w_bf16(l + 1)), _p(self._flip), st), "pvd_cnn_flip_weights")
+            out = ws["dz"][l & 1]
+            nat.check(self.lib.pvd_cnn_layer_grad(_p(dz), _p(self._flip), _p(dh if l < 4 else None),
+                                                  _p(dh if l > 0 else None), _p(ws["mask"][l]), _p(out), _p(parts),
+                                                  shape[0], shape[1], shape[2], st), "pvd_cnn_layer_grad")
+            dz = out
+            nat.check(self.lib.pvd_reduce_rows(_p(parts), parts.shape[0], 32, _p(self.grad_b(l)), 0, st),
+                      "pvd_reduce_rows")
+            nat.check(self.lib.pvd_cnn_wgrad(_p(x if l == 0 else h[l - 1]), CIN[l], _p(dz), _p(self.grad_w(l)),
+                                             _p(ws["wwork"]), shape[0], shape[1], shape[2], st), "pvd_cnn_wgrad")
         # parameters that are structurally zero keep zero gradients
         self.grad_w(0).view(27, 32, 16)[:, :, IN_USED:] = 0.0
         self.grad_w(5).view(27, 32, 32)[:, 1:, :] = 0.0

@@ -649,3 +649,64 @@ def test_residual_layer_marching_matches_block_kernel(shape):
         nat.check(lib.pvd_cnn_conv_fwd(p(x), 32, p(w), p(b), nat.PVD_CNN_EPI_RESID_RELU, p(x), p(y), p(None), p(None),
                                        *shape, p(bl), p(bn), st), "conv")
     assert torch.equal(ys[0].view(torch.int16), ys[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 32), (2, 9, 64), (5, 17, 32), (33, 8, 32), (37, 20, 96)])
+def test_training_layers_and_layer_gradient(shape):
+    """The mask-writing training layers (input and residual) and the marching layer gradient,
+    at column and segment edges, against FP64: y and dz_out to BF16 rounding, dh' to FP32
+    sums of 864 products (1e-4 of max), masks exactly where |z| is clear of zero, bias sums to
+    n 2^-24 of their terms' magnitude."""
+    import ctypes
+
+    import torch
+
+    from pyvoxeldosimetry_amd import _native as nat
+    _say("training layers", shape)
+    lib = nat.load()
+    n = int(np.prod(shape))
+    rng = np.random.default_rng(n)
+    p = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)  # noqa: E731
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def bits(mask):
+        u = mask.cpu().numpy().view(np.uint32).reshape(shape)
+        return (u[..., None] >> np.arange(32, dtype=np.uint32)) & 1
+
+    for cin, cw in ((4, 16), (32, 32)):
+        x = ocnn.bf16_round(rng.normal(size=shape + (cw,)).astype(np.float32))
+        if cin == 4:
+            x[..., 4:] = 0.0
+        w = ocnn.bf16_round(rng.normal(scale=0.1, size=(27, 32, cw)).astype(np.float32))
+        b = rng.normal(scale=0.1, size=32).astype(np.float32)
+        z = ocnn.conv3(x, w) + b
+        y = torch.empty((n, 32), dtype=torch.bfloat16, device="cuda")
+        mask = torch.zeros(n, dtype=torch.int32, device="cuda")
+        xt, wt, bt = bf(x), bf(w), torch.from_numpy(b).cuda()
+        nat.check(lib.pvd_cnn_train_layer(p(xt), cin, p(wt), p(bt), p(y), p(mask), *shape, st), "train layer")
+        exp = np.maximum(z, 0) + (x if cin == 32 else 0.0)
+        np.testing.assert_allclose(y.float().cpu().numpy().reshape(shape + (32,)), exp, rtol=8e-3, atol=1e-3)
+        clear = np.abs(z) > 1e-4
+        np.testing.assert_array_equal(bits(mask)[clear], (z > 0)[clear])
+    dz = ocnn.bf16_round(rng.normal(size=shape + (32,)).astype(np.float32))
+    dh0 = rng.normal(size=shape + (32,)).astype(np.float32)
+    w = ocnn.bf16_round(rng.normal(scale=0.1, size=(27, 32, 32)).astype(np.float32))
+    flip = torch.empty(27 * 32 * 32, dtype=torch.bfloat16, device="cuda")
+    wt, dzt = bf(w), bf(dz)
+    nat.check(lib.pvd_cnn_flip_weights(p(wt), p(flip), st), "flip")
+    mb, grad = bits(mask), ocnn.conv3_input_grad(dz, w)
+    rows = int(lib.pvd_cnn_grad_parts(*shape))
+    for has_in, has_out in ((False, True), (True, True), (True, False)):
+        dh = torch.from_numpy(dh0).cuda().reshape(n, 32).clone()
+        out = torch.full((n, 32), float("nan"), device="cuda") if not has_in else dh
+        dzo = torch.full((n, 32), float("nan"), dtype=torch.bfloat16, device="cuda")
+        part = torch.full((rows, 32), float("nan"), device="cuda")
+        nat.check(lib.pvd_cnn_layer_grad(p(dzt), p(flip), p(dh if has_in else None), p(out if has_out else None), p(mask),
+                                         p(dzo), p(part), *shape, st), "layer grad")
+        exp = grad + (dh0 if has_in else 0.0)
+        if has_out:
+            np.testing.assert_allclose(out.cpu().numpy().reshape(shape + (32,)), exp, rtol=0, atol=1e-4 * np.abs(exp).max())
+        np.testing.assert_allclose(dzo.float().cpu().numpy().reshape(shape + (32,)), exp * mb, rtol=8e-3,
+                                   atol=2e-4 * np.abs(exp).max())
+        np.testing.assert_allclose(part.double().sum(0).cpu().numpy(), (exp * mb).sum((0, 1, 2)), rtol=0,
+                                   atol=1e-4 * np.abs(exp).max() * n ** 0.5 + 1e-6 * (np.abs(exp) * mb).sum((0, 1, 2)).max())

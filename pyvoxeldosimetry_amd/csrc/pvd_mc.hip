@@ -25,6 +25,8 @@
 // block in FP64 and added with FP64 atomics; the deposit map uses FP64 atomics.
 // Random numbers: Philox4x32-10 (Salmon et al., SC'11), counter = (history, draw,
 // stream) with separate streams for the electron and the photons.
+#include <algorithm>
+
 #include "pvd_internal.h"
 
 #include "../../include/pvd_learned.h"
@@ -36,8 +38,10 @@ struct Philox {
     __device__ __forceinline__ static void round(uint32_t &c0, uint32_t &c1, uint32_t &c2, uint32_t &c3, uint32_t k0,
                                                  uint32_t k1) {
         const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u;
-        const uint32_t h0 = __umulhi(M0, c0), l0 = M0 * c0;
-        const uint32_t h1 = __umulhi(M1, c2), l1 = M1 * c2;
+        // one 32 x 32 -> 64-bit product each (v_mad_u64_u32)
+        const uint64_t p0 = (uint64_t)M0 * c0, p1 = (uint64_t)M1 * c2;
+        const uint32_t h0 = (uint32_t)(p0 >> 32), l0 = (uint32_t)p0;
+        const uint32_t h1 = (uint32_t)(p1 >> 32), l1 = (uint32_t)p1;
         const uint32_t n0 = h1 ^ c1 ^ k0, n2 = h0 ^ c3 ^ k1;
         c0 = n0; c1 = l1; c2 = n2; c3 = l0;
     }
@@ -97,9 +101,21 @@ __device__ __forceinline__ float mu_en_of(const MCArgs &a, float e) {
     return table_lerp(a.mu_en, a.n_mu, (__logf(fmaxf(e, 1e-6f)) - a.mu_lo) * a.mu_inv_step);
 }
 
+constexpr int MC_BLOCK = 256;
+constexpr int MC_REFILL = 40;      // lanes without a spare history before a wave starts new ones
+constexpr int MC_WAVES = 20;       // waves per CU (five per SIMD fit)
+// Grids of at most this many voxels (80 KB of FP64: two workgroups per CU) are tallied in
+// LDS and added to the map once per workgroup.  Point kernels put every history into a few
+// voxels, whose global atomics queue: 2^21 histories on 13^3 68.2 -> 0.38 ms, 2^20 on 21^3
+// 18.0 -> 0.13 ms; a 15x12x9 map, 64 histories a voxel, 188 -> 81 us.
+constexpr long long kMcTileVoxels = 10000;
+
 // One photon packet carrying energy e (absorbed with mu_en at energy e_mu) and weight w
 // from position p (voxel units) along the unit direction d: exact voxel traversal,
-// kerma deposits; adds to the deposited and escaped totals.
+// kerma deposits; adds to the deposited and escaped totals.  The next voxel's density is
+// requested before the current deposit: a load's wait covers the memory operations issued
+// before it, so one issued after the atomic would wait for the atomic's round trip.
+template <typename I>
 __device__ void photon_packet(const MCArgs &a, const float *__restrict__ dens, double *__restrict__ edep, float px,
                               float py, float pz, float dx, float dy, float dz, float e, float e_mu, float w,
                               double &dep_tot, double &esc_tot) {
@@ -117,21 +133,29 @@ __device__ void photon_packet(const MCArgs &a, const float *__restrict__ dens, d
     float t = 0.0f, erem = e;
     const float e_stop = 1e-6f * e;
     const int max_steps = a.n[0] + a.n[1] + a.n[2] + 3;     // a straight ray crosses each plane once
+    auto inside = [&]() { return ix >= 0 && iy >= 0 && iz >= 0 && ix < a.n[0] && iy < a.n[1] && iz < a.n[2]; };
+    auto index = [&]() { return ((I)ix * (I)a.n[1] + (I)iy) * (I)a.n[2] + (I)iz; };
+    bool in = inside();
+    I vox = in ? index() : (I)0;
+    float rho_raw = dens ? dens[vox] : 1.0f;
     for (int step = 0; step < max_steps; ++step) {
-        if (ix < 0 || iy < 0 || iz < 0 || ix >= a.n[0] || iy >= a.n[1] || iz >= a.n[2] || erem <= e_stop) break;
+        if (!in || erem <= e_stop) break;
         const float tn = fminf(tmx, fminf(tmy, tmz));
-        const long long vox = ((long long)ix * a.n[1] + iy) * a.n[2] + iz;
-        const float rho = fmaxf(dens ? dens[vox] : 1.0f, a.rho_min_ph);
+        const I here = vox;
+        const float rho = fmaxf(rho_raw, a.rho_min_ph);
         const float dep = erem * (1.0f - __expf(-mu_mm * rho * (tn - t) * voxel_mm));
-        if (dep > 0.0f) {
-            atomicAdd(&edep[vox], (double)(w * dep));
-            dep_tot += (double)w * dep;
-            erem -= dep;
-        }
         t = tn;
         if (tn == tmx) { ix += sx; tmx += tdx; }
         else if (tn == tmy) { iy += sy; tmy += tdy; }
         else { iz += sz; tmz += tdz; }
+        in = inside();
+        vox = in ? index() : (I)0;
+        rho_raw = dens ? dens[vox] : 1.0f;
+        if (dep > 0.0f) {
+            atomicAdd(&edep[here], (double)(w * dep));
+            dep_tot += (double)w * dep;
+            erem -= dep;
+        }
     }
     esc_tot += (double)w * erem;
 }
@@ -150,116 +174,48 @@ __device__ __forceinline__ float range_of(const MCArgs &a, float e) {
     return 10.0f * a.ka * __powf(e, a.kb - a.kc * __logf(e));
 }
 
-__global__ __launch_bounds__(256) void pvd_mc_kernel(MCArgs a, const float *__restrict__ act,
-                                                     const float *__restrict__ dens, double *__restrict__ edep,
-                                                     double *__restrict__ totals) {
-    __shared__ double red[3][256 / 64];
-    const long long nvox = (long long)a.n[0] * a.n[1] * a.n[2];
-    const long long tid = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    const long long src = tid / a.histories;
-    long long v = -1;
-    if (src < a.n_src) v = a.active ? a.active[src] : src;
-    double emitted = 0.0, escaped = 0.0, deposited = 0.0;
-    if (v >= 0 && v < nvox && act[v] > 0.0f) {
-        const float w = act[v] / (float)a.histories;
-        const Philox rng{a.seed_lo, a.seed_hi};
-        const uint32_t hid_lo = (uint32_t)tid, hid_hi = (uint32_t)(tid >> 32);
-        uint32_t draw = 0;
-        uint4 r4 = rng(hid_lo, hid_hi, draw++, 0x5eedu);
-        const int vz = (int)(v % a.n[2]);
-        const int vy = (int)((v / a.n[2]) % a.n[1]);
-        const int vx = (int)(v / ((long long)a.n[2] * a.n[1]));
-        // position in voxel units, uniform inside the emitting voxel
-        float px = (float)vx + u01(r4.x), py = (float)vy + u01(r4.y), pz = (float)vz + u01(r4.z);
-        const float px0 = px, py0 = py, pz0 = pz;
-        float e0 = table_lerp(a.e_of_u, a.n_u, u01(r4.w) * (float)(a.n_u - 1));
-        r4 = rng(hid_lo, hid_hi, draw++, 0x5eedu);
-        float dx, dy, dz;
-        iso_dir(r4.x, r4.y, dx, dy, dz);
-        float r = fminf(range_of(a, e0), a.r_max);
-        const float r0 = fmaxf(r, 1e-6f);
-        const float dr = a.r_max / (float)(a.n_r - 1);
-        const float inv_dr = 1.0f / dr;
-        float e_cur = table_lerp(a.e_of_r, a.n_r, r * inv_dr);
-        const float e_start = e_cur;
-        // thick-target bremsstrahlung: the electron keeps (1 - Y) of its losses
-        float yb = 0.0f;
-        if (a.brems_z > 0.0f) {
-            const float x = 6.0e-4f * a.brems_z * e_start;
-            yb = x / (1.0f + x);
-        }
-        const float keep = 1.0f - yb;
-        if (a.electrons) emitted = (double)w * keep * e_cur;
-        // photon packets of every photon_every-th history of this voxel, weight x photon_every
-        const int hist = (int)(tid - src * a.histories);
-        if (hist % a.photon_every == 0 && (a.n_lines > 0 || yb > 0.0f)) {
-            const float wp = w * (float)a.photon_every;
-            uint32_t pd = 0;
-            for (int l = 0; l < a.n_lines; ++l) {
-                const uint4 q = rng(hid_lo, hid_hi, pd++, 0xf07u);
-                float qx, qy, qz;
-                iso_dir(q.x, q.y, qx, qy, qz);
-                const float wl = wp * a.line_y[l];
-                emitted += (double)wl * a.line_e[l];
-                photon_packet(a, dens, edep, px0, py0, pz0, qx, qy, qz, a.line_e[l], a.line_e[l], wl, deposited,
-                              escaped);
-            }
-            if (yb > 0.0f) {
-                const uint4 q = rng(hid_lo, hid_hi, pd++, 0xf07u);
-                float qx, qy, qz;
-                iso_dir(q.x, q.y, qx, qy, qz);
-                const float k = fmaxf(e_start * (1.0f - sqrtf(u01(q.z))), 1e-3f);    // energy spectrum ~ (E0 - k)
-                const float eb = yb * e_start;
-                emitted += (double)wp * eb;
-                // the packet carries Y E0 and is absorbed with mu_en at its sampled energy k
-                photon_packet(a, dens, edep, px0, py0, pz0, qx, qy, qz, eb, k, wp, deposited, escaped);
-            }
-        }
-        int guard = 0;
-        while (a.electrons && r > 0.0f && guard++ < 100000) {
-            const int ix = (int)floorf(px), iy = (int)floorf(py), iz = (int)floorf(pz);
-            if (ix < 0 || iy < 0 || iz < 0 || ix >= a.n[0] || iy >= a.n[1] || iz >= a.n[2]) {
-                escaped += (double)w * keep * e_cur;
-                break;
-            }
-            const long long vox = ((long long)ix * a.n[1] + iy) * a.n[2] + iz;
-            const float rho = fmaxf(dens ? dens[vox] : 1.0f, a.rho_min);
-            const float s = fminf(fminf(a.step_mm, r), a.half_voxel_mm * rho);   // water-equivalent mm
-            r = fmaxf(r - s, 0.0f);
-            const float e_next = r > 0.0f ? table_lerp(a.e_of_r, a.n_r, r * inv_dr) : 0.0f;
-            const float de = keep * (e_cur - e_next);
-            atomicAdd(&edep[vox], (double)(w * de));
-            deposited += (double)w * de;
-            e_cur = e_next;
-            const float len = (s / rho) * a.inv_voxel;   // geometric step in voxel units
-            px = fmaf(dx, len, px);
-            py = fmaf(dy, len, py);
-            pz = fmaf(dz, len, pz);
-            // Gaussian deflection about the current direction
-            r4 = rng(hid_lo, hid_hi, draw++, 0x5eedu);
-            const float g = sqrtf(-2.0f * __logf(u01(r4.x))) * __cosf(6.28318530718f * u01(r4.y));
-            const float th = a.scatter * sqrtf(s / r0) * g;
-            float st, ct, sp, cp;
-            __sincosf(th, &st, &ct);
-            __sincosf(6.28318530718f * u01(r4.z), &sp, &cp);
-            // orthonormal frame (e1, e2) perpendicular to d
-            float e1x, e1y, e1z;
-            if (fabsf(dz) < 0.9f) {            // e1 = normalize(d x z)
-                const float inv = rsqrtf(dx * dx + dy * dy);
-                e1x = dy * inv; e1y = -dx * inv; e1z = 0.0f;
-            } else {                            // e1 = normalize(d x x)
-                const float inv = rsqrtf(dy * dy + dz * dz);
-                e1x = 0.0f; e1y = dz * inv; e1z = -dy * inv;
-            }
-            const float e2x = dy * e1z - dz * e1y, e2y = dz * e1x - dx * e1z, e2z = dx * e1y - dy * e1x;
-            const float nx = ct * dx + st * (cp * e1x + sp * e2x);
-            const float ny = ct * dy + st * (cp * e1y + sp * e2y);
-            const float nz = ct * dz + st * (cp * e1z + sp * e2z);
-            const float inv = rsqrtf(nx * nx + ny * ny + nz * nz);
-            dx = nx * inv; dy = ny * inv; dz = nz * inv;
-        }
-    }
-    // block reduction of the energy bookkeeping, one FP64 atomic per block and quantity
+// Source voxel and weight of a history of source `src`; false if it emits nothing.
+// (I: 32-bit where the volume and the histories allow it; 64-bit divisions take 130
+// instructions each.)
+template <typename I>
+__device__ __forceinline__ bool mc_source(const MCArgs &a, const float *__restrict__ act, I src, I &v, float &w) {
+    const long long vl = a.active ? a.active[src] : (long long)src;
+    if (vl < 0 || vl >= (long long)a.n[0] * a.n[1] * a.n[2] || !(act[vl] > 0.0f)) return false;
+    v = (I)vl;
+    w = act[vl] / (float)a.histories;
+    return true;
+}
+
+// First draw of a history: its position in the emitting voxel and its initial energy.
+template <typename I>
+__device__ __forceinline__ void mc_birth(const MCArgs &a, const Philox &rng, I id, I v, float &px, float &py, float &pz,
+                                         float &r, float &e_start) {
+    const uint4 r4 = rng((uint32_t)id, (uint32_t)((unsigned long long)id >> 32), 0u, 0x5eedu);
+    const I vxy = v / (I)a.n[2];
+    const int vz = (int)(v - vxy * (I)a.n[2]);
+    const int vx = (int)(vxy / (I)a.n[1]);
+    const int vy = (int)(vxy - (I)vx * (I)a.n[1]);
+    // position in voxel units, uniform inside the emitting voxel
+    px = (float)vx + u01(r4.x);
+    py = (float)vy + u01(r4.y);
+    pz = (float)vz + u01(r4.z);
+    const float e0 = table_lerp(a.e_of_u, a.n_u, u01(r4.w) * (float)(a.n_u - 1));
+    r = fminf(range_of(a, e0), a.r_max);
+    const float dr = a.r_max / (float)(a.n_r - 1);
+    const float inv_dr = 1.0f / dr;
+    e_start = table_lerp(a.e_of_r, a.n_r, r * inv_dr);
+}
+
+// thick-target bremsstrahlung yield: the electron keeps (1 - Y) of its losses
+__device__ __forceinline__ float brems_yield(const MCArgs &a, float e_start) {
+    if (!(a.brems_z > 0.0f)) return 0.0f;
+    const float x = 6.0e-4f * a.brems_z * e_start;
+    return x / (1.0f + x);
+}
+
+// block reduction of the energy bookkeeping, one FP64 atomic per block and quantity
+__device__ __forceinline__ void mc_totals(double emitted, double deposited, double escaped, double *totals) {
+    __shared__ double red[3][MC_BLOCK / 64];
     double vals[3] = {emitted, deposited, escaped};
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -270,9 +226,239 @@ __global__ __launch_bounds__(256) void pvd_mc_kernel(MCArgs a, const float *__re
     __syncthreads();
     if (threadIdx.x < 3) {
         double s = 0.0;
-        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) s += red[threadIdx.x][i];
+        for (int i = 0; i < MC_BLOCK / 64; ++i) s += red[threadIdx.x][i];
         atomicAdd(&totals[threadIdx.x], s);
     }
+}
+
+// Deposit map of a workgroup: the global map, or (TILE) a copy of it in LDS.
+template <bool TILE>
+__device__ __forceinline__ double *mc_tile(const MCArgs &a, double *edep) {
+    if constexpr (!TILE) return edep;
+    extern __shared__ double mc_lds[];
+    const int nvox = a.n[0] * a.n[1] * a.n[2];
+    for (int i = threadIdx.x; i < nvox; i += MC_BLOCK) mc_lds[i] = 0.0;
+    __syncthreads();
+    return mc_lds;
+}
+template <bool TILE>
+__device__ __forceinline__ void mc_flush(const MCArgs &a, const double *tile, double *edep) {
+    if constexpr (TILE) {
+        const int nvox = a.n[0] * a.n[1] * a.n[2];
+        __syncthreads();
+        // every workgroup starts elsewhere, so they do not queue on one address
+        const int at = (int)(blockIdx.x * 977u % (unsigned)nvox);
+        for (int i = threadIdx.x; i < nvox; i += MC_BLOCK) {
+            const int k = i + at < nvox ? i + at : i + at - nvox;
+            if (tile[k] != 0.0) atomicAdd(&edep[k], tile[k]);
+        }
+    }
+}
+
+// Electrons.  A history is 1 .. 50 steps long (a wave of 64 would run as long as its
+// longest, about twice its mean), so a wave owns a run of `chunk` histories and a lane
+// whose history has ended goes on with a spare one it holds; once MC_REFILL lanes lack a
+// spare (or no lane has work) they start the next histories together.  Deposits of
+// consecutive steps in one voxel are summed in a register (FP64) and added to the map when
+// the electron leaves it.  Histories, random numbers and steps are the same for every
+// mapping of histories to lanes.  (64^3 phantom, 16 histories a voxel, with photons: 2260 us
+// with a thread per history, its photons walked by one lane of 16 and a 64-bit index; now
+// 1210.  What is left is the atomics: without the photons' 820.)
+template <typename I>
+__device__ __forceinline__ void mc_electrons(const MCArgs &a, const float *__restrict__ act,
+                                             const float *__restrict__ dens, double *__restrict__ map, long long next,
+                                             long long end, double &emitted, double &deposited, double &escaped) {
+    const Philox rng{a.seed_lo, a.seed_hi};
+    const int lane = threadIdx.x & 63;
+    const float dr = a.r_max / (float)(a.n_r - 1);
+    const float inv_dr = 1.0f / dr;
+    bool active = false, spare = false;
+    I hid = 0, s_id = 0;
+    uint32_t draw = 0;
+    float w = 0.0f, keep = 0.0f, px = 0.0f, py = 0.0f, pz = 0.0f, dx = 0.0f, dy = 0.0f, dz = 0.0f;
+    float r = 0.0f, r0 = 1.0f, e_cur = 0.0f;
+    float s_w = 0.0f, s_px = 0.0f, s_py = 0.0f, s_pz = 0.0f, s_dx = 0.0f, s_dy = 0.0f, s_dz = 0.0f, s_r = 0.0f, s_e = 0.0f;
+    int guard = 0;
+    I cur = 0;                          // voxel whose deposits wait in `pend`
+    double pend = 0.0;
+    for (;;) {
+        const unsigned long long lack = __ballot(!spare);
+        if (next < end && (__popcll(lack) >= MC_REFILL || !__any(active || spare))) {
+            const long long id = next + __popcll(lack & ((1ull << lane) - 1));
+            I v;
+            if (!spare && id < end && mc_source<I>(a, act, (I)id / (I)a.histories, v, s_w)) {
+                s_id = (I)id;
+                mc_birth<I>(a, rng, s_id, v, s_px, s_py, s_pz, s_r, s_e);
+                const uint4 r4 = rng((uint32_t)s_id, (uint32_t)((unsigned long long)s_id >> 32), 1u, 0x5eedu);
+                iso_dir(r4.x, r4.y, s_dx, s_dy, s_dz);
+                spare = true;
+            }
+            next += __popcll(lack);
+        }
+        if (!active && spare) {
+            spare = false;
+            hid = s_id;
+            w = s_w;
+            px = s_px; py = s_py; pz = s_pz;
+            dx = s_dx; dy = s_dy; dz = s_dz;
+            r = s_r;
+            e_cur = s_e;
+            draw = 2;
+            guard = 0;
+            r0 = fmaxf(r, 1e-6f);
+            keep = 1.0f - brems_yield(a, e_cur);
+            emitted += (double)w * keep * e_cur;
+            active = r > 0.0f;
+        }
+        if (!__any(active)) {
+            if (next >= end && !__any(spare)) break;
+            continue;
+        }
+        if (active) {
+            const int ix = (int)floorf(px), iy = (int)floorf(py), iz = (int)floorf(pz);
+            if (ix < 0 || iy < 0 || iz < 0 || ix >= a.n[0] || iy >= a.n[1] || iz >= a.n[2]) {
+                escaped += (double)w * keep * e_cur;
+                active = false;
+            } else {
+                const I vox = ((I)ix * (I)a.n[1] + (I)iy) * (I)a.n[2] + (I)iz;
+                const float rho = fmaxf(dens ? dens[vox] : 1.0f, a.rho_min);
+                const float s = fminf(fminf(a.step_mm, r), a.half_voxel_mm * rho);   // water-equivalent mm
+                r = fmaxf(r - s, 0.0f);
+                const float e_next = r > 0.0f ? table_lerp(a.e_of_r, a.n_r, r * inv_dr) : 0.0f;
+                const float de = keep * (e_cur - e_next);
+                if (vox != cur) {
+                    if (pend != 0.0) atomicAdd(&map[cur], pend);
+                    cur = vox;
+                    pend = 0.0;
+                }
+                pend += (double)(w * de);
+                deposited += (double)w * de;
+                e_cur = e_next;
+                active = r > 0.0f && ++guard < 100000;
+                if (active) {
+                    const float len = (s / rho) * a.inv_voxel;   // geometric step in voxel units
+                    px = fmaf(dx, len, px);
+                    py = fmaf(dy, len, py);
+                    pz = fmaf(dz, len, pz);
+                    // Gaussian deflection about the current direction
+                    const uint4 r4 = rng((uint32_t)hid, (uint32_t)((unsigned long long)hid >> 32), draw++, 0x5eedu);
+                    const float g = sqrtf(-2.0f * __logf(u01(r4.x))) * __cosf(6.28318530718f * u01(r4.y));
+                    const float th = a.scatter * sqrtf(s / r0) * g;
+                    float st, ct, sp, cp;
+                    __sincosf(th, &st, &ct);
+                    __sincosf(6.28318530718f * u01(r4.z), &sp, &cp);
+                    // orthonormal frame (e1, e2) perpendicular to d
+                    float e1x, e1y, e1z;
+                    if (fabsf(dz) < 0.9f) {            // e1 = normalize(d x z)
+                        const float inv = rsqrtf(dx * dx + dy * dy);
+                        e1x = dy * inv; e1y = -dx * inv; e1z = 0.0f;
+                    } else {                            // e1 = normalize(d x x)
+                        const float inv = rsqrtf(dy * dy + dz * dz);
+                        e1x = 0.0f; e1y = dz * inv; e1z = -dy * inv;
+                    }
+                    const float e2x = dy * e1z - dz * e1y, e2y = dz * e1x - dx * e1z, e2z = dx * e1y - dy * e1x;
+                    const float nx = ct * dx + st * (cp * e1x + sp * e2x);
+                    const float ny = ct * dy + st * (cp * e1y + sp * e2y);
+                    const float nz = ct * dz + st * (cp * e1z + sp * e2z);
+                    const float inv = rsqrtf(nx * nx + ny * ny + nz * nz);
+                    dx = nx * inv; dy = ny * inv; dz = nz * inv;
+                }
+            }
+        }
+    }
+    if (pend != 0.0) atomicAdd(&map[cur], pend);
+}
+
+// Photons: packet t is line t mod kinds (the last kind: bremsstrahlung) of the
+// photon_every-th histories of a voxel, weight x photon_every.
+template <typename I>
+__device__ __forceinline__ void mc_photons(const MCArgs &a, const float *__restrict__ act, const float *__restrict__ dens,
+                                           double *__restrict__ map, long long first, long long step, long long total,
+                                           int per_src, int kinds, double &emitted, double &deposited, double &escaped) {
+    const Philox rng{a.seed_lo, a.seed_hi};
+    for (long long t = first; t < total; t += step) {
+        const I k = (I)t / (I)kinds, src = k / (I)per_src;
+        const int l = (int)((I)t - k * (I)kinds);
+        const I id = src * (I)a.histories + (k - src * (I)per_src) * (I)a.photon_every;
+        I v;
+        float w;
+        if (!mc_source<I>(a, act, src, v, w)) continue;
+        float px, py, pz, r, e_start;
+        mc_birth<I>(a, rng, id, v, px, py, pz, r, e_start);
+        const float wp = w * (float)a.photon_every;
+        const uint4 q = rng((uint32_t)id, (uint32_t)((unsigned long long)id >> 32), (uint32_t)l, 0xf07u);
+        float qx, qy, qz;
+        iso_dir(q.x, q.y, qx, qy, qz);
+        if (l < a.n_lines) {
+            const float wl = wp * a.line_y[l];
+            emitted += (double)wl * a.line_e[l];
+            photon_packet<I>(a, dens, map, px, py, pz, qx, qy, qz, a.line_e[l], a.line_e[l], wl, deposited, escaped);
+        } else {
+            const float yb = brems_yield(a, e_start);
+            if (!(yb > 0.0f)) continue;
+            const float kq = fmaxf(e_start * (1.0f - sqrtf(u01(q.z))), 1e-3f);    // energy spectrum ~ (E0 - k)
+            const float eb = yb * e_start;
+            emitted += (double)wp * eb;
+            // the packet carries Y E0 and is absorbed with mu_en at its sampled energy k
+            photon_packet<I>(a, dens, map, px, py, pz, qx, qy, qz, eb, kq, wp, deposited, escaped);
+        }
+    }
+}
+
+// Every wave transports a share of the electrons and of the photons; odd waves the photons
+// first, even waves the electrons, so both kinds run at any time: the photons' deposits are
+// bound by the rate of scattered FP64 atomics (a packet crosses 40 voxels of a 64^3 grid,
+// each in its own cache line; about 2e10 a second) and leave the vector units idle, the
+// electrons' steps by the vector units.
+template <bool TILE, typename I>
+__global__ __launch_bounds__(MC_BLOCK) void pvd_mc_kernel(MCArgs a, const float *__restrict__ act,
+                                                          const float *__restrict__ dens, double *__restrict__ edep,
+                                                          double *__restrict__ totals, long long packets, int per_src,
+                                                          int kinds, long long n_hist, long long chunk) {
+    double *map = mc_tile<TILE>(a, edep);
+    double emitted = 0.0, escaped = 0.0, deposited = 0.0;
+    const int wave = threadIdx.x >> 6;
+    const long long next = ((long long)blockIdx.x * (MC_BLOCK / 64) + wave) * chunk;
+    const long long end = a.electrons ? std::min(next + chunk, n_hist) : 0;
+    for (int phase = 0; phase < 2; ++phase) {
+        if ((phase ^ wave) & 1)
+            mc_photons<I>(a, act, dens, map, blockIdx.x * (long long)MC_BLOCK + threadIdx.x, (long long)gridDim.x * MC_BLOCK,
+                          packets, per_src, kinds, emitted, deposited, escaped);
+        else
+            mc_electrons<I>(a, act, dens, map, next, end, emitted, deposited, escaped);
+    }
+    mc_flush<TILE>(a, map, edep);
+    mc_totals(emitted, deposited, escaped, totals);
+}
+
+template <bool TILE, typename I>
+hipError_t launch_mc(const MCArgs &a, const float *act, const float *dens, double *edep, double *totals, long long n_hist,
+                     int per_src, int kinds, long long nvox, hipStream_t st) {
+    const size_t lds = TILE ? sizeof(double) * (size_t)nvox : 0;
+    if (TILE) {
+        static bool attr = false;
+        if (!attr) {
+            const int most = (int)(sizeof(double) * kMcTileVoxels);
+            const hipError_t e = hipFuncSetAttribute((const void *)pvd_mc_kernel<TILE, I>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, most);
+            if (e != hipSuccess) return e;
+            attr = true;
+        }
+    }
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        cus = 256;
+    constexpr int wpb = MC_BLOCK / 64;
+    // workgroups for the whole chip (with an LDS tile: two per CU); a wave gets at least 64
+    // histories
+    const long long packets = a.n_src * per_src * kinds;
+    const long long waves = std::min((long long)cus * (TILE ? 2 * wpb : MC_WAVES), (n_hist + 63) / 64);
+    const long long chunk = (n_hist + waves - 1) / waves;
+    const long long blocks = ((n_hist + chunk - 1) / chunk + wpb - 1) / wpb;
+    hipLaunchKernelGGL((pvd_mc_kernel<TILE, I>), dim3((unsigned)blocks), dim3(MC_BLOCK), lds, st, a, act, dens, edep,
+                       totals, packets, per_src, kinds, n_hist, chunk);
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -312,12 +498,18 @@ hipError_t pvd_launch_mc(const pvd_mc_params *p, const float *act, const float *
     a.mu_lo = (float)p->mu_log_e_lo;
     a.mu_inv_step = p->n_mu > 1 ? (float)((p->n_mu - 1) / (p->mu_log_e_hi - p->mu_log_e_lo)) : 0.0f;
     a.rho_min_ph = (float)p->rho_min;
-    const long long threads = a.n_src * p->histories;
-    if (threads == 0) return hipSuccess;
-    const long long blocks = (threads + 255) / 256;
-    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(pvd_mc_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, act, dens, edep, totals);
-    return hipGetLastError();
+    const long long n_hist = a.n_src * p->histories;
+    if (n_hist == 0) return hipSuccess;
+    const long long nvox = (long long)a.n[0] * a.n[1] * a.n[2];
+    const int per_src = (p->histories + p->photon_every - 1) / p->photon_every;
+    const int kinds = a.n_lines + (a.brems_z > 0.0f ? 1 : 0);
+    // 32-bit indexes where voxels, histories (and the last wave's overshoot) and packets fit
+    const bool small = nvox < 0x7fffffffLL && n_hist < 0x70000000LL && a.n_src * per_src * (kinds + 1) < 0x70000000LL;
+    const bool tile = nvox <= kMcTileVoxels;
+    if (tile && small) return launch_mc<true, uint32_t>(a, act, dens, edep, totals, n_hist, per_src, kinds, nvox, st);
+    if (tile) return launch_mc<true, unsigned long long>(a, act, dens, edep, totals, n_hist, per_src, kinds, nvox, st);
+    if (small) return launch_mc<false, uint32_t>(a, act, dens, edep, totals, n_hist, per_src, kinds, nvox, st);
+    return launch_mc<false, unsigned long long>(a, act, dens, edep, totals, n_hist, per_src, kinds, nvox, st);
 }
 
 extern "C" int pvd_mc_dose(const pvd_mc_params *p, const float *activity, const float *density, double *edep,

@@ -710,3 +710,27 @@ def test_training_layers_and_layer_gradient(shape):
                                    atol=2e-4 * np.abs(exp).max())
         np.testing.assert_allclose(part.double().sum(0).cpu().numpy(), (exp * mb).sum((0, 1, 2)), rtol=0,
                                    atol=1e-4 * np.abs(exp).max() * n ** 0.5 + 1e-6 * (np.abs(exp) * mb).sum((0, 1, 2)).max())
+
+
+@pytest.mark.parametrize("shape,histories,every", [((1, 1, 1), 1, 1), ((3, 5, 7), 63, 16), ((21, 22, 21), 3, 2),
+                                                   ((22, 21, 22), 3, 2), ((40, 9, 31), 17, 5)])
+def test_monte_carlo_maps_histories_alike(shape, histories, every):
+    """Deposit maps tallied in LDS (at most 10000 voxels: 21x22x21 is below, 22x21x22 above)
+    and in memory, around the wave and spare-history steps: deposits and escapes sum to the
+    emitted energy, and the tally depends on the seed only (FP64 sums in another order:
+    1e-12 of the maximum)."""
+    import torch
+
+    from pyvoxeldosimetry_amd.learned.mc import MonteCarlo
+    _say("mc mapping", shape, histories, every)
+    g = torch.Generator().manual_seed(sum(shape))
+    act = torch.rand(shape, generator=g).cuda()
+    rho = (0.3 + torch.rand(shape, generator=g)).cuda()
+    for nuclide in ("Y90", "Lu177"):
+        mc = MonteCarlo(nuclide, photon_every=every)
+        e = mc.edep(act, rho, 2.0, histories, seed=5)
+        emitted, deposited, escaped = mc.last_totals.tolist()
+        assert deposited + escaped == pytest.approx(emitted, rel=1e-5)
+        again = mc.edep(act, rho, 2.0, histories, seed=5)
+        assert float((e - again).abs().max()) <= 1e-12 * float(e.max())
+        assert float(e.min()) >= 0.0

@@ -102,3 +102,24 @@ def test_more_parameters_than_samples_fail_like_the_reference():
     assert not p.any() and not auc.any() and not any(info["success"])
     with pytest.raises(ValueError):
         TimeCurveFitting(64.1).fit_time_activity_curve_advanced(T4, _maps(y, (4, 4, 4)), model="other")
+
+
+@pytest.mark.parametrize("T", [2, 4, 5, 8, 9, 16])
+def test_sample_counts_of_the_compiled_forms(T):
+    """Every compiled sample count at its edges (up to 4, 8, 16 samples): the basic fit against
+    curve_fit, tolerances as above."""
+    from pyvoxeldosimetry_amd.time_integration import TimeCurveFitting
+    _say("tac sample counts", T)
+    rng = np.random.default_rng(T)
+    shape = (4, 5, 13)                              # 260 voxels: one past a block
+    n = int(np.prod(shape))
+    times = list(np.linspace(2.0, 150.0, T))
+    A0 = rng.uniform(1e3, 1e5, n)
+    lam = rng.uniform(0.004, 0.06, n)
+    y = A0[:, None] * np.exp(-lam[:, None] * np.array(times)) * rng.normal(1.0, 0.02, (n, T))
+    y = y.astype(np.float32).astype(np.float64)
+    tcf = TimeCurveFitting(64.1)
+    p, acc = tcf.fit_time_activity_curve(times, _maps(y, shape))
+    pe, acce = tac.fit_basic(times, y, 64.1)
+    np.testing.assert_allclose(p.reshape(2, -1), pe, rtol=2e-5, atol=1e-9)
+    np.testing.assert_allclose(acc.reshape(-1), acce, rtol=5e-5)

@@ -127,3 +127,29 @@ def test_ct_phantom_density_is_its_hu_map_through_the_device_producer():
     p = ct_phantom()
     rho = density_from_hu(torch.from_numpy(p.meta["hu"]).cuda())
     assert torch.equal(rho.cpu(), torch.from_numpy(p.density))
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (1, 1, 3), (2, 2, 1), (3, 5, 7), (9, 4, 2), (5, 7, 13), (6, 33, 31), (40, 41, 50)])
+@pytest.mark.parametrize("handle", [True, False])
+def test_tissue_map_item_edges(shape, handle):
+    """Items of four voxels that span two z-rows, the last n % 4 voxels, volumes below one
+    item or one wave chunk, and many metal items per workgroup (every fifth voxel)."""
+    _say("tissue items", shape, handle)
+    rng = np.random.default_rng(sum(shape))
+    ct = rng.normal(40.0, 300.0, size=shape).astype(np.float32)
+    ct[rng.random(shape) < 0.2] = 2800.0
+    ct.reshape(-1)[-1] = 3000.0                                # metal in the last, partial item
+    _check(ct, handle)
+
+
+def test_tissue_map_of_an_unaligned_view():
+    """Maps that are not 16-byte aligned take the scalar form: the same values."""
+    import torch
+    from pyvoxeldosimetry_amd.tissue import TissueComposition
+    _say("tissue unaligned")
+    rng = np.random.default_rng(5)
+    flat = torch.from_numpy(rng.normal(40.0, 900.0, size=7 * 9 * 11 + 1).astype(np.float32)).cuda()
+    view = flat[1:].view(7, 9, 11)
+    tc = TissueComposition()
+    for a, b in zip(tc.map(view), tc.map(view.clone())):
+        assert torch.equal(a, b)

@@ -67,8 +67,9 @@ typedef struct pvd_plan_params {
     int flags;      /* PVD_FLAG_*                                               */
     int tile[3];    /* lines per FFT tile: x pass, y pass (kz columns), z pass  */
                     /* (complex line pairs); power of two <= 64, 0 = 16 (x: 8   */
-                    /* for the two-step lengths 288..512)                        */
-    int max_radix;  /* largest power-of-two Stockham radix: 16 or 8, 0 = 16     */
+                    /* for the two-step lengths 288..512; 8 or 4 for the         */
+                    /* Stockham passes of small volumes)                         */
+    int max_radix;  /* largest power-of-two Stockham radix: 16 or 8, 0 = the plan's choice */
 } pvd_plan_params;
 
 typedef struct pvd_plan_info {

@@ -128,7 +128,7 @@ def tuned_plan(shape, kernel_shape, mode, kernel_dev, max_candidates: int = 6, s
             plan.close()
     if best is None:
         raise RuntimeError(f"no usable convolution plan for shape {shape}, kernel {kernel_shape}")
-    tile, radix, stockham = list(best[1].tile) if best[2] == "fft" else None, 16, False
+    tile, radix, stockham = list(best[1].tile) if best[2] == "fft" else None, best[1].max_radix, False
     if best[2] == "fft" and search_tiles:
         fn = best[1].fft_n
 
@@ -141,7 +141,8 @@ def tuned_plan(shape, kernel_shape, mode, kernel_dev, max_candidates: int = 6, s
             p.set_kernel(kernel_dev)
             return time_plan(p), p
 
-        # from the tiles the plan chose itself (16 lines, 8 on x for some two-step lengths)
+        # from the tiles the plan chose itself (16 lines; 8 on x for some two-step lengths, 8 or
+        # 4 for the Stockham passes of small volumes)
         for axis in (2, 1, 0):
             for t in (8, 16, 32):
                 if t == tile[axis]:
@@ -155,11 +156,12 @@ def tuned_plan(shape, kernel_shape, mode, kernel_dev, max_candidates: int = 6, s
                     tile = cand
                 elif res is not None:
                     res[1].close()
-        res = trial(tile, 8)
+        other = 24 - radix
+        res = trial(tile, other)
         if res is not None and res[0] < 0.98 * best[0]:
             best[1].close()
             best = (res[0], res[1], "fft", fn)
-            radix = 8
+            radix = other
         elif res is not None:
             res[1].close()
         res = trial(tile, radix, True)

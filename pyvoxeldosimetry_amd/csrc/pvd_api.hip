@@ -173,6 +173,8 @@ struct pvd_plan {
     int lo[3]{}, s[3]{};           // kernel placement (first used sample, shift)
     int tile[3]{};                 // tile targets of the x, y, z passes
     int max_radix = 16;            // largest power-of-two Stockham radix
+    double share[3]{1, 1, 1};      // waves of everything that runs beside the x, y and z passes,
+                                   // themselves included, per wave of their own (batches)
     bool has_kernel = false;
     pvd_vol_d vol{};               // descriptor template
     launch_cfg cfg[PVD_NPASS_FFT];
@@ -195,6 +197,11 @@ struct batch_launch_d {
     int first = 0, nmem = 0;           // members in the base/vol pools
 };
 
+// Tiles of one member: its plan's, except that the other members' waves count too.
+struct batch_tiles_d {
+    int llz, ltky, ltkx, tiles[PVD_NPASS_FFT];
+};
+
 struct pvd_batch {
     std::vector<pvd_plan *> plans;
     int dev = 0;
@@ -203,6 +210,7 @@ struct pvd_batch {
     pvd_vol_d *d_tab = nullptr;        // device table read by the batch kernels
     int *d_pool = nullptr;             // device member pools: tile bases, then volume indices
     std::vector<batch_launch_d> launches;   // in pass order
+    std::vector<batch_tiles_d> lay;    // the members' tiles within the batch
     int pool_n = 0;
     std::vector<char> ready;           // volume inputs set
     hipEvent_t uploaded = nullptr;     // last table upload (host table reusable after it)
@@ -331,6 +339,23 @@ bool x_offsets_fit(long long Nx, long long Px, long long Py, long long Hp, long 
     return (Nx - 1) * wplane * 8 <= lim && (Px - 1) * Py * Hp * 8 <= lim;
 }
 
+// Lines per tile of a Stockham pass whose tile the plan chooses.  A 16-line tile of a
+// short transform is one or two wavefronts (16 elements per thread), so a small volume's
+// pass puts fewer waves on the chip than it has SIMDs and runs at the latency of one
+// tile: halve the tile, down to `least` lines, while the pass (`share` times over: the
+// other members of a batch run beside it) has fewer than kFewWaves waves, two for each
+// of 1024 SIMDs.  Measured, whole dose calls in us, 16 lines against the rule's: 64^3
+// 50.1 -> 35.5, 72x72x50 56.0 -> 43.9, 100^3 62.9 -> 56.1, 125^3 77.1 -> 69.7; the line
+// lies between z lines of 64 points at 1772 waves (75.6 -> 69.3 with 8) and of 125 points
+// at 2500 (89.3, 90.5 with 8).  In a batch of sixteen 64^3 volumes 16 lines take 103 us and
+// small tiles 131, of four 74 and 65.
+constexpr double kFewWaves = 2048;
+template <typename Tiles>
+int few_waves_tile(int n, int lines, int least, double share, Tiles tiles) {
+    while (lines > least && share * tiles(lines) * ((lines * n + 1023) / 1024) < kFewWaves) lines /= 2;
+    return lines;
+}
+
 // Host-only layout of an FFT plan: tiles, register paths, launch shapes and buffer
 // sizes (no device call).
 int fft_layout(pvd_plan *p) {
@@ -338,15 +363,25 @@ int fft_layout(pvd_plan *p) {
     const int Nx = p->N[0], Ny = p->N[1];
     const int Px = p->P[0], Py = p->P[1], Pz = p->P[2];
     v.H = Pz / 2 + 1;
+    const bool regs = !(p->prm.flags & PVD_FLAG_STOCKHAM);
+    const long long nlines = (long long)Nx * Ny;
+    auto z_tiles = [&](int l) { return (nlines + 2 * l - 1) / (2 * l); };
+    auto y_tiles = [&](int l) { return (long long)Nx * ((v.H + l - 1) / l); };
+    auto x_tiles = [&](int l) { return (long long)Py * ((v.H + l - 1) / l); };
     int lz, bz; size_t ldsz;
     pick_tile(Pz, p->tile[2], 1, &lz, &bz, &ldsz);
+    if (p->prm.tile[2] == 0 && regs && !z_reg_code(Pz))
+        pick_tile(Pz, few_waves_tile(Pz, lz, 4, p->share[2], z_tiles), 1, &lz, &bz, &ldsz);
     // z blocks are a power-of-two multiple of the lines per tile, so the z passes'
     // I/O phases (blockDim / lines threads per line pair) keep every thread busy
     // (at most 1024: both factors are powers of two)
     { int per = 1; while (per * lz < bz) per *= 2; bz = per * lz; }
     int tky, by; size_t ldsy;
     pick_tile(Py, p->tile[1], 0, &tky, &by, &ldsy);
-    const bool regs = !(p->prm.flags & PVD_FLAG_STOCKHAM);
+    // y: whole 128-byte lines of 16 columns are worth more than waves (80x100x60 45.2 us, with
+    // 8-column y tiles 46.8) except where they make one wavefront (64^3 37.4, with 8 35.7)
+    if (p->prm.tile[1] == 0 && regs && !xy_two_step_len(Py) && tky * Py <= 1024)
+        pick_tile(Py, few_waves_tile(Py, tky, 8, p->share[1], y_tiles), 0, &tky, &by, &ldsy);
     // x tile left to the plan: 8 columns for the fused two-step lengths 16 * B with
     // B >= 18 (the X pass holds a column's two transforms and its spectrum values in
     // registers there, and half-width tiles fit more workgroups per CU)
@@ -354,6 +389,8 @@ int fft_layout(pvd_plan *p) {
     if (p->prm.tile[0] == 0 && regs && xy_two_step_len(Px) && Px >= 16 * 18 && Px < 16 * PVD_XY_LDS_B) tile_x = 8;
     int tkx, bx; size_t ldsx;
     pick_tile(Px, tile_x, 0, &tkx, &bx, &ldsx);
+    if (p->prm.tile[0] == 0 && regs && !xy_two_step_len(Px))
+        pick_tile(Px, few_waves_tile(Px, tkx, 4, p->share[0], x_tiles), 0, &tkx, &bx, &ldsx);
     // y/x register paths: 1 = the 256-point path (16-line tiles, no reference-mode fold;
     // checked again in the kernel); 2 = the two-step P = 16 * rb (rb in kXyRegB) in its
     // own kernel instances
@@ -390,6 +427,24 @@ int fft_layout(pvd_plan *p) {
             break;
         }
     }
+    // largest radix left to the plan: 8 where no Stockham axis needs more stages with it than
+    // with 16 (64 = 8 * 8 rather than 16 * 4: as many passes over LDS, twice the threads with
+    // work in the first), else 16 (48 = 16 * 3, not 8 * 2 * 3).  Measured: 64^3 37.6 us with
+    // 16 * 4, 35.5 with 8 * 8; 48^3 36.1 with 16 * 3, 40.6 with 8 * 2 * 3
+    if (p->prm.max_radix == 0 && regs) {
+        pvd_axis_d r8[3]{};
+        bool as_few = true;
+        for (int a = 0; a < 3; ++a) {
+            r8[a].nst = factor_radices(p->P[a], r8[a].radix, 8);
+            const bool stockham = a == 2 ? v.ax[a].reg == 0 : !xy_two_step_len(p->P[a]);
+            as_few = as_few && (!stockham || r8[a].nst <= v.ax[a].nst);
+        }
+        for (int a = 0; as_few && a < 3; ++a) {
+            v.ax[a].nst = r8[a].nst;
+            memcpy(v.ax[a].radix, r8[a].radix, sizeof r8[a].radix);
+        }
+        if (as_few) p->max_radix = 8;
+    }
     // the two-step instances run blocks of at most PVD_XY_MAX_BLOCK threads
     if (v.ax[1].reg == 2) by = std::min(by, PVD_XY_MAX_BLOCK);
     if (v.ax[0].reg == 2) bx = std::min(bx, PVD_XY_MAX_BLOCK);
@@ -408,10 +463,7 @@ int fft_layout(pvd_plan *p) {
         const bool reg32 = (ax.reg == 1 && Px == 256) || (ax.reg == 2 && ax.rb < PVD_XY_LDS_B);
         if (reg32 && !x_offsets_fit(Nx, Px, Py, v.Hp, v.wplane)) ax.reg = 0, ax.ra = ax.ra_log = ax.rb = 0;
     }
-    const long long nlines = (long long)Nx * Ny;
-    const long long tz = (nlines + 2 * lz - 1) / (2 * lz);
-    const long long ty = (long long)Nx * ((v.H + tky - 1) / tky);
-    const long long tx = (long long)Py * ((v.H + tkx - 1) / tkx);
+    const long long tz = z_tiles(lz), ty = y_tiles(tky), tx = x_tiles(tkx);
     if (tz > 0x7fffffffLL || ty > 0x7fffffffLL || tx > 0x7ffffff0LL) return fail(PVD_ENOTSUP, "grid too large");
     p->cfg[PVD_PASS_FZ] = {(int)tz, bz, ldsz};
     p->cfg[PVD_PASS_IZ] = {(int)tz, bz, ldsz};
@@ -864,15 +916,38 @@ int pvd_batch_create(pvd_batch **out, pvd_plan *const *plans, int nvol) {
     b->ready.assign(nvol, 0);
     int rc = PVD_OK;
     do {
+        // the members' layouts in the batch: how many waves the passes have in all, then
+        // each member's tiles with them counted (the same transforms on other tiles: the
+        // bits are those of the member's own plan)
+        std::vector<pvd_plan> lay;
+        double all[3] = {0, 0, 0};
+        for (int turn = 0; turn < 2 && !rc; ++turn)
+            for (int i = 0; i < nvol && !rc; ++i) {
+                static const int kPass[3] = {PVD_PASS_X, PVD_PASS_FY, PVD_PASS_FZ};
+                if (turn == 0) lay.push_back(*plans[i]);
+                pvd_plan &q = lay[i];
+                for (int a = 0; a < 3; ++a) {
+                    const launch_cfg &c = q.cfg[kPass[a]];
+                    q.share[a] = turn == 0 ? kFewWaves : all[a] / ((double)c.grid * c.block);
+                }
+                rc = fft_layout(&q);
+                for (int a = 0; a < 3 && turn == 0; ++a)
+                    all[a] += (double)q.cfg[kPass[a]].grid * q.cfg[kPass[a]].block;
+            }
+        if (rc) break;
+        for (const pvd_plan &q : lay) {
+            batch_tiles_d t = {q.vol.llz, q.vol.ltky, q.vol.ltkx, {}};
+            std::copy(q.vol.tiles, q.vol.tiles + PVD_NPASS_FFT, t.tiles);
+            b->lay.push_back(t);
+        }
         // Each pass launches once per group of volumes that run the same kernel instance
-        // with the same block as their own plans (so a batched volume gives the bits of
-        // its single-volume plan); a group's grid concatenates its members' tiles.
+        // with the same block; a group's grid concatenates its members' tiles.
         std::vector<int> bases, vols;
         for (int pass = 0; pass < PVD_NPASS_FFT && !rc; ++pass) {
             std::vector<std::vector<int>> groups;
             std::vector<long long> keys;
             for (int i = 0; i < nvol; ++i) {
-                const long long key = batch_instance_key(plans[i], pass);
+                const long long key = batch_instance_key(&lay[i], pass);
                 size_t g = 0;
                 while (g < keys.size() && keys[g] != key) ++g;
                 if (g == keys.size()) { keys.push_back(key); groups.emplace_back(); }
@@ -886,7 +961,7 @@ int pvd_batch_create(pvd_batch **out, pvd_plan *const *plans, int nvol) {
                 L.nmem = (int)grp.size();
                 long long total = 0;
                 for (int i : grp) {
-                    const launch_cfg &pc = plans[i]->cfg[pass];
+                    const launch_cfg &pc = lay[i].cfg[pass];
                     L.cfg.block = pc.block;
                     L.cfg.lds = std::max(L.cfg.lds, pc.lds);
                     bases.push_back((int)total);
@@ -923,7 +998,7 @@ int pvd_batch_create(pvd_batch **out, pvd_plan *const *plans, int nvol) {
             rc = fail(PVD_EHIP, "create event");
             break;
         }
-        for (int i = 0; i < nvol; ++i) b->h_tab[i] = plans[i]->vol;
+        for (int i = 0; i < nvol; ++i) b->h_tab[i] = lay[i].vol;
     } while (0);
     if (rc) {
         pvd_batch_destroy(b);
@@ -950,7 +1025,13 @@ int pvd_batch_set_volume(pvd_batch *b, int i, const float *const *acts, const do
         PVD_HIP(hipEventSynchronize(b->uploaded), "wait for descriptor upload");
         b->upload_pending = false;
     }
-    fill_desc(p, acts, w, T, density, dose, scale, &b->h_tab[i]);
+    pvd_vol_d &v = b->h_tab[i];
+    fill_desc(p, acts, w, T, density, dose, scale, &v);
+    const batch_tiles_d &t = b->lay[i];
+    v.llz = t.llz;
+    v.ltky = t.ltky;
+    v.ltkx = t.ltkx;
+    std::copy(t.tiles, t.tiles + PVD_NPASS_FFT, v.tiles);
     b->ready[i] = 1;
     return PVD_OK;
 }
@@ -986,7 +1067,7 @@ int batch_capture(pvd_batch *b) {
             a.vol = b->d_pool + b->pool_n + L.first;
             a.nmem = L.nmem;
             a.ntiles = L.cfg.grid;
-            PVD_HIP(pvd_launch_fft_pass_batch(L.pass, b->plans[L.exemplar]->vol, a, L.cfg.grid, L.cfg.block,
+            PVD_HIP(pvd_launch_fft_pass_batch(L.pass, b->h_tab[L.exemplar], a, L.cfg.grid, L.cfg.block,
                                               L.cfg.lds, b->fork[k]),
                     "launch batch FFT pass");
         }
@@ -1006,7 +1087,7 @@ int batch_launch(pvd_batch *b, hipStream_t st) {
         a.vol = b->d_pool + b->pool_n + L.first;
         a.nmem = L.nmem;
         a.ntiles = L.cfg.grid;
-        PVD_HIP(pvd_launch_fft_pass_batch(L.pass, b->plans[L.exemplar]->vol, a, L.cfg.grid, L.cfg.block, L.cfg.lds,
+        PVD_HIP(pvd_launch_fft_pass_batch(L.pass, b->h_tab[L.exemplar], a, L.cfg.grid, L.cfg.block, L.cfg.lds,
                                           st),
                 "launch batch FFT pass");
     }

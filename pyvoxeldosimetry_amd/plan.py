@@ -79,7 +79,7 @@ class ConvPlan:
                  max_radix: int = 0, stockham: bool = False, smooth_lengths: bool = False):
         """``tile``: lines per FFT tile of the (x, y, z) passes (powers of two, 0 = 16, but 8
         on x for the two-step lengths 288..512);
-        ``max_radix``: largest power-of-two Stockham radix (16 or 8, 0 = 16);
+        ``max_radix``: largest power-of-two Stockham radix (16 or 8, 0 = the plan's choice);
         ``stockham``: LDS Stockham stages on every axis instead of the register-resident
         transforms (256-point y/x, two-step y/x/z);
         ``smooth_lengths``: automatic FFT lengths from the 7-smooth rule only (by default a

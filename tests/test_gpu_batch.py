@@ -181,3 +181,15 @@ def test_batch_errors():
     with pytest.raises(ValueError):
         b.set_volume(0, [dev(acts[1][0])], [1.0])          # wrong shape for volume 0
     b.close()
+
+
+@pytest.mark.parametrize("count", [1, 3, 24])
+def test_batch_tiles_follow_the_waves_of_all_members(count):
+    """Small volumes take smaller tiles alone than in a large batch, which fills the chip
+    with 16-line ones: bit-exact with the single plans on either side."""
+    _say("batch of small volumes", count)
+    rng = np.random.default_rng(count)
+    shapes = [(40 + 7 * (i % 3), 50, 60 + i % 5) for i in range(count)]
+    k = dpk.y90_kernel(4.0, (9, 9, 9), fix_centre=True)
+    acts = [rng.random(s).astype(np.float32) for s in shapes]
+    _batch_vs_single(shapes, [k] * count, acts)

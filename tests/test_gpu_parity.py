@@ -509,3 +509,26 @@ def test_register_paths_on_thin_volumes(shape, kshape):
     got = plan.dose(dev_tensor(a)).cpu().numpy()
     plan.close()
     assert_parity(got, conv.ref_conv(a.astype(np.float64), k), what=f"thin {shape}")
+
+
+@pytest.mark.parametrize("shape,mode", [((64, 64, 64), "reference"), ((61, 47, 50), "reference"),
+                                        ((30, 33, 70), "linear"), ((5, 100, 9), "linear")])
+def test_small_tiles_of_small_volumes_give_the_bits_of_16_line_tiles(shape, mode):
+    """The 4- and 8-line tiles a plan picks for the Stockham passes of a small volume run
+    the transforms of its 16-line tiles: the same bits, and the oracle's dose."""
+    from pyvoxeldosimetry_amd import ConvPlan
+    _say("small tiles", shape, mode)
+    rng = np.random.default_rng(sum(shape))
+    a = rng.random(shape).astype(np.float32)
+    k = dpk.lu177_kernel(2.0, (9, 7, 5))
+    plan = ConvPlan(shape, k.shape, mode=mode, algo="fft")
+    assert min(plan.tile) == 4
+    plan.set_kernel(k)
+    got = plan.dose(dev_tensor(a)).cpu().numpy()
+    full = ConvPlan(shape, k.shape, mode=mode, algo="fft", tile=(16, 16, 16), max_radix=plan.max_radix)
+    full.set_kernel(k)
+    assert np.array_equal(got, full.dose(dev_tensor(a)).cpu().numpy())
+    ref = conv.ref_conv if mode == "reference" else conv.linear_same
+    assert_parity(got, ref(a.astype(np.float64), k), what=f"small tiles {shape} {mode}")
+    plan.close()
+    full.close()

@@ -126,3 +126,20 @@ def test_describe_rejects_bad_parameters():
         describe_plan((8, 8, 8), (3, 3, 3), fft_n=(9, 8, 8))       # aliases: needs 8 or >= 10
     with pytest.raises(NotImplementedError):
         describe_plan((64, 64, 64), (31, 31, 31), algo="direct")    # 31 > 16 taps
+
+
+@pytest.mark.parametrize("shape,tile,radix", [
+    ((64, 64, 64), (4, 8, 4), 8),              # 64 = 8 * 8 in as many stages as 16 * 4
+    ((48, 48, 48), (4, 8, 4), 16),             # 48 = 16 * 3
+    ((100, 100, 100), (4, 16, 4), 8),          # y blocks of two wavefronts keep 16 columns
+    ((128, 64, 64), (16, 8, 4), 8),            # x is a register length: its radices do not count
+    ((300, 189, 64), (8, 16, 8), 8),           # 1772 waves of z lines: one halving
+    ((400, 400, 64), (8, 16, 16), 8),          # enough waves (x: 8 columns of 16 * 25)
+])
+def test_small_volumes_take_small_tiles_of_the_stockham_passes(shape, tile, radix):
+    d = describe_plan(shape, (11, 11, 11), "reference", algo="fft")
+    assert (d["tile"], d["max_radix"]) == (tile, radix), d
+    kept = describe_plan(shape, (11, 11, 11), "reference", algo="fft", tile=(16, 16, 16), max_radix=16)
+    assert (kept["tile"], kept["max_radix"]) == ((16, 16, 16), 16)
+    old = describe_plan(shape, (11, 11, 11), "reference", algo="fft", stockham=True)
+    assert (old["tile"], old["max_radix"]) == ((16, 16, 16), 16)

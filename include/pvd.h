@@ -190,7 +190,9 @@ int pvd_conv_dose_direct_noalloc(const int n[3], const int k[3], int mode, const
                                  const float *act, const float *density, float *dose, double scale, void *stream);
 
 /* Per-pass GPU milliseconds of the last dose call of a PVD_FLAG_PROFILE plan
- * (synchronises on it).  Writes min(n, n_passes) values; returns n_passes. */
+ * (synchronises on it).  Writes min(n, n_passes) values; returns n_passes.  Where a small
+ * volume runs the z and y transforms of its planes in one launch, the z pass has the time
+ * of both and the y pass none. */
 int pvd_plan_timings(pvd_plan *plan, float *ms, int n);
 /* Names of the passes, for reports. */
 const char *pvd_pass_name(const pvd_plan *plan, int i);

@@ -93,8 +93,9 @@ def tuned_plan(shape, kernel_shape, mode, kernel_dev, max_candidates: int = 6, s
         hit = cache.get(key)
     if hit is not None:
         fft = hit["algo"] == "fft"
+        walked = fft and not hit.get("own", False)     # tiles and radix found by the walk
         plan = ConvPlan(shape, kernel_shape, mode=mode, algo=hit["algo"], fft_n=hit.get("fft_n") if fft else None,
-                        tile=hit.get("tile") if fft else None, max_radix=hit.get("max_radix", 0) if fft else 0,
+                        tile=hit.get("tile") if walked else None, max_radix=hit.get("max_radix", 0) if walked else 0,
                         stockham=bool(hit.get("stockham", False)) and fft, device=dev)
         plan.set_kernel(kernel_dev)
         return plan
@@ -129,6 +130,7 @@ def tuned_plan(shape, kernel_shape, mode, kernel_dev, max_candidates: int = 6, s
     if best is None:
         raise RuntimeError(f"no usable convolution plan for shape {shape}, kernel {kernel_shape}")
     tile, radix, stockham = list(best[1].tile) if best[2] == "fft" else None, best[1].max_radix, False
+    chosen = False                         # a trial of the walk below was the faster
     if best[2] == "fft" and search_tiles:
         fn = best[1].fft_n
 
@@ -153,7 +155,7 @@ def tuned_plan(shape, kernel_shape, mode, kernel_dev, max_candidates: int = 6, s
                 if res is not None and res[0] < 0.98 * best[0]:
                     best[1].close()
                     best = (res[0], res[1], "fft", fn)
-                    tile = cand
+                    tile, chosen = cand, True
                 elif res is not None:
                     res[1].close()
         other = 24 - radix
@@ -161,20 +163,23 @@ def tuned_plan(shape, kernel_shape, mode, kernel_dev, max_candidates: int = 6, s
         if res is not None and res[0] < 0.98 * best[0]:
             best[1].close()
             best = (res[0], res[1], "fft", fn)
-            radix = other
+            radix, chosen = other, True
         elif res is not None:
             res[1].close()
         res = trial(tile, radix, True)
         if res is not None and res[0] < 0.98 * best[0]:
             best[1].close()
             best = (res[0], res[1], "fft", fn)
-            stockham = True
+            stockham, chosen = True, True
         elif res is not None:
             res[1].close()
+    # a plan left to its own choices is made again as one: explicit tiles would give up the
+    # passes that only such a plan takes (whole planes of small volumes)
+    own = best[2] == "fft" and not chosen
     with _lock:
         cache = _load_cache()
         cache[key] = {"algo": best[2], "fft_n": list(best[3]) if best[3] else None, "ms": best[0],
                       "tile": tile if best[2] == "fft" else None, "max_radix": radix if best[2] == "fft" else 0,
-                      "stockham": stockham}
+                      "stockham": stockham, "own": own}
         _save_cache(cache)
     return best[1]

@@ -178,6 +178,7 @@ struct pvd_plan {
     bool has_kernel = false;
     pvd_vol_d vol{};               // descriptor template
     launch_cfg cfg[PVD_NPASS_FFT];
+    launch_cfg plane;              // FZ + FY and IY + IZ as one launch each (grid 0: five passes)
     size_t work_elems = 0, spec_elems = 0;   // complex elements of the workspace and spectrum
     float2 *work = nullptr;
     float2 *spec = nullptr;
@@ -356,6 +357,31 @@ int few_waves_tile(int n, int lines, int least, double share, Tiles tiles) {
     return lines;
 }
 
+// The plane form of a small volume (pvd_fft_plane.hip): whole x-planes in LDS where the z
+// and y transforms are Stockham stages whose tiles the plan chooses and a workgroup holds
+// the plane (two planes with an odd Ny, so that the line pairs stay those of the five
+// passes) at PVD_PLANE_PER elements a thread: 8192, 16 would spill.  Five passes -> plane
+// form, whole calls in us: 64^3 35.4 -> 27.7, 100^3 58.3 -> 47.3, 30x80x80 42.5 -> 35.2,
+// 512x64x64 65.2 -> 39.0, 400x63x100 77.4 -> 49.6, 500x126x126 122 -> 120.  The line on the
+// odd side: 31x63x126 (16 workgroups of 1024 threads) 46.9 -> 48.8, 200x63x125 64.7 -> 46.8.
+void plane_layout(pvd_plan *p, bool regs) {
+    const pvd_vol_d &v = p->vol;
+    p->plane = launch_cfg();
+    if (!regs || p->prm.tile[1] || p->prm.tile[2] || v.ax[2].reg || xy_two_step_len(p->P[1])) return;
+    if (p->P[1] < 2 || p->P[2] < 2) return;                         // the first stages split and merge
+    for (int a = 1; a < 3; ++a)
+        for (int i = 0; i < v.ax[a].nst; ++i)
+            if (v.ax[a].radix[i] > 8) return;                       // not compiled: its registers would spill
+    const int Nx = p->N[0], Ny = p->N[1], Py = p->P[1], Pz = p->P[2], g = Ny % 2 ? 2 : 1;
+    const size_t elems = std::max((size_t)Pz * pvd_plane_ldz(Ny, g), (size_t)Py * pvd_plane_ldy(v.H, g));
+    const size_t lds = sizeof(float2) * (round_up(Pz, 8) + round_up(Py, 8) + elems);
+    const int most = std::max(Pz * ((g * Ny + 1) / 2), Py * g * v.H);
+    const int block = std::max(256, round_up((most + PVD_PLANE_PER - 1) / PVD_PLANE_PER, 64));
+    if (lds > kFftLdsCap || block > 1024) return;
+    if (g == 2 && block > 640 && Nx < 64) return;      // few workgroups with two large planes each
+    p->plane = {(Nx + g - 1) / g, block, lds};
+}
+
 // Host-only layout of an FFT plan: tiles, register paths, launch shapes and buffer
 // sizes (no device call).
 int fft_layout(pvd_plan *p) {
@@ -471,6 +497,7 @@ int fft_layout(pvd_plan *p) {
     p->cfg[PVD_PASS_IY] = {(int)ty, by, ldsy};
     p->cfg[PVD_PASS_X] = {(int)tx, bx, ldsx};
     for (int i = 0; i < PVD_NPASS_FFT; ++i) v.tiles[i] = p->cfg[i].grid;
+    plane_layout(p, regs);
     p->work_elems = (size_t)Nx * v.wplane;
     p->spec_elems = (size_t)Px * Py * v.Hp;
     p->bytes = sizeof(float2) * (p->work_elems + p->spec_elems);
@@ -510,7 +537,15 @@ int launch_fft(pvd_plan *p, const pvd_vol_d &v, hipStream_t st) {
     if (prof) PVD_HIP(hipEventRecord(p->ev[0], st), "record event");
     for (int pass = 0; pass < PVD_NPASS_FFT; ++pass) {
         const launch_cfg &c = p->cfg[pass];
-        PVD_HIP(pvd_launch_fft_pass(pass, v, c.grid, c.block, c.lds, st), "launch FFT pass");
+        if (p->plane.grid && pass != PVD_PASS_X) {
+            // the y pass rides in the launch of the z pass beside it
+            if (pass == PVD_PASS_FZ || pass == PVD_PASS_IZ)
+                PVD_HIP(pvd_launch_fft_plane(pass == PVD_PASS_IZ, v, p->plane.grid, p->plane.block,
+                                             p->plane.lds, st),
+                        "launch FFT plane pass");
+        } else {
+            PVD_HIP(pvd_launch_fft_pass(pass, v, c.grid, c.block, c.lds, st), "launch FFT pass");
+        }
         if (prof) PVD_HIP(hipEventRecord(p->ev[pass + 1], st), "record event");
     }
     p->profiled_call = prof;

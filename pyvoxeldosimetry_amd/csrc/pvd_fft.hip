@@ -103,6 +103,7 @@ hipError_t pvd_set_fft_lds_limits(size_t bytes) {
     PVD_SETATTR(pvd_fft_pass_batch<PVD_PASS_X>);
     PVD_SETATTR(pvd_fft_pass_batch<PVD_PASS_IY>);
 #undef PVD_SETATTR
+    if (e == hipSuccess) e = pvd_fft_plane_set_lds(bytes);
     if (e == hipSuccess) e = pvd_fft_z_set_lds(bytes);
     if (e == hipSuccess) e = pvd_fft_xy1_set_lds(bytes);
     if (e == hipSuccess) e = pvd_fft_xy2_set_lds(bytes);

@@ -426,6 +426,15 @@ hipError_t pvd_launch_fft_pass(int pass, const pvd_vol_d &v, int grid, int block
 hipError_t pvd_launch_fft_pass_batch(int pass, const pvd_vol_d &v, const pvd_batch_args &a, int grid, int block,
                                      size_t lds, hipStream_t st);
 hipError_t pvd_set_fft_lds_limits(size_t bytes);
+// small volumes: the z and y transforms of whole x-planes (one per workgroup, two with an
+// odd Ny) in one launch each way (pvd_fft_plane.hip).  Pitches in LDS of g planes: z lines
+// by line pair and y lines by kz column, odd so that neither direction meets one bank.
+inline __host__ __device__ int pvd_plane_ldz(int ny, int g) { return ((g * ny + 1) / 2) | 1; }
+inline __host__ __device__ int pvd_plane_ldy(int h, int g) { return (g * h) | 1; }
+// elements per thread, at most
+#define PVD_PLANE_PER 8
+hipError_t pvd_launch_fft_plane(bool inverse, const pvd_vol_d &v, int grid, int block, size_t lds, hipStream_t st);
+hipError_t pvd_fft_plane_set_lds(size_t bytes);
 // per source file of the z instances (pvd_fft_z.hip) and of the y/x two-step
 // instances (pvd_fft_xy1/2/3.hip); `batch` selects the table-reading instance
 hipError_t pvd_fft_launch_z(int pass, bool rz, int tp, const pvd_vol_d *v, const pvd_batch_args *a, int grid,

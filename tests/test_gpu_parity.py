@@ -532,3 +532,36 @@ def test_small_tiles_of_small_volumes_give_the_bits_of_16_line_tiles(shape, mode
     assert_parity(got, ref(a.astype(np.float64), k), what=f"small tiles {shape} {mode}")
     plan.close()
     full.close()
+
+
+@pytest.mark.parametrize("shape,kshape,mode", [
+    ((4, 2, 2), (2, 2, 2), "reference"),          # the smallest axes with a stage
+    ((3, 33, 20), (3, 5, 7), "reference"),        # odd Ny: two planes a workgroup, the last alone; wraps
+    ((4, 45, 50), (5, 3, 9), "linear"),           # odd Ny, both planes of every workgroup
+    ((65, 63, 126), (3, 3, 3), "reference"),      # the most of two planes: 63 * 64 * 2 of 8192; odd Nx
+    ((3, 126, 126), (3, 7, 5), "reference"),      # the most of one: 126 * 64 columns of 8192
+    ((2, 100, 41), (3, 9, 9), "reference"),       # a wrap on z (41 -> 49) beside none on y
+])
+def test_plane_passes_give_the_bits_of_the_five_passes(shape, kshape, mode):
+    """Small volumes run z and y of whole planes in one launch each way: the bits of the five
+    passes (explicit tiles), with two weighted maps, densities and a scale, and the oracle's
+    dose."""
+    from pyvoxeldosimetry_amd import ConvPlan
+    _say("plane passes", shape, mode)
+    rng = np.random.default_rng(sum(shape))
+    acts = [rng.random(shape).astype(np.float32) for _ in range(2)]
+    dens = rng.uniform(0.3, 1.9, shape).astype(np.float32)
+    k = rng.random(kshape)
+    w, scale = [0.75, 1.5], 0.5
+    plan = ConvPlan(shape, kshape, mode=mode, algo="fft")
+    plan.set_kernel(k)
+    five = ConvPlan(shape, kshape, mode=mode, algo="fft", tile=plan.tile, max_radix=plan.max_radix)
+    five.set_kernel(k)
+    args = ([dev_tensor(a) for a in acts], w)
+    got = plan.dose_weighted(*args, density=dev_tensor(dens), scale=scale).cpu().numpy()
+    assert np.array_equal(got, five.dose_weighted(*args, density=dev_tensor(dens), scale=scale).cpu().numpy())
+    total = sum(x * a.astype(np.float64) for x, a in zip(w, acts))
+    ref = (conv.ref_conv if mode == "reference" else conv.linear_same)(total, k)
+    assert_parity(got, scale * ref / dens.astype(np.float64), what=f"plane {shape} {mode}")
+    plan.close()
+    five.close()

@@ -38,8 +38,8 @@ int pvd_resample(const float *in, int n0, int n1, int n2, const double *in_spaci
  * (whole-sample symmetric) boundaries: the c with f[i] = (c[i-1] + 4 c[i] + c[i+1])/6
  * along every axis (Unser's exact interpolating spline; the prefilter of ITK's
  * BSplineInterpolateImageFunction, which sitkBSpline uses).  Computed per axis as
- * the symmetric FIR c[i] = sum_k h[k] f[mirror(i + k)], h[k] = sqrt(3) z^|k| with
- * z = sqrt(3) - 2, |k| <= 14 (|z|^15 < 3e-9).  coef and tmp: n0*n1*n2 floats each,
+ * c[i] = sum_k h[k] f[mirror(i + k)], h[k] = sqrt(3) z^|k| with z = sqrt(3) - 2, over at
+ * least |k| <= 14 (|z|^15 < 3e-9).  coef and tmp: n0*n1*n2 floats each,
  * neither aliasing `in`.  No reference counterpart beyond the SimpleITK call. */
 int pvd_bspline_prefilter(const float *in, int n0, int n1, int n2, float *coef, float *tmp, void *stream);
 

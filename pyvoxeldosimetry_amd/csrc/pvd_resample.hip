@@ -4,7 +4,7 @@
 // tile of output rows from it (resample_staged); nearest, and outputs much coarser than
 // the input, gather each output's neighbours (resample_kernel).  Coordinates are formed
 // in FP64 so that equal spacings map every output voxel exactly onto an input voxel.
-// The cubic B-spline coefficients come from a separable mirror-boundary FIR prefilter
+// The cubic B-spline coefficients come from a separable mirror-boundary prefilter
 // (two launches: x, then y and z).
 #include "pvd_internal.h"
 #include "../../include/pvd_resample.h"
@@ -328,104 +328,104 @@ hipError_t launch_staged(const ResampleArgs &a, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Cubic B-spline prefilter taps h[k] = sqrt(3) z^k, z = sqrt(3) - 2, k = 0..14 (FP64-built).
+// Cubic B-spline prefilter: c[i] = sum_k sqrt(3) z^|k| w[i + k], z = sqrt(3) - 2, as one
+// recursion from each side over a window of the line (Unser's factorisation of the
+// inverse).  A window starts and ends kBsK samples beyond its outputs, mirrored at the
+// volume's ends: the tail left out is below z^15 = 2.6e-9 of a sample.
 constexpr int kBsK = 14;
-struct BsTaps { float h[kBsK + 1]; };
-constexpr BsTaps bs_taps() {
-    BsTaps t{};
-    const double z = 1.7320508075688772935 - 2.0;
-    double p = 1.7320508075688772935;
-    for (int k = 0; k <= kBsK; ++k) { t.h[k] = (float)p; p *= z; }
-    return t;
-}
+constexpr float kBsZ0 = (float)(1.7320508075688772935 - 2.0), kBsGain = 1.7320508075688772935f;
 
-// One output of the prefilter, sum_{|k| <= 14} h[|k|] w[k], from a window centred on c.
-template <typename Window>
-__device__ __forceinline__ float bs_fir(const Window &w, int c) {
-    constexpr BsTaps T = bs_taps();
-    float acc = T.h[0] * w[c];
+// R outputs from the R + 28 samples get(0) ..: p and m are the sums over k <= 0 and k > 0.
+// A recursion never forgets an infinity or a NaN, which may reach 14 samples and no
+// further: a window that ends with one takes the 29-tap sum of each output.
+template <int R, typename Get>
+__device__ __forceinline__ void bs_line(const Get &get, float (&c)[R]) {
+    float w[R + 2 * kBsK];
 #pragma unroll
-    for (int k = 1; k <= kBsK; ++k) acc = fmaf(T.h[k], w[c - k] + w[c + k], acc);
-    return acc;
+    for (int i = 0; i < R + 2 * kBsK; ++i) w[i] = get(i);
+    float p = 0.0f, m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < R + kBsK; ++i) {
+        p = fmaf(kBsZ0, p, w[i]);
+        if (i >= kBsK) c[i - kBsK] = p;
+    }
+#pragma unroll
+    for (int i = R + 2 * kBsK - 1; i >= kBsK; --i) {
+        if (i < R + kBsK) c[i - kBsK] = kBsGain * fmaf(kBsZ0, m, c[i - kBsK]);
+        m = fmaf(kBsZ0, m, w[i]);
+    }
+    if (!isfinite(p) || !isfinite(m)) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            float h = kBsGain, acc = h * get(i + kBsK);
+            for (int k = 1; k <= kBsK; ++k) {
+                h *= kBsZ0;
+                acc = fmaf(h, get(i + kBsK - k) + get(i + kBsK + k), acc);
+            }
+            c[i] = acc;
+        }
+    }
 }
 
-// The prefilter runs along x in one launch and along y and z in a second (the FIR of
-// each axis is 29 taps, 43 operations: compute stays under the memory time).  A thread
-// owns one column of R consecutive outputs along the filtered axis: R + 28 loads, all
-// issued before the first is used, instead of 29 per output with an index division each
-// in three launches: 301x301x233 1288 -> 146 us (x 49, yz 94), 68 at the copy rate; the
-// yz launch is bound by its FIRs and the LDS round trip.  Same sums in the same order.
-constexpr int kBsX = 48;           // outputs per thread along x
+// The prefilter runs along x in one launch and along y and z in a second.  A thread owns
+// one column of R consecutive outputs along the filtered axis: R + 28 loads, all issued
+// before the first is used, and four operations an output (43 as a 29-tap FIR).
+// 301x301x233: x 52 us, yz 104 -> 86, the call 184 -> 170 (32 each at the copy rate: the 28 samples a thread reads
+// beyond its outputs, and the yz launch's three barriers with 20 waves per CU; 32 or 40
+// rows a tile took fewer samples but fewer waves, and 180 us for the whole call instead
+// of 173).
+constexpr int kBsX = 32;           // outputs per thread along x
 constexpr int kBsY = 24;           // outputs per thread along y (rows of the z tile)
-constexpr int kBsZ = 14;           // outputs per unit along z
-constexpr int kBsCols = 34 * kBsZ + 2 * kBsK;      // columns of a z tile (at most): 504
+constexpr int kBsZ = 27;           // outputs per unit along z (odd: neighbouring units in other LDS banks)
+constexpr int kBsCols = 17 * kBsZ + 2 * kBsK;      // columns of a z tile (at most): 487
 
 __global__ __launch_bounds__(256) void bspline_x(const float *__restrict__ src, float *__restrict__ dst, int n0,
                                                  long long plane, long long gx) {
     const long long p = blockIdx.x % gx * 256LL + threadIdx.x;
     const int x0 = (int)(blockIdx.x / gx) * kBsX;
     const long long pc = p < plane ? p : plane - 1;
-    float w[kBsX + 2 * kBsK];
-#pragma unroll
-    for (int i = 0; i < kBsX + 2 * kBsK; ++i)
-        w[i] = src[(long long)mirror_index(min(x0 + i - kBsK, n0 - 1 + kBsK), n0) * plane + pc];
+    float c[kBsX];
+    bs_line([&](int i) { return src[(long long)mirror_index(min(x0 + i - kBsK, n0 - 1 + kBsK), n0) * plane + pc]; }, c);
     if (p >= plane) return;
 #pragma unroll
     for (int i = 0; i < kBsX; ++i)
-        if (x0 + i < n0) dst[(long long)(x0 + i) * plane + p] = bs_fir(w, i + kBsK);
+        if (x0 + i < n0) dst[(long long)(x0 + i) * plane + p] = c[i];
 }
 
 // y in registers, then z through LDS: column c of a tile holds z = mirror(z0 - 14 + c),
-// kBsY rows; phase 2 takes units of 14 consecutive outputs of a row (42 LDS words), puts
-// the results back into the tile and stores whole rows.
+// kBsY rows; phase 2 takes units of kBsZ consecutive outputs of a row (one per thread,
+// kBsZ + 28 LDS words), puts the results back into the tile and stores whole rows.
 __global__ __launch_bounds__(512) void bspline_yz(const float *__restrict__ src, float *__restrict__ dst, int n1,
                                                   int n2, int zt, int ld, int nzt, int nyt, long long tiles) {
     extern __shared__ float tile[];
     const int tid = threadIdx.x;
     const int cols = zt + 2 * kBsK;
     const int upr = zt / kBsZ;                       // units per row
-    const int units = kBsY * upr;                    // at most 2 * blockDim (host)
+    const bool unit = tid < kBsY * upr;              // at most blockDim (host)
+    float *row = tile + (unit ? tid / upr * ld + tid % upr * kBsZ : 0);
     for (long long t = blockIdx.x; t < tiles; t += gridDim.x) {
         const int z0 = (int)(t % nzt) * zt, y0 = (int)(t / nzt % nyt) * kBsY;
         const long long base = t / nzt / nyt * n1 * n2;
         if (tid < cols) {
             const int z = mirror_index(min(z0 + tid - kBsK, n2 - 1 + kBsK), n2);
             const float *col = src + base + z;
-            float w[kBsY + 2 * kBsK];
+            float c[kBsY];
+            bs_line([&](int i) { return col[(long long)mirror_index(min(y0 + i - kBsK, n1 - 1 + kBsK), n1) * n2]; }, c);
 #pragma unroll
-            for (int i = 0; i < kBsY + 2 * kBsK; ++i)
-                w[i] = col[(long long)mirror_index(min(y0 + i - kBsK, n1 - 1 + kBsK), n1) * n2];
-#pragma unroll
-            for (int i = 0; i < kBsY; ++i) tile[i * ld + tid] = bs_fir(w, i + kBsK);
+            for (int i = 0; i < kBsY; ++i) tile[i * ld + tid] = c[i];
         }
         __syncthreads();
-        float r[2][kBsZ];
-#pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            const int u = tid + it * (int)blockDim.x;
-            if (u < units) {
-                const float *p = tile + (u / upr) * ld + (u % upr) * kBsZ;
-                float w[3 * kBsZ];
-#pragma unroll
-                for (int i = 0; i < 3 * kBsZ; ++i) w[i] = p[i];
-#pragma unroll
-                for (int i = 0; i < kBsZ; ++i) r[it][i] = bs_fir(w, i + kBsK);
-            }
-        }
+        float c[kBsZ];
+        if (unit) bs_line([&](int i) { return row[i]; }, c);
         __syncthreads();
+        if (unit) {
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            const int u = tid + it * (int)blockDim.x;
-            if (u < units) {
-                float *p = tile + (u / upr) * ld + (u % upr) * kBsZ;
-#pragma unroll
-                for (int i = 0; i < kBsZ; ++i) p[i] = r[it][i];
-            }
+            for (int i = 0; i < kBsZ; ++i) row[i] = c[i];
         }
         __syncthreads();
         const int nz = min(zt, n2 - z0), rows = min(kBsY, n1 - y0);
         for (int i = 0; i < rows; ++i)
-            for (int c = tid; c < nz; c += blockDim.x) dst[base + (long long)(y0 + i) * n2 + z0 + c] = tile[i * ld + c];
+            for (int k = tid; k < nz; k += blockDim.x) dst[base + (long long)(y0 + i) * n2 + z0 + k] = tile[i * ld + k];
         __syncthreads();
     }
 }
@@ -444,7 +444,7 @@ extern "C" int pvd_bspline_prefilter(const float *in, int n0, int n1, int n2, fl
     // z tiles of equal width, a multiple of the unit; a thread per column
     const int nt = (n2 + kBsCols - 2 * kBsK - 1) / (kBsCols - 2 * kBsK);
     const int zt = ((n2 + nt - 1) / nt + kBsZ - 1) / kBsZ * kBsZ;
-    const int block = (std::max(zt + 2 * kBsK, kBsY * (zt / kBsZ) / 2) + 63) / 64 * 64;
+    const int block = (std::max(zt + 2 * kBsK, kBsY * (zt / kBsZ)) + 63) / 64 * 64;
     const int ld = zt + 2 * kBsK + 1;
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(bspline_x, dim3((unsigned)blocks_x), dim3(256), 0, st, in, tmp, n0, plane, gx);

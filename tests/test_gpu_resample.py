@@ -123,3 +123,27 @@ def test_staged_interpolation_edges(shape, ratio):
         got = resample(img, (1.0, 1.0, 1.0), ratio, mode, output_shape=out_shape, scale=1.0)
         exp = ors.resample(img, (1.0, 1.0, 1.0), ratio, mode, shape=out_shape)
         np.testing.assert_allclose(got, exp, rtol=0, atol=tol * np.abs(img).max())
+
+
+@pytest.mark.parametrize("shape", [(40, 33, 29), (33, 25, 55), (70, 49, 81)])
+def test_prefilter_windows_and_what_a_non_finite_sample_reaches(shape):
+    """The prefilter at the edges of its windows (32 along x, 24 along y, 27 along z) against
+    the FP64 FIR, 2e-6 of max|image| (rounding of three FP32 recursions), and one infinite
+    sample: the outputs more than 14 + 2 samples from it along an axis stay as they were."""
+    from pyvoxeldosimetry_amd.resample import resample
+    _say("prefilter", shape)
+    rng = np.random.default_rng(sum(shape))
+    img = rng.normal(size=shape).astype(np.float32)
+    got = resample(img, (1.0, 1.0, 1.0), (1.0, 1.0, 1.0), "cubic", output_shape=shape, scale=1.0)
+    exp = ors.resample(img, (1.0, 1.0, 1.0), (1.0, 1.0, 1.0), "cubic", shape=shape)
+    np.testing.assert_allclose(got, exp, rtol=0, atol=2e-6 * np.abs(img).max())
+    at = (3, 2, 5)
+    bad = img.copy()
+    bad[at] = np.inf
+    out = resample(bad, (1.0, 1.0, 1.0), (1.0, 1.0, 1.0), "cubic", output_shape=shape, scale=1.0)
+    assert not np.isfinite(out[at])
+    far = np.zeros(shape, bool)
+    for a, p in enumerate(at):
+        i = np.arange(shape[a]).reshape([-1 if b == a else 1 for b in range(3)])
+        far |= np.abs(i - p) > 14 + 2
+    np.testing.assert_allclose(out[far], got[far], rtol=0, atol=2e-6 * np.abs(img).max())

@@ -643,8 +643,8 @@ constexpr int OUT_YS = 28;                                     // floats per hal
 template <int BX, int BY>
 constexpr size_t out_lds_bytes() { return (size_t)(BX + 2) * (BY + 2) * HZ * OUT_YS * 4; }
 
-// BX x BY rows per block: 2 x 4 (816 halo voxels, 26 row blocks of 32) for region lists,
-// 4 x 4 (1224, 39) for whole volumes; one thread per output voxel in the sums.
+// BX x BY rows per block: 2 x 4 (816 halo voxels, 26 row blocks of 32) for region lists;
+// one thread per output voxel in the sums.
 template <int BX, int BY>
 __global__ __launch_bounds__(FWD_THREADS) void cnn_conv_out(ConvArgs a) {
     constexpr int HYL = BY + 2;
@@ -716,6 +716,103 @@ __global__ __launch_bounds__(FWD_THREADS) void cnn_conv_out(ConvArgs a) {
                 a.y32[((long long)(x0 + ox) * a.n1 + (y0 + oy)) * a.n2 + z0 + z] = sum + b0;
             }
         }
+    }
+}
+
+// Whole volumes: the output layer marching along x.  A workgroup owns 8 y-rows x 32
+// z-voxels of one segment of planes; each input plane's halo (10 x 34 voxels) goes through
+// the tap GEMM once and its 27 values per voxel are added to the three output planes they
+// reach, whose sums a thread carries (the taps of a voxel are added plane after plane, in
+// tap order: the bits of the block form).  Y lies tap by tap (pitch 356 words: 16-byte
+// stores of 4 voxels and reads along z meet every bank once), in two buffers, with one
+// barrier a plane; the next two planes' loads are in flight during it.
+// Bound by the reads of h: 1.33 (y, z halo) x 1.13 (segments of 16) of 134 MB at 128^3.
+// 128^3 61 -> 31 us, 176x150x160 134 -> 61, 256x256x224 452 -> 219 (5.4 TB/s of h), against
+// 4 x 4-row blocks with two barriers a block, Y voxel by voxel (4-way bank conflicts) and no
+// load in flight over the sums; 64^3 and smaller the same.  A mask applied to a fetched
+// plane at once, instead of before its MFMAs, waits for the load: 44 us.
+constexpr int OM_Y = 8, OM_THREADS = 256, OM_HALO = (OM_Y + 2) * HZ, OM_GROUPS = (OM_HALO + 31) / 32, OM_PITCH = 356;
+constexpr size_t OM_LDS = 2 * (size_t)27 * OM_PITCH * 4;
+static_assert(OM_PITCH >= OM_GROUPS * 32 && OM_PITCH % 8 == 4, "a tap's row holds every group; odd in 16 bytes");
+
+__global__ __launch_bounds__(OM_THREADS) void cnn_conv_out_march(ConvArgs a, int seg, int nby, int nbz) {
+    extern __shared__ uint4 lds_u4[];
+    float *lds = reinterpret_cast<float *>(lds_u4);
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int m = lane & 31, kh = lane >> 5;
+    constexpr int NW = OM_THREADS / 64, GPW = (OM_GROUPS + NW - 1) / NW;
+    bf16x8 bw[2];
+#pragma unroll
+    for (int cc = 0; cc < 2; ++cc) {
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (m < 27) v = *reinterpret_cast<const uint4 *>(a.w + ((size_t)m * 32 * 32 + cc * 16 + kh * 8));
+        bw[cc] = __builtin_bit_cast(bf16x8, v);
+    }
+    const float b0 = a.bias ? a.bias[0] : 0.0f;
+    const int bz = blockIdx.x % nbz, by = blockIdx.x / nbz % nby, sx = blockIdx.x / (nbz * nby);
+    const int x0 = sx * seg, x1 = min(x0 + seg, a.n0), y0 = by * OM_Y, z0 = bz * 32;
+    const long long plane = (long long)a.n1 * a.n2;
+    // this lane's halo voxels: offset in a plane, or none
+    long long off[GPW];
+    bool in[GPW];
+#pragma unroll
+    for (int j = 0; j < GPW; ++j) {
+        const int u = (wave + j * NW) * 32 + m;
+        const int gy = y0 + u / HZ - 1, gz = z0 + u % HZ - 1;
+        in[j] = u < OM_HALO && gy >= 0 && gy < a.n1 && gz >= 0 && gz < a.n2;
+        off[j] = in[j] ? ((long long)gy * a.n2 + gz) * 32 + kh * 8 : kh * 8;
+    }
+    uint4 ring[2][GPW][2];                           // the two planes ahead
+    auto fetch = [&](int gx, uint4 (*av)[2]) {
+        const uint16_t *src = a.x + min(max(gx, 0), a.n0 - 1) * plane * 32;
+#pragma unroll
+        for (int j = 0; j < GPW; ++j)
+#pragma unroll
+            for (int cc = 0; cc < 2; ++cc) av[j][cc] = *reinterpret_cast<const uint4 *>(src + off[j] + cc * 16);
+    };
+    const int oy = tid >> 5, oz = tid & 31;
+    float s0 = 0.0f, s1 = 0.0f;                      // sums of planes p - 1 and p before plane p
+    auto step = [&](int p, uint4 (*av)[2], float *ys) {
+        const bool ix = p >= 0 && p < a.n0;
+#pragma unroll
+        for (int j = 0; j < GPW; ++j) {
+            const int g = wave + j * NW;
+            if (g >= OM_GROUPS) continue;            // wave-uniform
+            // (masked here, not when loaded: a use would wait for the load)
+#pragma unroll
+            for (int cc = 0; cc < 2; ++cc)
+                if (!(ix && in[j])) av[j][cc] = make_uint4(0u, 0u, 0u, 0u);
+            f32x16 acc = {};
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av[j][0]), bw[0], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av[j][1]), bw[1], acc, 0, 0, 0);
+            if (m < 27) {
+#pragma unroll
+                for (int i = 0; i < 16; i += 4)      // rows mfma_row(i ..): 4 consecutive voxels
+                    *reinterpret_cast<float4 *>(ys + m * OM_PITCH + g * 32 + mfma_row(i, lane)) =
+                        make_float4(acc[i], acc[i + 1], acc[i + 2], acc[i + 3]);
+            }
+        }
+        if (p + 2 <= x1) fetch(p + 2, av);
+        lds_barrier();       // Y of plane p; the other buffer's readers are past the previous one
+        const float *yr = ys + oy * HZ + oz;
+        float t0 = s0, t1 = s1, t2 = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            const int o = t / 3 * HZ + t % 3;
+            t2 += yr[t * OM_PITCH + o];              // dx = -1: plane p + 1
+            t1 += yr[(9 + t) * OM_PITCH + o];
+            t0 += yr[(18 + t) * OM_PITCH + o];       // dx = +1: plane p - 1, now complete
+        }
+        if (p > x0 && y0 + oy < a.n1)
+            a.y32[(p - 1) * plane + (long long)(y0 + oy) * a.n2 + z0 + oz] = t0 + b0;
+        s0 = t1;
+        s1 = t2;
+    };
+    fetch(x0 - 1, ring[0]);
+    fetch(x0, ring[1]);
+    for (int p = x0 - 1; p <= x1; p += 2) {
+        step(p, ring[0], lds);
+        if (p + 1 <= x1) step(p + 1, ring[1], lds + 27 * OM_PITCH);
     }
 }
 
@@ -1246,16 +1343,33 @@ hipError_t launch_out(const ConvArgs &a, int blocks, hipStream_t st) {
     return hipGetLastError();
 }
 
-// whole volumes (no region list): 4 x 4-row blocks for the input and output layers
-#ifndef PVD_CNN_IO44
-#define PVD_CNN_IO44 1
-#endif
+hipError_t launch_out_march(const ConvArgs &a, hipStream_t st) {
+    static bool attr = false;
+    if (!attr) {
+        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_out_march,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)OM_LDS);
+        if (e != hipSuccess) return e;
+        attr = true;
+    }
+    // two workgroups a CU (77 KB of LDS each), segments of at least 4 planes
+    const int nby = (a.n1 + OM_Y - 1) / OM_Y, nbz = a.n2 >> 5;
+    const long long cols = (long long)nby * nbz;
+    const long long want = std::max(1LL, 2LL * num_cus() / cols);
+    const int seg = std::max(4, (int)((a.n0 + want - 1) / want));
+    const long long grid = cols * ((a.n0 + seg - 1) / seg);
+    if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(cnn_conv_out_march, dim3((unsigned)grid), dim3(OM_THREADS), OM_LDS, st, a, seg, nby, nbz);
+    return hipGetLastError();
+}
+
+// whole volumes (no region list): 4 x 4-row blocks for the input layer, the marching
+// kernel for the output layer
 template <bool IN>
 hipError_t launch_io(const ConvArgs &a, int grid, bool whole, hipStream_t st) {
-    if (whole && PVD_CNN_IO44) {
+    if (whole && !IN) return launch_out_march(a, st);
+    if (whole) {
         const long long t = (long long)((a.n0 + 3) / 4) * ((a.n1 + 3) / 4) * (a.n2 >> 5);
-        const int g = (int)(t < num_cus() ? t : num_cus());
-        return IN ? launch_in<4, 4>(a, g, st) : launch_out<4, 4>(a, g, st);
+        return launch_in<4, 4>(a, (int)(t < num_cus() ? t : num_cus()), st);
     }
     return IN ? launch_in<FWD_BX, FWD_BY>(a, grid, st) : launch_out<FWD_BX, FWD_BY>(a, grid, st);
 }

@@ -129,6 +129,38 @@ def test_input_layer_with_four_live_channels(shape):
         _conv(lib, xt, 4, wt, bt, nat.PVD_CNN_EPI_LINEAR_F32, shape, y32=r)
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 32), (2, 8, 32), (5, 9, 64), (9, 17, 96), (70, 40, 128)])
+def test_output_layer_marching_edges(shape):
+    """The output layer of whole volumes at the edges of its 8-row columns and segments,
+    against the FP64 oracle and bit for bit against the block kernel (a region list of every
+    block).  FP32 sums of 27 taps of 32 products: 1e-4 of values of order 5, as above."""
+    import ctypes
+    import torch
+    from pyvoxeldosimetry_amd import _native as nat
+    _say("cnn output layer", shape)
+    lib = nat.load()
+    rng = np.random.default_rng(sum(shape))
+    n = int(np.prod(shape))
+    x = ocnn.bf16_round(rng.normal(size=shape + (32,)).astype(np.float32))
+    w = ocnn.bf16_round(rng.normal(scale=0.1, size=(27, 32, 32)).astype(np.float32))
+    b = rng.normal(scale=0.1, size=32).astype(np.float32)
+    xt, wt, bt = bf(x).reshape(n, 32), bf(w), torch.from_numpy(b).cuda()
+    r, q = torch.empty(n, device="cuda"), torch.empty(n, device="cuda")
+    _conv(lib, xt, 32, wt, bt, nat.PVD_CNN_EPI_LINEAR_F32, shape, y32=r)
+    w0 = np.zeros_like(w)
+    w0[:, 0] = w[:, 0]
+    z = ocnn.conv3(x, w0)[..., 0] + b[0]
+    np.testing.assert_allclose(r.cpu().numpy().reshape(shape), z, rtol=1e-5, atol=1e-4)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    nblk = -(-shape[0] // 2) * -(-shape[1] // 4) * (shape[2] // 32)
+    blocks = torch.arange(nblk, device="cuda", dtype=torch.int32)
+    count = torch.tensor([nblk], device="cuda", dtype=torch.int32)
+    nat.check(lib.pvd_cnn_conv_fwd(p(xt), 32, p(wt), p(bt), nat.PVD_CNN_EPI_LINEAR_F32, None, None, None, p(q),
+                                   *shape, p(blocks), p(count), None), "pvd_cnn_conv_fwd")
+    torch.cuda.synchronize()
+    assert torch.equal(r, q)
+
+
 @pytest.mark.parametrize("cin", [16, 32])
 def test_conv_forward_many_blocks_per_workgroup(cin):
     """A grid with more output blocks than workgroups (ragged in x and y): every

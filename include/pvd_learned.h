@@ -85,6 +85,14 @@ int pvd_cnn_conv_fwd(const void *x, int cin, const void *w, const float *bias, i
                      void *y, void *act, float *y32, int n0, int n1, int n2, const int *blocks, const int *nblocks,
                      void *stream);
 
+/* The ReLU input layer from the FP32 maps: pvd_cnn_pack_inputs and pvd_cnn_conv_fwd (cin 4)
+ * in one pass, the same bits.  The maps have rows of n2 voxels `pitch` floats apart (a
+ * volume's nz; larger than n2 for a slab along z of a larger volume, which ends in zeros
+ * like the volume itself).  w [27][32][16] and bias as there; y 16-byte aligned. */
+int pvd_cnn_input_layer(const float *activity, const float *density, const float *dose_plain, const float *act_max,
+                        const float *dose_max, long long pitch, const void *w, const float *bias, void *y, int n0,
+                        int n1, int n2, const int *blocks, const int *nblocks, void *stream);
+
 /* Training forward of a whole volume: the ReLU input layer (cin 4) or a residual layer
  * y = x + relu(conv(x) + b) (cin 32) as in pvd_cnn_conv_fwd, and mask[v], whose bit c is
  * set where the BF16 of relu(...) of channel c is not 0 (the activations themselves are

@@ -90,6 +90,7 @@ SIGNATURES = {
     # include/pvd_learned.h
     "pvd_mc_dose": (_I, [ctypes.c_void_p, _P, _P, _P, _P, _P]),
     "pvd_cnn_conv_fwd": (_I, [_P, _I, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _P, _P, _P]),
+    "pvd_cnn_input_layer": (_I, [_P, _P, _P, _P, _P, ctypes.c_longlong, _P, _P, _P, _I, _I, _I, _P, _P, _P]),
     "pvd_cnn_train_layer": (_I, [_P, _I, _P, _P, _P, _P, _I, _I, _I, _P]),
     "pvd_cnn_grad_parts": (ctypes.c_size_t, [_I, _I, _I]),
     "pvd_cnn_layer_grad": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),

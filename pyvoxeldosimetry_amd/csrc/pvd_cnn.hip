@@ -520,10 +520,30 @@ constexpr size_t in_lds_bytes() {
     return (size_t)IN_CHUNKS * 32 * IN_WS + (size_t)in_halo<BX, BY>() * 8 + (size_t)(FWD_THREADS / 64) * FWD_STAGE;
 }
 
+// the network's inputs as FP32 maps (rows of n2 voxels `pitch` floats apart) and the device
+// maxima that scale the activity and the plain dose
+struct InMaps {
+    const float *map[3];               // activity, density, plain dose
+    const float *amax, *dmax;
+    long long pitch;
+};
+
+__device__ __forceinline__ float inv_scale(const float *m) { return 1.0f / fmaxf(*m, 1e-30f); }
+
+// the packer's four channels of one voxel
+__device__ __forceinline__ uint2 pack_input(float act, float dens, float dose, float sa, float sd) {
+    return make_uint2((uint32_t)f2bf(act * sa) | (uint32_t)f2bf(dens) << 16, (uint32_t)f2bf(dose * sd));
+}
+
 // BX x BY rows per block (2 x 4: the blocks of region lists; 4 x 4 for whole volumes,
-// less halo per output); each of the 8 waves computes BX * BY / 8 rows.
-template <int BX, int BY>
-__global__ __launch_bounds__(FWD_THREADS) void cnn_conv_in(ConvArgs a) {
+// less halo per output); each of the 8 waves computes BX * BY / 8 rows.  MAPS: the halo
+// comes from the FP32 maps and is packed on its way into LDS (the same bits): 12 bytes a
+// voxel instead of a pack pass (12 in, 32 out) and 32 bytes of which 8 are live.  128^3:
+// pack 14.5 + 40.5 us -> 45.0, 512x256x224: 288 + 546 -> 556.  What is left is each block's
+// two barriers and its epilogue (134 MB of y at 3 TB/s); twice the workgroups per CU (128
+// VGPRs) measured 45.0 and 669.
+template <int BX, int BY, bool MAPS>
+__global__ __launch_bounds__(FWD_THREADS) void cnn_conv_in(ConvArgs a, InMaps mp) {
     constexpr int IN_HALO = in_halo<BX, BY>(), HYL = BY + 2, NR = BX * BY / 8;
     static_assert(NR * 8 == BX * BY, "whole rows per wave");
     extern __shared__ uint4 lds_u4[];
@@ -549,18 +569,30 @@ __global__ __launch_bounds__(FWD_THREADS) void cnn_conv_in(ConvArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) bias4[g][j] = a.bias ? a.bias[8 * g + 4 * kh + j] : 0.0f;
     constexpr int PER_T = (IN_HALO + FWD_THREADS - 1) / FWD_THREADS;
-    uint2 pf[PER_T];
+    uint2 pf[MAPS ? 1 : PER_T];
+    float pm[MAPS ? PER_T : 1][3];
+    uint32_t inside = 0;                 // MAPS: bit u, voxel u of this thread lies in the volume
+    const float sa = MAPS ? inv_scale(mp.amax) : 0.0f, sd = MAPS ? inv_scale(mp.dmax) : 0.0f;
     auto fetch = [&](int b) {
         const int bz = b % nbz, by = (b / nbz) % nby, bx = b / (nbz * nby);
         const int x0 = bx * BX, y0 = by * BY, z0 = bz * 32;
+        inside = 0;
 #pragma unroll
         for (int u = 0; u < PER_T; ++u) {
             const int vox = tid + u * FWD_THREADS;
             const int hz = vox % HZ, hy = (vox / HZ) % HYL, hx = vox / (HZ * HYL);
             const int gx = x0 + hx - 1, gy = y0 + hy - 1, gz = z0 + hz - 1;
-            pf[u] = make_uint2(0u, 0u);
-            if (vox < IN_HALO && gx >= 0 && gx < a.n0 && gy >= 0 && gy < a.n1 && gz >= 0 && gz < a.n2)
-                pf[u] = *reinterpret_cast<const uint2 *>(a.x + (((long long)gx * a.n1 + gy) * a.n2 + gz) * 16);
+            const bool in = vox < IN_HALO && gx >= 0 && gx < a.n0 && gy >= 0 && gy < a.n1 && gz >= 0 && gz < a.n2;
+            if constexpr (MAPS) {
+                // (read at voxel 0 where outside and masked when packed)
+                const long long o = in ? ((long long)gx * a.n1 + gy) * mp.pitch + gz : 0;
+                inside |= (uint32_t)in << u;
+#pragma unroll
+                for (int c = 0; c < 3; ++c) pm[u][c] = mp.map[c][o];
+            } else {
+                pf[u] = make_uint2(0u, 0u);
+                if (in) pf[u] = *reinterpret_cast<const uint2 *>(a.x + (((long long)gx * a.n1 + gy) * a.n2 + gz) * 16);
+            }
         }
     };
     if ((int)blockIdx.x < total) fetch(block_of(blockIdx.x));
@@ -572,7 +604,14 @@ __global__ __launch_bounds__(FWD_THREADS) void cnn_conv_in(ConvArgs a) {
 #pragma unroll
         for (int u = 0; u < PER_T; ++u) {
             const int vox = tid + u * FWD_THREADS;
-            if (vox < IN_HALO) *reinterpret_cast<uint2 *>(hl + vox * 8) = pf[u];
+            if (vox < IN_HALO) {
+                if constexpr (MAPS) {
+                    const uint2 v = pack_input(pm[u][0], pm[u][1], pm[u][2], sa, sd);
+                    *reinterpret_cast<uint2 *>(hl + vox * 8) = (inside >> u) & 1u ? v : make_uint2(0u, 0u);
+                } else {
+                    *reinterpret_cast<uint2 *>(hl + vox * 8) = pf[u];
+                }
+            }
         }
         lds_barrier();
         if (bi + (int)gridDim.x < total) fetch(block_of(bi + gridDim.x));
@@ -1103,17 +1142,15 @@ __global__ __launch_bounds__(RED_COLS * RED_GROUPS) void reduce_rows(const float
     if (g == 0 && c < cols) out[c] = accumulate ? out[c] + red[0][l] : red[0][l];
 }
 
-__device__ __forceinline__ float inv_scale(const float *m) { return 1.0f / fmaxf(*m, 1e-30f); }
-
 __global__ __launch_bounds__(256) void cnn_pack(const float *__restrict__ a, const float *__restrict__ d,
                                                 const float *__restrict__ dp, const float *__restrict__ amax,
                                                 const float *__restrict__ dmax, uint16_t *__restrict__ x,
                                                 long long n) {
     const float sa = inv_scale(amax), sd = inv_scale(dmax);
     for (long long v = blockIdx.x * 256LL + threadIdx.x; v < n; v += (long long)gridDim.x * 256) {
-        const uint32_t c0 = f2bf(a[v] * sa), c1 = f2bf(d[v]), c2 = f2bf(dp[v] * sd);
+        const uint2 c = pack_input(a[v], d[v], dp[v], sa, sd);
         uint4 *row = reinterpret_cast<uint4 *>(x + v * 16);
-        row[0] = make_uint4(c0 | (c1 << 16), c2, 0u, 0u);
+        row[0] = make_uint4(c.x, c.y, 0u, 0u);
         row[1] = make_uint4(0u, 0u, 0u, 0u);
     }
 }
@@ -1315,18 +1352,23 @@ hipError_t launch_layer(const ConvArgs &a, hipStream_t st) {
     return a.mask ? launch_march<MR_MASK>(q, st) : launch_march<MR_FWD>(q, st);
 }
 
-template <int BX, int BY>
-hipError_t launch_in(const ConvArgs &a, int blocks, hipStream_t st) {
+template <int BX, int BY, bool MAPS>
+hipError_t launch_in_as(const ConvArgs &a, const InMaps &mp, int blocks, hipStream_t st) {
     static bool attr = false;
     constexpr size_t lds = in_lds_bytes<BX, BY>();
     if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_in<BX, BY>,
+        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_in<BX, BY, MAPS>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
         attr = true;
     }
-    hipLaunchKernelGGL((cnn_conv_in<BX, BY>), dim3(blocks), dim3(FWD_THREADS), lds, st, a);
+    hipLaunchKernelGGL((cnn_conv_in<BX, BY, MAPS>), dim3(blocks), dim3(FWD_THREADS), lds, st, a, mp);
     return hipGetLastError();
+}
+
+template <int BX, int BY>
+hipError_t launch_in(const ConvArgs &a, const InMaps *mp, int blocks, hipStream_t st) {
+    return mp ? launch_in_as<BX, BY, true>(a, *mp, blocks, st) : launch_in_as<BX, BY, false>(a, InMaps{}, blocks, st);
 }
 
 template <int BX, int BY>
@@ -1365,13 +1407,13 @@ hipError_t launch_out_march(const ConvArgs &a, hipStream_t st) {
 // whole volumes (no region list): 4 x 4-row blocks for the input layer, the marching
 // kernel for the output layer
 template <bool IN>
-hipError_t launch_io(const ConvArgs &a, int grid, bool whole, hipStream_t st) {
+hipError_t launch_io(const ConvArgs &a, int grid, bool whole, hipStream_t st, const InMaps *mp = nullptr) {
     if (whole && !IN) return launch_out_march(a, st);
     if (whole) {
         const long long t = (long long)((a.n0 + 3) / 4) * ((a.n1 + 3) / 4) * (a.n2 >> 5);
-        return launch_in<4, 4>(a, (int)(t < num_cus() ? t : num_cus()), st);
+        return launch_in<4, 4>(a, mp, (int)(t < num_cus() ? t : num_cus()), st);
     }
-    return IN ? launch_in<FWD_BX, FWD_BY>(a, grid, st) : launch_out<FWD_BX, FWD_BY>(a, grid, st);
+    return IN ? launch_in<FWD_BX, FWD_BY>(a, mp, grid, st) : launch_out<FWD_BX, FWD_BY>(a, grid, st);
 }
 
 template <int CIN>
@@ -1451,6 +1493,24 @@ int pvd_cnn_conv_fwd(const void *x, int cin, const void *w, const float *bias, i
         }
     }
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch CNN convolution");
+}
+
+int pvd_cnn_input_layer(const float *activity, const float *density, const float *dose_plain, const float *act_max,
+                        const float *dose_max, long long pitch, const void *w, const float *bias, void *y, int n0,
+                        int n1, int n2, const int *blocks, const int *nblocks, void *stream) {
+    if ((blocks == nullptr) != (nblocks == nullptr)) return pvd_set_error(PVD_EINVAL, "blocks and nblocks go together");
+    if (int rc = check_grid(n0, n1, n2)) return rc;
+    if (!activity || !density || !dose_plain || !act_max || !dose_max || !w || !y)
+        return pvd_set_error(PVD_EINVAL, "null argument");
+    if (pitch < n2) return pvd_set_error(PVD_EINVAL, "pitch %lld below the row length %d", pitch, n2);
+    if (reinterpret_cast<uintptr_t>(y) & 15) return pvd_set_error(PVD_EINVAL, "y must be 16-byte aligned");
+    const ConvArgs a{nullptr, (const uint16_t *)w, bias, nullptr, (uint16_t *)y, nullptr, nullptr, n0, n1, n2, blocks,
+                     nblocks, nullptr};
+    const InMaps mp{{activity, density, dose_plain}, act_max, dose_max, pitch};
+    const long long total = (long long)((n0 + FWD_BX - 1) / FWD_BX) * ((n1 + FWD_BY - 1) / FWD_BY) * (n2 >> 5);
+    const hipError_t e = launch_io<true>(a, (int)(total < num_cus() ? total : num_cus()), blocks == nullptr,
+                                         (hipStream_t)stream, &mp);
+    return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch CNN input layer");
 }
 
 int pvd_cnn_train_layer(const void *x, int cin, const void *w, const float *bias, void *y, unsigned *mask, int n0,

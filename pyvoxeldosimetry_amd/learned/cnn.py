@@ -151,8 +151,10 @@ class ResidualCNN:
                   "pvd_cnn_conv_fwd")
 
     # ------------------------------------------------------------------ forward / backward
-    def forward(self, x, shape, keep_activations: bool = True, blocks=None):
-        """x: BF16 [n, 16] inputs; returns the FP32 correction r [n] (workspace tensor).
+    def forward(self, x, shape, keep_activations: bool = True, blocks=None, maps=None):
+        """x: BF16 [n, 16] inputs, or (inference) ``maps``: activity, density and plain dose,
+        FP32, the device maxima of activity and plain dose that scale them, and the pitch
+        of the maps' rows in floats; returns the FP32 correction r [n] (workspace tensor).
         ``keep_activations=False`` (inference) skips the ReLU masks backward needs (a
         whole-volume forward writes them).
         ``blocks``: (block list, count) device tensors from ``pvd_cnn_region_blocks``:
@@ -167,7 +169,13 @@ class ResidualCNN:
                                                        shape[0], shape[1], shape[2], self._stream()),
                           "pvd_cnn_train_layer")
         else:
-            self._conv(x, 4, 0, nat.PVD_CNN_EPI_RELU, shape, y=h[0], blocks=blocks)
+            if maps is not None:
+                bl, bn = blocks if blocks is not None else (None, None)
+                nat.check(self.lib.pvd_cnn_input_layer(*(_p(t) for t in maps[:5]), maps[5], _p(self.w_bf16(0)),
+                                                       _p(self.bias(0)), _p(h[0]), *shape, _p(bl), _p(bn),
+                                                       self._stream()), "pvd_cnn_input_layer")
+            else:
+                self._conv(x, 4, 0, nat.PVD_CNN_EPI_RELU, shape, y=h[0], blocks=blocks)
             for l in range(1, 5):
                 self._conv(h[l - 1], 32, l, nat.PVD_CNN_EPI_RESID_RELU, shape, y=h[l], resid=h[l - 1], blocks=blocks)
         self._conv(h[4], 32, 5, nat.PVD_CNN_EPI_LINEAR_F32, shape, y32=ws["r"], blocks=blocks)

@@ -245,14 +245,15 @@ class LearnedCorrector:
         if e < 32:
             raise ValueError("tile_z must be at least 32")
         halo = 6
+        act, rho = act.contiguous(), rho.contiguous()
         amax, dmax = self.input_maxima(act, dp)
         r = torch.empty(shape, dtype=torch.float32, device=self.device)
         for s0, s1, a, b in z_slabs(nz, e, halo):
             sl = (slice(None), slice(None), slice(s0, s1))
-            xs, _ = self.pack(act[sl].contiguous(), rho[sl].contiguous(), dp[sl].contiguous(), scales=(amax, dmax))
             sshape = (shape[0], shape[1], s1 - s0)
             blocks = self.region_blocks(dp[sl].contiguous(), dmax, self.region_frac) if region else None
-            rs = self.net.forward(xs, sshape, keep_activations=False, blocks=blocks).reshape(sshape)
+            rs = self.net.forward(None, sshape, keep_activations=False, blocks=blocks,
+                                  maps=(act[sl], rho[sl], dp[sl], amax, dmax, nz)).reshape(sshape)
             r[:, :, a:b] = rs[:, :, a - s0:b - s0]
         self._keep_scales = (amax, dmax)
         return r.reshape(-1), dmax
@@ -275,9 +276,11 @@ class LearnedCorrector:
             ext = tile_z or slab_extent(shape[2], shape[0] * shape[1])
             r, dmax = self.network_tiled(act, rho, dp, ext, region)
         elif r_override is None:
-            x, dmax = self.pack(act, rho, dp)
+            amax, dmax = self.input_maxima(act, dp)
             blocks = self.region_blocks(dp, dmax, apply_frac) if region else None
-            r = self.net.forward(x, shape, keep_activations=False, blocks=blocks)
+            r = self.net.forward(None, shape, keep_activations=False, blocks=blocks,
+                                 maps=(act.contiguous(), rho.contiguous(), dp, amax, dmax, shape[2]))
+            self._keep = (amax, dmax)      # alive until the next call, past the asynchronous kernels
         else:
             dmax = dp.max().reshape(1)
             r = r_override.reshape(-1).contiguous()

@@ -129,6 +129,47 @@ def test_input_layer_with_four_live_channels(shape):
         _conv(lib, xt, 4, wt, bt, nat.PVD_CNN_EPI_LINEAR_F32, shape, y32=r)
 
 
+@pytest.mark.parametrize("shape,z0", [((1, 1, 32), 0), ((3, 5, 32), 7), ((5, 9, 64), 0), ((9, 6, 96), 3)])
+def test_input_layer_from_maps_gives_the_packed_bits(shape, z0):
+    """The input layer from the FP32 maps, a volume or a slab along z of a deeper one, whole
+    and through a region list: the bits of packing and the cin = 4 layer (which the test
+    above checks against the oracle), a NaN voxel and infinities included."""
+    import ctypes
+    import torch
+    from pyvoxeldosimetry_amd import _native as nat
+    _say("cnn input layer from maps", shape, z0)
+    lib = nat.load()
+    g = torch.Generator(device="cuda").manual_seed(sum(shape))
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    n, pitch = int(np.prod(shape)), shape[2] + 2 * z0
+    full = [torch.randn(shape[:2] + (pitch,), device="cuda", generator=g) * s for s in (0.1, 1.0, 3.0)]
+    full[0][0, 0, z0 + 1], full[1][0, 0, z0 + 9], full[2][-1, -1, z0 + 30] = float("nan"), float("inf"), -float("inf")
+    slab = [t[:, :, z0:z0 + shape[2]] for t in full]
+    mx = torch.tensor([0.4, 9.0], device="cuda")
+    w = (torch.randn((27, 32, 16), device="cuda", generator=g) * 0.1).to(torch.bfloat16)
+    b = torch.randn(32, device="cuda", generator=g) * 0.1
+    x = torch.empty((n, 16), dtype=torch.bfloat16, device="cuda")
+    dense = [t.contiguous() for t in slab]
+    nat.check(lib.pvd_cnn_pack_inputs(*(p(t) for t in dense), p(mx), p(mx[1:]), p(x), n, None), "pack")
+    want = torch.empty((n, 32), dtype=torch.bfloat16, device="cuda")
+    torch.cuda.synchronize()
+    _conv(lib, x, 4, w, b, nat.PVD_CNN_EPI_RELU, shape, y=want)
+    nblk = -(-shape[0] // 2) * -(-shape[1] // 4) * (shape[2] // 32)
+    blocks = torch.arange(nblk, device="cuda", dtype=torch.int32)
+    count = torch.tensor([nblk], device="cuda", dtype=torch.int32)
+    torch.cuda.synchronize()
+    for lists in ((None, None), (p(blocks), p(count))):
+        got = torch.zeros_like(want)
+        torch.cuda.synchronize()
+        nat.check(lib.pvd_cnn_input_layer(*(p(t) for t in slab), p(mx), p(mx[1:]), pitch, p(w), p(b), p(got), *shape,
+                                          *lists, None), "pvd_cnn_input_layer")
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    with pytest.raises(ValueError):
+        nat.check(lib.pvd_cnn_input_layer(*(p(t) for t in slab), p(mx), p(mx[1:]), shape[2] - 1, p(w), p(b), p(want),
+                                          *shape, None, None, None), "pvd_cnn_input_layer")
+
+
 @pytest.mark.parametrize("shape", [(1, 1, 32), (2, 8, 32), (5, 9, 64), (9, 17, 96), (70, 40, 128)])
 def test_output_layer_marching_edges(shape):
     """The output layer of whole volumes at the edges of its 8-row columns and segments,

@@ -144,6 +144,21 @@ int pvd_cnn_wgrad(const void *x, int cin, const void *dz, float *dw, float *work
 int pvd_cnn_loss(const float *r, const float *dp, const float *dt, const float *m, long long n_voxels,
                  float inv_count, void *dr, float *loss_part, void *stream);
 
+/* The output layer's gradients, whose dL/dr has one channel (dr: BF16 [n]):
+ *   pvd_cnn_out_loss  pvd_cnn_loss with dr as [n] instead of channel 0 of [n][32]
+ *   pvd_cnn_out_wgrad dw[tap][0][ci] of dw [27][32][32] = sum_v x[v + d(tap)][ci] dr[v]; the
+ *                     rows of the other outputs are left alone; work as for pvd_cnn_wgrad
+ *   pvd_cnn_out_grad  pvd_cnn_layer_grad of that layer from w [27][32][32] as it is (not
+ *                     flipped; output channel 0), dh_in = 0; pvd_cnn_out_grad_parts rows
+ *                     of dbias_part
+ * x, dh_out and dz_out 16-byte aligned. */
+int pvd_cnn_out_loss(const float *r, const float *dp, const float *dt, const float *m, long long n_voxels,
+                     float inv_count, void *dr, float *loss_part, void *stream);
+int pvd_cnn_out_wgrad(const void *x, const void *dr, float *dw, float *work, int n0, int n1, int n2, void *stream);
+size_t pvd_cnn_out_grad_parts(int n0, int n1, int n2);
+int pvd_cnn_out_grad(const void *dr, const void *w, float *dh_out, const unsigned *mask, void *dz_out, float *dbias_part,
+                     int n0, int n1, int n2, void *stream);
+
 /* Adam on FP32 master weights; also refreshes the BF16 copy. */
 int pvd_cnn_adam(float *param, const float *grad, float *m, float *v, void *param_bf16, long long n, float lr,
                  float beta1, float beta2, float eps, int step, void *stream);

@@ -93,6 +93,7 @@ SIGNATURES = {
     "pvd_cnn_input_layer": (_I, [_P, _P, _P, _P, _P, ctypes.c_longlong, _P, _P, _P, _I, _I, _I, _P, _P, _P]),
     "pvd_cnn_train_layer": (_I, [_P, _I, _P, _P, _P, _P, _I, _I, _I, _P]),
     "pvd_cnn_grad_parts": (ctypes.c_size_t, [_I, _I, _I]),
+    "pvd_cnn_out_grad_parts": (ctypes.c_size_t, [_I, _I, _I]),
     "pvd_cnn_layer_grad": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),
     "pvd_cnn_region_block_count": (ctypes.c_size_t, [_I, _I, _I]),
     "pvd_cnn_region_blocks": (_I, [_P, _I, _I, _I, _P, ctypes.c_float, _P, _P, _P, _P]),
@@ -100,6 +101,9 @@ SIGNATURES = {
     "pvd_cnn_relu_grad": (_I, [_P, _P, _P, _P, ctypes.c_longlong, _P]),
     "pvd_cnn_wgrad_work_floats": (ctypes.c_size_t, [_I, _I, _I]),
     "pvd_cnn_wgrad": (_I, [_P, _I, _P, _P, _P, _I, _I, _I, _P]),
+    "pvd_cnn_out_loss": (_I, [_P, _P, _P, _P, ctypes.c_longlong, ctypes.c_float, _P, _P, _P]),
+    "pvd_cnn_out_wgrad": (_I, [_P, _P, _P, _P, _I, _I, _I, _P]),
+    "pvd_cnn_out_grad": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),
     "pvd_cnn_loss": (_I, [_P, _P, _P, _P, ctypes.c_longlong, ctypes.c_float, _P, _P, _P]),
     "pvd_cnn_adam": (_I, [_P, _P, _P, _P, _P, ctypes.c_longlong, ctypes.c_float, ctypes.c_float, ctypes.c_float,
                           ctypes.c_float, _I, _P]),

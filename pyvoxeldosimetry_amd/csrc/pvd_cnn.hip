@@ -1030,6 +1030,219 @@ __global__ __launch_bounds__(WG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 }
 
 // ---------------------------------------------------------------------------------
+// Gradients of the output layer.  Its dL/dr has one channel, kept as BF16 [n] rather than
+// channel 0 of 32 (the kernels above would compute 31 channels of zeros on 134 MB of them).
+//
+// Weights: dw[t][ci] = sum_u x[u][ci] dr[u - d(t)], one GEMM of the 27 taps (32 rows)
+// against the 32 channels instead of a GEMM per tap; x is read once, without a halo.  A
+// tile is 8 rows of 32 voxels, a row per wave: x channels-last as in cnn_wgrad (transposing
+// reads), the dr halo in three copies shifted by one voxel so that a tap's 8 voxels are one
+// aligned read.  Bound by reading x: 128^3 123 us (cnn_wgrad on 32 channels of dr) -> 30
+// (134 MB at 4.5 TB/s).
+constexpr int OW_Y = 8, OW_ROW = 80, OW_HALO = 3 * (OW_Y + 2) * HZ;      // bytes of a dr row, halo voxels
+constexpr int OW_XB = OW_Y * 32 * 64, OW_PL = (OW_Y + 2) * OW_ROW, OW_COPY = 3 * OW_PL, OW_BUF = OW_XB + 3 * OW_COPY;
+constexpr int OW_RED = 8 * 27 * 32 * 4;
+constexpr size_t OW_LDS = 2 * OW_BUF > OW_RED ? 2 * OW_BUF : OW_RED;
+constexpr int OW_BLOCKS_PER_CU = 3;
+
+__global__ __launch_bounds__(WG_THREADS) void cnn_out_wgrad(WgradArgs a) {
+    extern __shared__ uint4 lds_u4[];
+    char *lds = reinterpret_cast<char *>(lds_u4);
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int m = lane & 31, kh = lane >> 5;
+    const int nby = (a.n1 + OW_Y - 1) / OW_Y, nbz = a.n2 >> 5, total = a.n0 * nby * nbz;
+    const int tv = (lane >> 5) * 8 + ((lane & 15) >> 2), tc = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+    const int tap = min(m, 26), dx = tap / 9 - 1, dy = tap / 3 % 3 - 1, dz = tap % 3 - 1;
+    const int aoff = OW_XB + (1 - dz) * OW_COPY + (1 - dx) * OW_PL + (wave + 1 - dy) * OW_ROW + kh * 16;
+    const int boff = wave * 32 * 64 + tv * 64 + tc * 2;
+    constexpr int NX = OW_Y * 32 * 4 / WG_THREADS, ND = (OW_HALO + WG_THREADS - 1) / WG_THREADS;
+    uint4 px[NX];
+    uint16_t pd[ND];
+    uint32_t xin = 0, din = 0;             // which of them lie in the volume
+    auto fetch = [&](int b) {
+        const int z0 = b % nbz * 32, y0 = b / nbz % nby * OW_Y, x0 = b / (nbz * nby);
+        xin = din = 0;
+#pragma unroll
+        for (int u = 0; u < NX; ++u) {
+            const int i = tid + u * WG_THREADS, oy = y0 + (i >> 7);
+            xin |= (uint32_t)(oy < a.n1) << u;
+            px[u] = reinterpret_cast<const uint4 *>(
+                a.x + (((long long)x0 * a.n1 + min(oy, a.n1 - 1)) * a.n2 + z0 + ((i >> 2) & 31)) * 32)[i & 3];
+        }
+#pragma unroll
+        for (int u = 0; u < ND; ++u) {
+            const int e = tid + u * WG_THREADS, hz = e % HZ, row = e / HZ % (OW_Y + 2), pl = e / (HZ * (OW_Y + 2));
+            const int gx = x0 + pl - 1, gy = y0 + row - 1, gz = z0 + hz - 1;
+            const bool in = e < OW_HALO && gx >= 0 && gx < a.n0 && gy >= 0 && gy < a.n1 && gz >= 0 && gz < a.n2;
+            din |= (uint32_t)in << u;
+            pd[u] = a.dz[in ? ((long long)gx * a.n1 + gy) * a.n2 + gz : 0];
+        }
+    };
+    auto put = [&](char *buf) {
+#pragma unroll
+        for (int u = 0; u < NX; ++u)
+            reinterpret_cast<uint4 *>(buf)[tid + u * WG_THREADS] = (xin >> u) & 1u ? px[u] : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+        for (int u = 0; u < ND; ++u) {
+            const int e = tid + u * WG_THREADS, hz = e % HZ, row = e / HZ % (OW_Y + 2), pl = e / (HZ * (OW_Y + 2));
+            if (e >= OW_HALO) continue;
+            const uint16_t v = (din >> u) & 1u ? pd[u] : (uint16_t)0;
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                if (hz >= c && hz - c < 32)
+                    *reinterpret_cast<uint16_t *>(buf + OW_XB + c * OW_COPY + pl * OW_PL + row * OW_ROW + (hz - c) * 2) = v;
+        }
+    };
+    f32x16 acc[2] = {f32x16{}, f32x16{}};
+    if ((int)blockIdx.x < total) {
+        fetch(blockIdx.x);
+        put(lds);
+    }
+    int cur = 0;
+    for (int b = blockIdx.x; b < total; b += gridDim.x, cur ^= 1) {
+        lds_barrier();     // this tile's buffer written; the other one read by every wave
+        const char *buf = lds + cur * OW_BUF;
+        if (b + (int)gridDim.x < total) fetch(b + gridDim.x);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            uint4 f = *reinterpret_cast<const uint4 *>(buf + aoff + c * 32);
+            if (m >= 27) f = make_uint4(0u, 0u, 0u, 0u);
+            const uint2 b0 = lds_read_tr(buf + boff + c * 16 * 64), b1 = lds_read_tr(buf + boff + (c * 16 + 4) * 64);
+            acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, f), frag4(b0.x, b0.y, b1.x, b1.y),
+                                                             acc[c], 0, 0, 0);
+        }
+        if (b + (int)gridDim.x < total) put(lds + (cur ^ 1) * OW_BUF);
+    }
+    // work[blockIdx][tap][ci]: the waves' sums in wave order
+    float *red = reinterpret_cast<float *>(lds_u4);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int t = mfma_row(i, lane);
+        if (t < 27) red[(wave * 27 + t) * 32 + m] = acc[0][i] + acc[1][i];
+    }
+    __syncthreads();
+    for (int e = tid; e < 27 * 32; e += WG_THREADS) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) sum += red[w * 27 * 32 + e];
+        a.work[(size_t)blockIdx.x * 27 * 32 + e] = sum;
+    }
+}
+
+// Input: dh[v][ci] = sum_t dr[v + d(t)] w[26 - t][0][ci], the 27 taps as one K of 32 (two
+// MFMAs per 32 voxels instead of 54), with the epilogue of cnn_conv_march's first gradient
+// layer (dh, ReLU mask, dz', channel sums) and its columns; dr planes (8 + 2 rows) go round a ring of four.  Bound by storing dh and dz'
+// (402 MB at 128^3): 106 us (cnn_conv_march on 32 channels of dr) -> 85; 98 with that
+// kernel's segments, one workgroup a CU.
+constexpr int OG_ROW = 36, OG_PLANE = (MR_Y + 2) * OG_ROW;               // voxels of a dr row, a plane
+constexpr size_t OG_LDS = 4 * OG_PLANE * 2 + 8 * FWD_STAGE;
+
+__global__ __launch_bounds__(FWD_THREADS) void cnn_out_grad(MarchArgs q) {
+    extern __shared__ uint4 lds_u4[];
+    const ConvArgs &a = q.c;
+    char *stage = reinterpret_cast<char *>(lds_u4);
+    uint16_t *ring = reinterpret_cast<uint16_t *>(stage + 8 * FWD_STAGE);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    char *stg = stage + wave * FWD_STAGE;
+    const int m = lane & 31, kh = lane >> 5;
+    const int cols = q.nby * q.nbz * q.nseg, per = gridDim.x / 8;
+    const int col = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (col >= cols) return;
+    const int bz = col % q.nbz, by = col / q.nbz % q.nby, x0 = col / (q.nbz * q.nby) * q.seg;
+    const int x1 = min(x0 + q.seg, a.n0), y0 = by * MR_Y, z0 = bz * 32;
+    const long long pvox = (long long)a.n1 * a.n2;
+    // weights: row ci = m, K = tap
+    bf16x8 wf[2];
+    int toff[2][8], tdx[2][8];             // this lane half's taps: offset in a plane, plane
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        uint32_t w2[4];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int t = c * 16 + kh * 8 + j, tt = min(t, 26);
+            const uint32_t v = t < 27 ? a.w[(size_t)(26 - tt) * 32 * 32 + m] : 0u;
+            w2[j >> 1] = j & 1 ? w2[j >> 1] | v << 16 : v;
+            tdx[c][j] = tt / 9 - 1;
+            toff[c][j] = (wave + tt / 3 % 3) * OG_ROW + m + tt % 3;
+        }
+        wf[c] = frag4(w2[0], w2[1], w2[2], w2[3]);
+    }
+    // one halo voxel of a plane per thread
+    const int hy = tid / HZ, hz = tid % HZ, gy = y0 + hy - 1, gz = z0 + hz - 1;
+    const bool mine = tid < (MR_Y + 2) * HZ, in = mine && gy >= 0 && gy < a.n1 && gz >= 0 && gz < a.n2;
+    const long long goff = in ? (long long)gy * a.n2 + gz : 0;
+    auto fetch = [&](int p) { return a.x[(p >= 0 && p < a.n0 ? p : 0) * pvox + goff]; };
+    auto put = [&](int p, uint16_t v) {
+        if (mine) ring[(p & 3) * OG_PLANE + hy * OG_ROW + hz] = in && p >= 0 && p < a.n0 ? v : (uint16_t)0;
+    };
+    for (int p = x0 - 1; p <= x0 + 1; ++p) put(p, fetch(p));
+    lds_barrier();
+    const int oy = y0 + wave;
+    const bool live = oy < a.n1;           // wave-uniform
+    const long long row0 = (long long)min(oy, a.n1 - 1) * a.n2 + z0;
+    u32x4 *yb = reinterpret_cast<u32x4 *>(a.y) + row0 * 4;
+    float bs[16] = {};
+    for (int p = x0; p < x1; ++p) {
+        if (p > x0) lds_barrier();         // plane p + 1 written; slot (p + 2) & 3 read by every wave
+        const uint16_t next = fetch(p + 2);
+        const long long vox = p * pvox + row0 + m;
+        uint32_t mk = a.mask[vox];
+        f32x16 acc = {};
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            uint32_t f[4];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t v = ring[((p + tdx[c][j]) & 3) * OG_PLANE + toff[c][j]];
+                f[j >> 1] = j & 1 ? f[j >> 1] | v << 16 : v;
+            }
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[c], frag4(f[0], f[1], f[2], f[3]), acc, 0, 0, 0);
+        }
+        put(p + 2, next);
+        mk = live ? mk >> (4 * kh) : 0u;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            f32x4 d;
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                d[j] = acc[4 * g + j];
+                v[j] = (mk >> (8 * g + j)) & 1u ? d[j] : 0.0f;
+                bs[4 * g + j] += v[j];
+            }
+            if (live) reinterpret_cast<f32x4 *>(q.dh_out)[vox * 8 + 2 * g + kh] = d;
+            *reinterpret_cast<uint2 *>(stg + m * 64 + ((g ^ ((m >> 2) & 3)) << 4) + kh * 8) =
+                make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+        }
+        if (live) {
+            u32x4 *dst = yb + p * pvox * 4;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int v = h * 16 + (lane >> 2);
+                dst[h * 64 + lane] = *reinterpret_cast<const u32x4 *>(stg + v * 64 + (((lane & 3) ^ ((v >> 2) & 3)) << 4));
+            }
+        }
+    }
+    float *red = reinterpret_cast<float *>(lds_u4);
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        float v = bs[i];
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o);
+        if (m == 0) red[wave * 32 + 8 * (i >> 2) + 4 * kh + (i & 3)] = v;
+    }
+    lds_barrier();
+    if (tid < 32) {
+        float v = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) v += red[w * 32 + tid];
+        q.part[(size_t)col * 32 + tid] = v;
+    }
+}
+
+// ---------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void cnn_flip(const uint16_t *w, uint16_t *wt) {
     const int i = blockIdx.x * 256 + threadIdx.x;     // over 27*32*32
     if (i >= 27 * 32 * 32) return;
@@ -1064,24 +1277,48 @@ __global__ __launch_bounds__(256) void cnn_relu_grad(const float *__restrict__ d
     }
 }
 
+// ROWS: dr as channel 0 of 32 (the layout of pvd_cnn_wgrad and pvd_cnn_layer_grad); else
+// [n].  Four voxels' loads in flight a thread: 128^3 with rows 56 us (64 bytes stored a
+// voxel), without 14.
+template <bool ROWS>
 __global__ __launch_bounds__(256) void cnn_loss(const float *__restrict__ r, const float *__restrict__ dp,
                                                 const float *__restrict__ dt, const float *__restrict__ mk,
                                                 long long n, float inv_count, uint16_t *__restrict__ dr,
                                                 float *__restrict__ part) {
     __shared__ float red[3][256];
     float se = 0.0f, sw = 0.0f, sg = 0.0f;
-    for (long long v = blockIdx.x * 256LL + threadIdx.x; v < n; v += (long long)gridDim.x * 256) {
-        const float w = mk[v];
-        const float e = dp[v] * r[v] - (dt[v] - dp[v]);
-        se += w * e * e;
-        sw += w;
-        const uint16_t g = f2bf(2.0f * w * e * dp[v] * inv_count);
-        sg += bf2f(g);
-        uint4 *row = reinterpret_cast<uint4 *>(dr + v * 32);
-        row[0] = make_uint4((uint32_t)g, 0u, 0u, 0u);
-        row[1] = make_uint4(0u, 0u, 0u, 0u);
-        row[2] = make_uint4(0u, 0u, 0u, 0u);
-        row[3] = make_uint4(0u, 0u, 0u, 0u);
+    const long long step = (long long)gridDim.x * 256;
+    constexpr int U = 4;
+    for (long long v0 = blockIdx.x * 256LL + threadIdx.x; v0 < n; v0 += U * step) {
+        float xw[U], xp[U], xr[U], xt[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long long v = v0 + u * step < n ? v0 + u * step : v0;
+            xw[u] = mk[v];
+            xp[u] = dp[v];
+            xr[u] = r[v];
+            xt[u] = dt[v];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long long v = v0 + u * step;
+            if (v >= n) break;
+            const float w = xw[u];
+            const float e = xp[u] * xr[u] - (xt[u] - xp[u]);
+            se += w * e * e;
+            sw += w;
+            const uint16_t g = f2bf(2.0f * w * e * xp[u] * inv_count);
+            sg += bf2f(g);
+            if (ROWS) {
+                uint4 *row = reinterpret_cast<uint4 *>(dr + v * 32);
+                row[0] = make_uint4((uint32_t)g, 0u, 0u, 0u);
+                row[1] = make_uint4(0u, 0u, 0u, 0u);
+                row[2] = make_uint4(0u, 0u, 0u, 0u);
+                row[3] = make_uint4(0u, 0u, 0u, 0u);
+            } else {
+                dr[v] = g;
+            }
+        }
     }
     red[0][threadIdx.x] = se;
     red[1][threadIdx.x] = sw;
@@ -1119,7 +1356,8 @@ __global__ __launch_bounds__(256) void cnn_adam(float *p, const float *g, float 
 // the 256 x 27648 weight partials 61 us; both now take 4-6 us.)
 constexpr int RED_COLS = 32, RED_GROUPS = 32;
 __global__ __launch_bounds__(RED_COLS * RED_GROUPS) void reduce_rows(const float *__restrict__ part, int rows, int cols,
-                                                                     float *__restrict__ out, int accumulate) {
+                                                                     float *__restrict__ out, int accumulate,
+                                                                     int pitch) {
     __shared__ float red[RED_GROUPS][RED_COLS + 1];
     const int l = threadIdx.x & (RED_COLS - 1), g = threadIdx.x / RED_COLS;
     const int c = blockIdx.x * RED_COLS + l;
@@ -1139,7 +1377,8 @@ __global__ __launch_bounds__(RED_COLS * RED_GROUPS) void reduce_rows(const float
         if (g < h) red[g][l] += red[g + h][l];
         __syncthreads();
     }
-    if (g == 0 && c < cols) out[c] = accumulate ? out[c] + red[0][l] : red[0][l];
+    float *o = out + (size_t)blockIdx.x * pitch + l;         // `pitch` floats per 32 columns
+    if (g == 0 && c < cols) *o = accumulate ? *o + red[0][l] : red[0][l];
 }
 
 __global__ __launch_bounds__(256) void cnn_pack(const float *__restrict__ a, const float *__restrict__ d,
@@ -1328,6 +1567,14 @@ void march_plan(MarchArgs *q, int n0, int n1, int n2) {
             q->nseg = nseg;
         }
     }
+}
+
+// cnn_out_grad: segments half as long, for two workgroups a CU (a segment's halo is two planes
+// of one-channel dr)
+void out_grad_plan(MarchArgs *q, int n0, int n1, int n2) {
+    march_plan(q, n0, n1, n2);
+    q->seg = (q->seg + 1) / 2;
+    q->nseg = (n0 + q->seg - 1) / q->seg;
 }
 
 template <int MODE>
@@ -1590,7 +1837,7 @@ int pvd_cnn_wgrad(const void *x, int cin, const void *dz, float *dw, float *work
     if (e != hipSuccess) return pvd_hip_error(e, "launch weight gradient");
     const int cols = 27 * 32 * cin;
     hipLaunchKernelGGL(reduce_rows, dim3((cols + RED_COLS - 1) / RED_COLS), dim3(RED_COLS * RED_GROUPS), 0, st,
-                       (const float *)work, blocks, cols, dw, 0);
+                       (const float *)work, blocks, cols, dw, 0, RED_COLS);
     e = hipGetLastError();
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch reduction");
 }
@@ -1598,10 +1845,72 @@ int pvd_cnn_wgrad(const void *x, int cin, const void *dz, float *dw, float *work
 int pvd_cnn_loss(const float *r, const float *dp, const float *dt, const float *m, long long n, float inv_count,
                  void *dr, float *loss_part, void *stream) {
     if (!r || !dp || !dt || !m || !dr || !loss_part || n < 1) return pvd_set_error(PVD_EINVAL, "bad argument");
-    hipLaunchKernelGGL(cnn_loss, dim3(PVD_CNN_LOSS_BLOCKS), dim3(256), 0, (hipStream_t)stream, r, dp, dt, m, n, inv_count,
+    hipLaunchKernelGGL(cnn_loss<true>, dim3(PVD_CNN_LOSS_BLOCKS), dim3(256), 0, (hipStream_t)stream, r, dp, dt, m, n, inv_count,
                        (uint16_t *)dr, loss_part);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch loss");
+}
+
+int pvd_cnn_out_loss(const float *r, const float *dp, const float *dt, const float *m, long long n, float inv_count,
+                     void *dr, float *loss_part, void *stream) {
+    if (!r || !dp || !dt || !m || !dr || !loss_part || n < 1) return pvd_set_error(PVD_EINVAL, "bad argument");
+    hipLaunchKernelGGL(cnn_loss<false>, dim3(PVD_CNN_LOSS_BLOCKS), dim3(256), 0, (hipStream_t)stream, r, dp, dt, m, n,
+                       inv_count, (uint16_t *)dr, loss_part);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch loss");
+}
+
+int pvd_cnn_out_wgrad(const void *x, const void *dr, float *dw, float *work, int n0, int n1, int n2, void *stream) {
+    if (int rc = check_grid(n0, n1, n2)) return rc;
+    if (!x || !dr || !dw || !work) return pvd_set_error(PVD_EINVAL, "null argument");
+    if (reinterpret_cast<uintptr_t>(x) & 15) return pvd_set_error(PVD_EINVAL, "x must be 16-byte aligned");
+    static bool attr = false;
+    if (!attr) {
+        const hipError_t e = hipFuncSetAttribute((const void *)cnn_out_wgrad,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)OW_LDS);
+        if (e != hipSuccess) return pvd_hip_error(e, "set LDS limit");
+        attr = true;
+    }
+    const long long total = (long long)n0 * ((n1 + OW_Y - 1) / OW_Y) * (n2 >> 5);
+    if (total > 0x7fffffffLL) return pvd_set_error(PVD_ENOTSUP, "grid too large");
+    // (32 partial sums of this layer fit where pvd_cnn_wgrad_work_floats has one workgroup's)
+    const long long most = std::min<long long>((long long)OW_BLOCKS_PER_CU * num_cus(), 32LL * wgrad_blocks(n0, n1, n2));
+    const int blocks = (int)std::min(total, most);
+    hipStream_t st = (hipStream_t)stream;
+    const WgradArgs a{(const uint16_t *)x, (const uint16_t *)dr, work, n0, n1, n2};
+    hipLaunchKernelGGL(cnn_out_wgrad, dim3(blocks), dim3(WG_THREADS), OW_LDS, st, a);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return pvd_hip_error(e, "launch output weight gradient");
+    hipLaunchKernelGGL(reduce_rows, dim3(27), dim3(RED_COLS * RED_GROUPS), 0, st, (const float *)work, blocks, 27 * 32, dw,
+                       0, 32 * 32);
+    e = hipGetLastError();
+    return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch reduction");
+}
+
+size_t pvd_cnn_out_grad_parts(int n0, int n1, int n2) {
+    if (n0 < 1 || n1 < 1 || n2 < 32) return 0;
+    MarchArgs q{};
+    out_grad_plan(&q, n0, n1, n2);
+    return (size_t)q.nby * q.nbz * q.nseg;
+}
+
+int pvd_cnn_out_grad(const void *dr, const void *w, float *dh_out, const unsigned *mask, void *dz_out, float *dbias_part,
+                     int n0, int n1, int n2, void *stream) {
+    if (int rc = check_grid(n0, n1, n2)) return rc;
+    if (!dr || !w || !dh_out || !mask || !dz_out || !dbias_part) return pvd_set_error(PVD_EINVAL, "null argument");
+    if ((reinterpret_cast<uintptr_t>(dz_out) | reinterpret_cast<uintptr_t>(dh_out)) & 15)
+        return pvd_set_error(PVD_EINVAL, "dz_out and dh_out must be 16-byte aligned");
+    MarchArgs q{};
+    q.c = ConvArgs{(const uint16_t *)dr, (const uint16_t *)w, nullptr, nullptr, (uint16_t *)dz_out, nullptr, nullptr, n0,
+                   n1, n2, nullptr, nullptr, const_cast<unsigned *>(mask)};
+    q.dh_out = dh_out;
+    q.part = dbias_part;
+    out_grad_plan(&q, n0, n1, n2);
+    const long long grid = ((long long)q.nby * q.nbz * q.nseg + 7) / 8 * 8;
+    if (grid > 0x7fffffffLL) return pvd_set_error(PVD_ENOTSUP, "grid too large");
+    hipLaunchKernelGGL(cnn_out_grad, dim3((unsigned)grid), dim3(FWD_THREADS), OG_LDS, (hipStream_t)stream, q);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch output layer gradient");
 }
 
 int pvd_cnn_adam(float *param, const float *grad, float *m, float *v, void *param_bf16, long long n, float lr,
@@ -1696,7 +2005,7 @@ size_t pvd_cnn_region_block_count(int n0, int n1, int n2) {
 int pvd_reduce_rows(const float *part, int rows, int cols, float *out, int accumulate, void *stream) {
     if (!part || !out || rows < 1 || cols < 1) return pvd_set_error(PVD_EINVAL, "bad argument");
     hipLaunchKernelGGL(reduce_rows, dim3((cols + RED_COLS - 1) / RED_COLS), dim3(RED_COLS * RED_GROUPS), 0,
-                       (hipStream_t)stream, part, rows, cols, out, accumulate);
+                       (hipStream_t)stream, part, rows, cols, out, accumulate, RED_COLS);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch reduction");
 }

@@ -126,10 +126,12 @@ class ResidualCNN:
                 "mask": [torch.zeros(n, dtype=torch.int32, device=self.device) for _ in range(5)],
                 "r": torch.zeros(n, dtype=torch.float32, device=self.device),
                 "dz": [torch.empty((n, 32), **bf) for _ in range(2)],
-                "dr": torch.empty((n, 32), **bf),
+                "dr": torch.empty(n, **bf),
                 "dh": torch.empty((n, 32), dtype=torch.float32, device=self.device),
                 "dbias_part": torch.empty((int(self.lib.pvd_cnn_grad_parts(*shape)), 32), dtype=torch.float32,
                                           device=self.device),
+                "dbias_out": torch.empty((int(self.lib.pvd_cnn_out_grad_parts(*shape)), 32), dtype=torch.float32,
+                                         device=self.device),
                 "wwork": torch.empty(int(self.lib.pvd_cnn_wgrad_work_floats(*shape)), dtype=torch.float32,
                                      device=self.device),
                 "loss_part": torch.empty((256, 3), dtype=torch.float32, device=self.device),
@@ -189,8 +191,8 @@ class ResidualCNN:
         cnt = float(mask.sum().item())
         if cnt <= 0:
             raise ValueError("empty loss mask")
-        nat.check(self.lib.pvd_cnn_loss(_p(ws["r"]), _p(dp), _p(dt), _p(mask), n, ctypes.c_float(1.0 / cnt),
-                                        _p(ws["dr"]), _p(ws["loss_part"]), self._stream()), "pvd_cnn_loss")
+        nat.check(self.lib.pvd_cnn_out_loss(_p(ws["r"]), _p(dp), _p(dt), _p(mask), n, ctypes.c_float(1.0 / cnt),
+                                            _p(ws["dr"]), _p(ws["loss_part"]), self._stream()), "pvd_cnn_out_loss")
         nat.check(self.lib.pvd_reduce_rows(_p(ws["loss_part"]), 256, 3, _p(ws["loss_sum"]), 0, self._stream()),
                   "pvd_reduce_rows")
         return ws["loss_sum"]        # [sum m e^2, sum m, sum dr]; loss = [0] / [1]
@@ -198,23 +200,28 @@ class ResidualCNN:
     def backward(self, x, shape):
         """Gradients of every parameter into self.grad (after forward + loss_and_grad)."""
         ws = self._workspace(shape)
-        h, dh, parts = ws["h"], ws["dh"], ws["dbias_part"]
+        h, dh = ws["h"], ws["dh"]
         st = self._stream()
         # layer 5
-        nat.check(self.lib.pvd_cnn_wgrad(_p(h[4]), 32, _p(ws["dr"]), _p(self.grad_w(5)), _p(ws["wwork"]),
-                                         shape[0], shape[1], shape[2], st), "pvd_cnn_wgrad")
+        nat.check(self.lib.pvd_cnn_out_wgrad(_p(h[4]), _p(ws["dr"]), _p(self.grad_w(5)), _p(ws["wwork"]),
+                                             shape[0], shape[1], shape[2], st), "pvd_cnn_out_wgrad")
         gb5 = self.grad_b(5)
         gb5.zero_()
         gb5[0:1].copy_(ws["loss_sum"][2:3])
-        dz = ws["dr"]
+        dz = None
         for l in range(4, -1, -1):
             # through layer l + 1 to dL/dh_l (kept for the skip connection) and, past the
             # ReLU of layer l, dz_l and its bias gradient
-            nat.check(self.lib.pvd_cnn_flip_weights(_p(self.w_bf16(l + 1)), _p(self._flip), st), "pvd_cnn_flip_weights")
-            out = ws["dz"][l & 1]
-            nat.check(self.lib.pvd_cnn_layer_grad(_p(dz), _p(self._flip), _p(dh if l < 4 else None),
-                                                  _p(dh if l > 0 else None), _p(ws["mask"][l]), _p(out), _p(parts),
-                                                  shape[0], shape[1], shape[2], st), "pvd_cnn_layer_grad")
+            out, parts = ws["dz"][l & 1], ws["dbias_out" if l == 4 else "dbias_part"]
+            if l == 4:
+                nat.check(self.lib.pvd_cnn_out_grad(_p(ws["dr"]), _p(self.w_bf16(5)), _p(dh), _p(ws["mask"][4]), _p(out),
+                                                    _p(parts), shape[0], shape[1], shape[2], st), "pvd_cnn_out_grad")
+            else:
+                nat.check(self.lib.pvd_cnn_flip_weights(_p(self.w_bf16(l + 1)), _p(self._flip), st),
+                          "pvd_cnn_flip_weights")
+                nat.check(self.lib.pvd_cnn_layer_grad(_p(dz), _p(self._flip), _p(dh), _p(dh if l > 0 else None),
+                                                      _p(ws["mask"][l]), _p(out), _p(parts), shape[0], shape[1],
+                                                      shape[2], st), "pvd_cnn_layer_grad")
             dz = out
             nat.check(self.lib.pvd_reduce_rows(_p(parts), parts.shape[0], 32, _p(self.grad_b(l)), 0, st),
                       "pvd_reduce_rows")

@@ -785,6 +785,59 @@ def test_training_layers_and_layer_gradient(shape):
                                    atol=1e-4 * np.abs(exp).max() * n ** 0.5 + 1e-6 * (np.abs(exp) * mb).sum((0, 1, 2)).max())
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 32), (2, 8, 32), (5, 9, 64), (9, 17, 96), (33, 20, 64)])
+def test_output_layer_gradients_of_one_channel(shape):
+    """Loss gradient, weight gradient and input gradient of the output layer with dr as one
+    channel, at the edges of their 8-row columns, against the 32-channel entry points with dr
+    in channel 0 and the FP64 oracle (FP32 sums, tolerances of the tests above)."""
+    import ctypes
+    import torch
+
+    from pyvoxeldosimetry_amd import _native as nat
+    _say("output layer gradients", shape)
+    lib = nat.load()
+    n = int(np.prod(shape))
+    rng = np.random.default_rng(n)
+    p = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)  # noqa: E731
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    r, dp, dt = (torch.from_numpy(rng.normal(size=n).astype(np.float32)).cuda() for _ in range(3))
+    mk = torch.from_numpy((rng.random(n) < 0.7).astype(np.float32)).cuda()
+    inv = ctypes.c_float(1.0 / 16)
+    dr32 = torch.full((n, 32), float("nan"), dtype=torch.bfloat16, device="cuda")
+    dr = torch.full((n,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    l32, l1 = (torch.empty((256, 3), device="cuda") for _ in range(2))
+    nat.check(lib.pvd_cnn_loss(p(r), p(dp), p(dt), p(mk), n, inv, p(dr32), p(l32), st), "loss")
+    nat.check(lib.pvd_cnn_out_loss(p(r), p(dp), p(dt), p(mk), n, inv, p(dr), p(l1), st), "out loss")
+    assert torch.equal(dr, dr32[:, 0]) and torch.equal(l1, l32) and not dr32[:, 1:].any()
+    e = dp.double() * r.double() - (dt.double() - dp.double())
+    np.testing.assert_allclose(dr.double().cpu(), (2.0 / 16 * mk.double() * e * dp.double()).cpu(), rtol=8e-3, atol=1e-6)
+    x = ocnn.bf16_round(rng.normal(size=shape + (32,)).astype(np.float32))
+    w = ocnn.bf16_round(rng.normal(scale=0.1, size=(27, 32, 32)).astype(np.float32))
+    xt, wt = bf(x), bf(w)
+    work = torch.full((int(lib.pvd_cnn_wgrad_work_floats(*shape)),), float("nan"), device="cuda")
+    dw = torch.full((27, 32, 32), 7.0, device="cuda")
+    nat.check(lib.pvd_cnn_out_wgrad(p(xt), p(dr), p(dw), p(work), *shape, st), "out wgrad")
+    assert (dw[:, 1:] == 7.0).all()                                    # other outputs' rows are left alone
+    dz = dr32.float().cpu().numpy().reshape(shape + (32,))
+    exp = ocnn.conv3_weight_grad(x, dz)[:, 0]
+    np.testing.assert_allclose(dw[:, 0].cpu().numpy(), exp, rtol=0, atol=2e-5 * n ** 0.5 * np.abs(dz).max())
+    # input gradient with the ReLU mask of the layer below
+    bits = rng.integers(0, 2 ** 32, size=n, dtype=np.uint32)
+    mask = torch.from_numpy(bits.view(np.int32)).cuda()
+    mb = ((bits[:, None] >> np.arange(32, dtype=np.uint32)) & 1).reshape(shape + (32,))
+    rows = int(lib.pvd_cnn_out_grad_parts(*shape))
+    dh = torch.full((n, 32), float("nan"), device="cuda")
+    dzo = torch.full((n, 32), float("nan"), dtype=torch.bfloat16, device="cuda")
+    part = torch.full((rows, 32), float("nan"), device="cuda")
+    nat.check(lib.pvd_cnn_out_grad(p(dr), p(wt), p(dh), p(mask), p(dzo), p(part), *shape, st), "out grad")
+    exp = ocnn.conv3_input_grad(dz, w)
+    top = np.abs(exp).max()
+    np.testing.assert_allclose(dh.cpu().numpy().reshape(shape + (32,)), exp, rtol=0, atol=1e-4 * top)
+    np.testing.assert_allclose(dzo.float().cpu().numpy().reshape(shape + (32,)), exp * mb, rtol=8e-3, atol=2e-4 * top)
+    np.testing.assert_allclose(part.double().sum(0).cpu().numpy(), (exp * mb).sum((0, 1, 2)), rtol=0,
+                               atol=1e-4 * top * n ** 0.5 + 1e-6 * (np.abs(exp) * mb).sum((0, 1, 2)).max())
+
+
 @pytest.mark.parametrize("shape,histories,every", [((1, 1, 1), 1, 1), ((3, 5, 7), 63, 16), ((21, 22, 21), 3, 2),
                                                    ((22, 21, 22), 3, 2), ((40, 9, 31), 17, 5)])
 def test_monte_carlo_maps_histories_alike(shape, histories, every):

@@ -1,7 +1,7 @@
 // Grid-to-grid resampling (nearest / trilinear / cubic B-spline) for the activity
 // <-> kernel resolution round trip of the dose path.  Linear and cubic interpolation
 // are separable: a workgroup interpolates the input along x once into LDS and writes a
-// tile of output rows from it (resample_staged); nearest, and outputs much coarser than
+// tile of output rows from it (resample_linear, resample_cubic); nearest, and outputs much coarser than
 // the input, gather each output's neighbours (resample_kernel).  Coordinates are formed
 // in FP64 so that equal spacings map every output voxel exactly onto an input voxel.
 // The cubic B-spline coefficients come from a separable mirror-boundary prefilter
@@ -153,23 +153,139 @@ __global__ __launch_bounds__(256) void resample_kernel(ResampleArgs a) {
 // The gather form above issues 8 (linear) or 64 (cubic) loads per output and is bound
 // by them; here a tile costs W loads per input element it spans, so the cost follows
 // the input samples per output and the pass goes to the HBM stores.  Gather -> staged:
-// 251x251x196 -> 512x512x400 linear 321 -> 155 us (94 at the copy rate), cubic 2139 ->
+// 251x251x196 -> 512x512x400 linear 321 -> 126 us (94 at the copy rate), cubic 2139 ->
 // 209; 301x301x233 -> 206x206x160 linear 51 -> 25 us, cubic 283 -> 41 (22).
 constexpr int kRsBlock = 256;      // threads
-constexpr int kRsSpan = 256;       // input columns of a tile (at most)
+constexpr int kRsU = 5;            // linear: columns per lane in flight in step 1
+constexpr int kRsSpan = 64 * kRsU; // input columns of a tile (at most)
+constexpr int kRsK = 8;            // linear: outputs along z per lane
+constexpr int kRsCubicU = 4, kRsCubicSpan = 256;   // cubic: the same two
 constexpr int kRsRows = 8;         // output rows of a tile (at most)
-constexpr int kRsU = 4;            // columns per lane in flight in step 1
+constexpr int kRsPlanes = 4;       // linear: output planes of a workgroup (at most)
 
 struct StagedArgs {
     ResampleArgs a;
     int tj, kt;                    // output rows and columns of a tile
+    int ti;                        // output planes of a workgroup
     int njt, nkc;                  // tiles along y and z
     int span, rows;                // LDS extents: input columns, input rows
     long long tiles;
 };
 
-template <int W>
-__global__ __launch_bounds__(kRsBlock) void resample_staged(StagedArgs q) {
+// Linear: an output takes the bilinear product of y and z from 2 x 2 values of S.  The
+// wave issue rate bound the tile-per-output-plane form (an FP64 coordinate, a row lookup and
+// a branch per output): a workgroup now keeps a lane's z positions over kRsPlanes output
+// planes and gives each wave whole rows, about 12 instructions an output.
+// 251x251x196 -> 512x512x400 150 -> 126 us (94 at the copy rate), 400x300x350 -> half 32.6
+// -> 29.7; eight planes a workgroup with 64 VGPRs 170.
+__global__ __launch_bounds__(kRsBlock) void resample_linear(StagedArgs q) {
+    extern __shared__ float rs_lds[];
+    __shared__ float s_wy[kRsRows];
+    __shared__ int s_ry[kRsRows][2];     // input rows of an output row (relative to ylo); < 0: outside
+    const ResampleArgs &a = q.a;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    constexpr int NW = kRsBlock / 64;
+    // XCD-contiguous bands of tiles (neighbouring tiles share input rows in one L2)
+    const long long G = gridDim.x;
+    const long long t = (long long)(blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
+    if (t >= q.tiles) return;
+    const int kc = (int)(t % q.nkc);
+    const long long ij = t / q.nkc;
+    const int jt = (int)(ij % q.njt), i0 = (int)(ij / q.njt) * q.ti, i1 = min(i0 + q.ti, a.m[0]);
+    const int j0 = jt * q.tj, nj = min(q.tj, a.m[1] - j0);
+    const int k0 = kc * q.kt, nk = min(q.kt, a.m[2] - k0);
+    // first and last input row the tile can touch, 0-filled tiles aside
+    const double cy1 = (j0 + nj - 1) * a.ratio[1];
+    const int ylo = min(max((int)floor(fmin(j0 * a.ratio[1], 2.0e9)), 0), a.n[1] - 1);
+    const int yb1 = (int)fmin(floor(cy1), (double)(a.n[1] - 1));
+    const int yhi = min(yb1 + 1, a.n[1] - 1);
+    const int ny = min(yhi - ylo + 1, q.rows);
+    const bool in_y = j0 * a.ratio[1] < a.n[1] - 0.5;
+    if (tid < nj) {
+        int b = 0;
+        float f = 0.0f;
+        const bool in = axis_pos((j0 + tid) * a.ratio[1], a.n[1], b, f);
+        s_ry[tid][0] = in ? max(b, 0) - ylo : -1;
+        s_ry[tid][1] = min(b + 1, a.n[1] - 1) - ylo;
+        s_wy[tid] = f;
+    }
+    // LDS column c is the input column zlo + c, clamped, so an output reads two consecutive
+    // columns.
+    const int zlo = (int)floor(fmin(k0 * a.ratio[2], 2.0e9));
+    int zc[kRsU];
+#pragma unroll
+    for (int c = 0; c < kRsU; ++c) {
+        zc[c] = min(zlo + lane + 64 * c, a.n[2] - 1);
+    }
+    // this lane's outputs k0 + lane + 64 u: first column (< 0: outside), fraction
+    int ko[kRsK];
+    float kf[kRsK];
+#pragma unroll
+    for (int u = 0; u < kRsK; ++u) {
+        int b = 0;
+        float f = 0.0f;
+        const bool in = axis_pos((k0 + lane + 64 * u) * a.ratio[2], a.n[2], b, f);
+        ko[u] = in ? min(b - zlo, q.span - 2) : -1;
+        kf[u] = f;
+    }
+    float *S = rs_lds;
+    for (int i = i0; i < i1; ++i) {
+        int bx;
+        float fx;
+        const bool in_xy = axis_pos(i * a.ratio[0], a.n[0], bx, fx) && in_y;       // uniform
+        if (in_xy) {
+            // 1. x: the planes and weights are uniform over the workgroup
+            const float *plane[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                plane[u] = a.in + ((long long)min(max(bx + u, 0), a.n[0] - 1) * a.n[1] + ylo) * a.n[2];
+            for (int y = wave; y < ny; y += NW) {
+                const long long r0 = (long long)y * a.n[2];
+                float v[kRsU][2];
+#pragma unroll
+                for (int c = 0; c < kRsU; ++c) {
+                    if (64 * c >= q.span) break;
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) v[c][u] = plane[u][r0 + zc[c]];
+                }
+#pragma unroll
+                for (int c = 0; c < kRsU; ++c) {
+                    if (64 * c >= q.span) break;
+                    if (lane + 64 * c < q.span) S[y * q.span + lane + 64 * c] = fmaf(fx, v[c][1] - v[c][0], v[c][0]);
+                }
+            }
+        }
+        lds_barrier();
+        // 2. y and z, and the stores: a row per wave
+        for (int jj = wave; jj < nj; jj += NW) {
+            float *o = a.out + ((long long)i * a.m[1] + j0 + jj) * a.m[2] + k0 + lane;
+            const int r0 = in_xy ? s_ry[jj][0] : -1;                   // uniform
+            if (r0 < 0) {
+                for (int u = 0; u < kRsK; ++u)
+                    if (lane + 64 * u < nk) o[64 * u] = 0.0f;
+                continue;
+            }
+            const float *p = S + r0 * q.span, *p1 = S + s_ry[jj][1] * q.span;
+            const float fy = s_wy[jj];
+#pragma unroll
+            for (int u = 0; u < kRsK; ++u) {
+                if (lane + 64 * u >= nk) break;
+                const int c = max(ko[u], 0);
+                const float e0 = fmaf(fy, p1[c] - p[c], p[c]);
+                const float e1 = fmaf(fy, p1[c + 1] - p[c + 1], p[c + 1]);
+                const float x = fmaf(kf[u], e1 - e0, e0);
+                o[64 * u] = a.scale * (ko[u] < 0 ? 0.0f : x);
+            }
+        }
+        lds_barrier();       // S is read
+    }
+}
+
+// Cubic: T[j][z] = S interpolated along y, then 4 values of T an output; an output plane per
+// workgroup.  (The linear kernel's form held 135 VGPRs here and took 120x250x250 @3.3 ->
+// 1.5 mm from 181 to 255 us.)
+__global__ __launch_bounds__(kRsBlock) void resample_cubic(StagedArgs q) {
+    constexpr int W = 4, B = 3;          // neighbours, and the furthest of them past the base index
     extern __shared__ float rs_lds[];
     __shared__ float s_wy[kRsRows][4];
     __shared__ int s_ry[kRsRows][4];     // input rows of an output row (relative to ylo); < 0: outside
@@ -190,11 +306,10 @@ __global__ __launch_bounds__(kRsBlock) void resample_staged(StagedArgs q) {
     // first and last input row and column the tile can touch (mirrored and clamped
     // neighbours lie within 3 of the base index), 0-filled tiles aside
     const double cy1 = (j0 + nj - 1) * a.ratio[1], cz1 = (k0 + nk - 1) * a.ratio[2];
-    constexpr int B = W == 4 ? 3 : 1;
-    const int ylo = min(max((int)floor(fmin(j0 * a.ratio[1], 2.0e9)) - (B - 1), 0), a.n[1] - 1);
+    const int ylo = min(max((int)floor(fmin(j0 * a.ratio[1], 2.0e9)) - 2, 0), a.n[1] - 1);
     const int yb1 = (int)fmin(floor(cy1), (double)(a.n[1] - 1));
     const int yhi = min(yb1 + B, a.n[1] - 1);
-    const int zlo = min(max((int)floor(fmin(k0 * a.ratio[2], 2.0e9)) - (B - 1), 0), a.n[2] - 1);
+    const int zlo = min(max((int)floor(fmin(k0 * a.ratio[2], 2.0e9)) - 2, 0), a.n[2] - 1);
     const int zhi = min((int)fmin(floor(cz1), (double)(a.n[2] - 1)) + B, a.n[2] - 1);
     const int ny = min(yhi - ylo + 1, q.rows), nz = min(zhi - zlo + 1, q.span);
     if (!axis_pos(i * a.ratio[0], a.n[0], bx, fx) || !(j0 * a.ratio[1] < a.n[1] - 0.5)) {
@@ -206,11 +321,11 @@ __global__ __launch_bounds__(kRsBlock) void resample_staged(StagedArgs q) {
         int b = 0;
         float f = 0.0f;
         const bool in = axis_pos((j0 + tid) * a.ratio[1], a.n[1], b, f);
-        float w[4] = {f, 0.0f, 0.0f, 0.0f};
-        if (W == 4) bspline3_weights(f, w);
+        float w[4];
+        bspline3_weights(f, w);
 #pragma unroll
         for (int v = 0; v < W; ++v) {
-            const int y = W == 4 ? mirror_index(b - 1 + v, a.n[1]) : min(max(b + v, 0), a.n[1] - 1);
+            const int y = mirror_index(b - 1 + v, a.n[1]);
             s_ry[tid][v] = in ? y - ylo : -1;
             s_wy[tid][v] = w[v];
         }
@@ -218,43 +333,40 @@ __global__ __launch_bounds__(kRsBlock) void resample_staged(StagedArgs q) {
     // 1. x: the planes and weights are uniform over the workgroup
     const float *plane[W];
     float wx[4];
-    if (W == 4) bspline3_weights(fx, wx);
+    bspline3_weights(fx, wx);
 #pragma unroll
     for (int u = 0; u < W; ++u) {
-        const int x = W == 4 ? mirror_index(bx - 1 + u, a.n[0]) : min(max(bx + u, 0), a.n[0] - 1);
+        const int x = mirror_index(bx - 1 + u, a.n[0]);
         plane[u] = a.in + (long long)x * a.n[1] * a.n[2];
     }
     float *S = rs_lds, *T = rs_lds + (size_t)q.rows * q.span;
     for (int y = wave; y < ny; y += kRsBlock / 64) {
         const long long r0 = (long long)(ylo + y) * a.n[2] + zlo;
-        for (int z0 = lane; z0 < nz; z0 += 64 * kRsU) {
-            float v[kRsU][W];
+        for (int z0 = lane; z0 < nz; z0 += 64 * kRsCubicU) {
+            float v[kRsCubicU][W];
 #pragma unroll
-            for (int c = 0; c < kRsU; ++c)
+            for (int c = 0; c < kRsCubicU; ++c)
 #pragma unroll
                 for (int u = 0; u < W; ++u) v[c][u] = plane[u][r0 + min(z0 + 64 * c, nz - 1)];
 #pragma unroll
-            for (int c = 0; c < kRsU; ++c) {
-                float x;
-                if (W == 4) x = fmaf(wx[3], v[c][W - 1], fmaf(wx[2], v[c][W - 2], fmaf(wx[1], v[c][1], wx[0] * v[c][0])));
-                else x = fmaf(fx, v[c][1] - v[c][0], v[c][0]);
-                if (z0 + 64 * c < nz) S[y * q.span + z0 + 64 * c] = x;
+            for (int c = 0; c < kRsCubicU; ++c) {
+                if (z0 + 64 * c < nz)
+                    S[y * q.span + z0 + 64 * c] =
+                        fmaf(wx[3], v[c][3], fmaf(wx[2], v[c][2], fmaf(wx[1], v[c][1], wx[0] * v[c][0])));
             }
         }
     }
     __syncthreads();
-    // 2. y (cubic)
-    if (W == 4) {
-        for (int jj = wave; jj < nj; jj += kRsBlock / 64) {
-            if (s_ry[jj][0] < 0) continue;
-            const float *s0 = S + s_ry[jj][0] * q.span, *s1 = S + s_ry[jj][1] * q.span;
-            const float *s2 = S + s_ry[jj][2] * q.span, *s3 = S + s_ry[jj][3] * q.span;
-            const float w0 = s_wy[jj][0], w1 = s_wy[jj][1], w2 = s_wy[jj][2], w3 = s_wy[jj][3];
-            for (int z = lane; z < nz; z += 64)
-                T[jj * q.span + z] = fmaf(w3, s3[z], fmaf(w2, s2[z], fmaf(w1, s1[z], w0 * s0[z])));
-        }
-        __syncthreads();
+    // 2. y
+    for (int jj = wave; jj < nj; jj += kRsBlock / 64) {
+        if (s_ry[jj][0] < 0) continue;
+        const float *s0 = S + s_ry[jj][0] * q.span, *s1 = S + s_ry[jj][1] * q.span;
+        const float *s2 = S + s_ry[jj][2] * q.span, *s3 = S + s_ry[jj][3] * q.span;
+        const float w0 = s_wy[jj][0], w1 = s_wy[jj][1], w2 = s_wy[jj][2], w3 = s_wy[jj][3];
+        for (int z = lane; z < nz; z += 64)
+            T[jj * q.span + z] = fmaf(w3, s3[z], fmaf(w2, s2[z], fmaf(w1, s1[z], w0 * s0[z])));
     }
+    __syncthreads();
     // 3. z, and the stores
     for (int k = tid; k < nk; k += kRsBlock) {
         int b = 0;
@@ -262,38 +374,27 @@ __global__ __launch_bounds__(kRsBlock) void resample_staged(StagedArgs q) {
         const bool inz = axis_pos((k0 + k) * a.ratio[2], a.n[2], b, f);
         float wz[4];
         int z[W];
-        if (W == 4) bspline3_weights(f, wz);
+        bspline3_weights(f, wz);
 #pragma unroll
         for (int v = 0; v < W; ++v) {
-            const int zz = W == 4 ? mirror_index(b - 1 + v, a.n[2]) : min(max(b + v, 0), a.n[2] - 1);
-            z[v] = inz ? zz - zlo : 0;
+            z[v] = inz ? mirror_index(b - 1 + v, a.n[2]) - zlo : 0;
         }
         for (int jj = 0; jj < nj; ++jj) {
-            const int r0 = s_ry[jj][0];
             float x = 0.0f;
-            if (inz && r0 >= 0) {
-                if (W == 4) {
-                    const float *p = T + jj * q.span;
-                    x = fmaf(wz[3], p[z[W - 1]], fmaf(wz[2], p[z[W - 2]], fmaf(wz[1], p[z[1]], wz[0] * p[z[0]])));
-                } else {
-                    const float *p = S + r0 * q.span, *p1 = S + s_ry[jj][1] * q.span;
-                    const float fy = s_wy[jj][0];
-                    const float e0 = fmaf(fy, p1[z[0]] - p[z[0]], p[z[0]]);
-                    const float e1 = fmaf(fy, p1[z[1]] - p[z[1]], p[z[1]]);
-                    x = fmaf(f, e1 - e0, e0);
-                }
+            if (inz && s_ry[jj][0] >= 0) {
+                const float *p = T + jj * q.span;
+                x = fmaf(wz[3], p[z[3]], fmaf(wz[2], p[z[2]], fmaf(wz[1], p[z[1]], wz[0] * p[z[0]])));
             }
             orow[(long long)jj * a.m[2] + k] = a.scale * x;
         }
     }
 }
 
-// Largest extent of input indices that `cnt` consecutive outputs touch on an axis of n
-// samples (any start): the kernel's lo .. hi range.
-int staged_extent(double ratio, int cnt, int n, int W) {
+// Largest extent of input indices, past + 1 beyond the last base index, that `cnt`
+// consecutive outputs span (any start).
+int staged_extent(double ratio, int cnt, int past) {
     // (one more than the real numbers need: the products are rounded)
-    const double e = std::floor((cnt - 1) * ratio) + 3.0 + (W == 4 ? 5 : 1);
-    return e < (double)n ? (int)e : n;
+    return (int)std::min(1.0e9, std::floor((cnt - 1) * ratio)) + 3 + past;
 }
 
 // Coarsest output / input spacing (along y and z) that takes the staged form: beyond it
@@ -302,30 +403,59 @@ int staged_extent(double ratio, int cnt, int n, int W) {
 // 3.0, 99 / 72 at 4.5, 32 / 34 at 8.3.
 constexpr double kStagedLinear = 2.5, kStagedCubic = 8.0;
 
-template <int W>
-hipError_t launch_staged(const ResampleArgs &a, hipStream_t st) {
+template <typename Kernel>
+hipError_t launch_staged(Kernel kernel, const StagedArgs &q, int tj, hipStream_t st) {
+    const size_t lds = sizeof(float) * q.span * (size_t)(q.rows + tj);
+    const long long grid = (q.tiles + 7) / 8 * 8;
+    if (grid > 0x7fffffffLL || q.span > kRsSpan || lds > 48 * 1024) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kRsBlock), lds, st, q);
+    return hipGetLastError();
+}
+
+hipError_t launch_linear(const ResampleArgs &a, hipStream_t st) {
     StagedArgs q{};
     q.a = a;
+    // outputs along z that a row's lanes and a tile's input columns hold, in equal tiles
+    q.kt = std::min(a.m[2], 64 * kRsK);
+    if (staged_extent(a.ratio[2], q.kt, 1) > kRsSpan)
+        q.kt = std::max(1, std::min(q.kt, (int)((kRsSpan - 9) / a.ratio[2])));
+    q.nkc = (a.m[2] + q.kt - 1) / q.kt;
+    q.kt = (a.m[2] + q.nkc - 1) / q.nkc;
+    q.nkc = (a.m[2] + q.kt - 1) / q.kt;
+    q.span = staged_extent(a.ratio[2], q.kt, 1);
+    q.tj = kRsRows;
+    while (q.tj > 1 && staged_extent(a.ratio[1], q.tj, 1) > 32) q.tj /= 2;
+    q.rows = std::min(staged_extent(a.ratio[1], q.tj, 1), a.n[1]);
+    q.njt = (a.m[1] + q.tj - 1) / q.tj;
+    // planes per workgroup: fewer while that leaves less than eight workgroups a CU
+    q.ti = kRsPlanes;
+    const long long per = (long long)q.njt * q.nkc;
+    while (q.ti > 1 && per * ((a.m[0] + q.ti - 1) / q.ti) < 2048) q.ti /= 2;
+    q.tiles = per * ((a.m[0] + q.ti - 1) / q.ti);
+    return launch_staged(resample_linear, q, 0, st);
+}
+
+hipError_t launch_cubic(const ResampleArgs &a, hipStream_t st) {
+    StagedArgs q{};
+    q.a = a;
+    const auto extent = [&](int d, int cnt) { return std::min(staged_extent(a.ratio[d], cnt, 5), a.n[d]); };
     // outputs along z whose input columns fit a tile
     q.kt = a.m[2];
-    if (staged_extent(a.ratio[2], q.kt, a.n[2], W) > kRsSpan) {
-        q.kt = std::max(1, std::min(a.m[2], (int)((kRsSpan - 9) / a.ratio[2])));
+    if (extent(2, q.kt) > kRsCubicSpan) {
+        q.kt = std::max(1, std::min(a.m[2], (int)((kRsCubicSpan - 9) / a.ratio[2])));
         const int nt = (a.m[2] + q.kt - 1) / q.kt;     // equal tiles
         q.kt = (a.m[2] + nt - 1) / nt;
     }
     q.kt = std::min(q.kt, 2048);
-    q.span = staged_extent(a.ratio[2], q.kt, a.n[2], W);
+    q.span = extent(2, q.kt);
     q.tj = kRsRows;
-    while (q.tj > 1 && staged_extent(a.ratio[1], q.tj, a.n[1], W) > 32) q.tj /= 2;
-    q.rows = staged_extent(a.ratio[1], q.tj, a.n[1], W);
+    while (q.tj > 1 && extent(1, q.tj) > 32) q.tj /= 2;
+    q.rows = extent(1, q.tj);
+    q.ti = 1;
     q.njt = (a.m[1] + q.tj - 1) / q.tj;
     q.nkc = (a.m[2] + q.kt - 1) / q.kt;
     q.tiles = (long long)a.m[0] * q.njt * q.nkc;
-    const size_t lds = sizeof(float) * q.span * (size_t)(q.rows + (W == 4 ? q.tj : 0));
-    const long long grid = (q.tiles + 7) / 8 * 8;
-    if (grid > 0x7fffffffLL || q.span > kRsSpan || lds > 48 * 1024) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(resample_staged<W>, dim3((unsigned)grid), dim3(kRsBlock), lds, st, q);
-    return hipGetLastError();
+    return launch_staged(resample_cubic, q, q.tj, st);
 }
 
 // Cubic B-spline prefilter: c[i] = sum_k sqrt(3) z^|k| w[i + k], z = sqrt(3) - 2, as one
@@ -482,9 +612,9 @@ extern "C" int pvd_resample(const float *in, int n0, int n1, int n2, const doubl
     if (g > 65536) g = 65536;
     hipError_t e;
     if (interp == PVD_INTERP_LINEAR && a.ratio[2] <= kStagedLinear && a.ratio[1] <= kStagedLinear) {
-        e = launch_staged<2>(a, (hipStream_t)stream);
+        e = launch_linear(a, (hipStream_t)stream);
     } else if (interp == PVD_INTERP_CUBIC && a.ratio[2] <= kStagedCubic && a.ratio[1] <= kStagedCubic) {
-        e = launch_staged<4>(a, (hipStream_t)stream);
+        e = launch_cubic(a, (hipStream_t)stream);
     } else {
         hipLaunchKernelGGL(resample_kernel, dim3((unsigned)g), dim3(256), 0, (hipStream_t)stream, a);
         e = hipGetLastError();

@@ -147,3 +147,22 @@ def test_prefilter_windows_and_what_a_non_finite_sample_reaches(shape):
         i = np.arange(shape[a]).reshape([-1 if b == a else 1 for b in range(3)])
         far |= np.abs(i - p) > 14 + 2
     np.testing.assert_allclose(out[far], got[far], rtol=0, atol=2e-6 * np.abs(img).max())
+
+
+@pytest.mark.parametrize("shape,ratio", [
+    ((9, 70, 40), (0.13, 0.07, 0.5)),        # four planes a workgroup, two left over, zeros past the end
+    ((3, 9, 260), (0.5, 1.0, 0.5)),          # 513 + outputs along z: two tiles of a row's lanes
+    ((2, 11, 330), (1.0, 0.9, 1.0)),         # more input columns than one tile
+    ((5, 6, 700), (1.5, 1.2, 2.4)),
+])
+def test_linear_tiles_of_several_planes(shape, ratio):
+    """The linear kernel's tiles (eight rows, 512 outputs or 320 input columns, up to four
+    planes) and their remainders: FP32 products with FP64 coordinates, 1e-6 of max|image|."""
+    from pyvoxeldosimetry_amd.resample import resample
+    _say("linear tiles", shape, ratio)
+    rng = np.random.default_rng(sum(shape))
+    img = rng.normal(size=shape).astype(np.float32)
+    out_shape = tuple(max(1, int(np.ceil(n / r)) + 1) for n, r in zip(shape, ratio))
+    got = resample(img, (1.0, 1.0, 1.0), ratio, "linear", output_shape=out_shape, scale=1.0)
+    exp = ors.resample(img, (1.0, 1.0, 1.0), ratio, "linear", shape=out_shape)
+    np.testing.assert_allclose(got, exp, rtol=0, atol=1e-6 * np.abs(img).max())

@@ -119,6 +119,11 @@ __device__ __forceinline__ void classify(const TissueArgs &a, float v, unsigned 
 constexpr int kItems = 4;
 constexpr int kTissueGrid = 2048;       // workgroups (at most)
 constexpr int kTissueBlock = 512;
+// Consecutive items a workgroup takes at once: 512 bytes of each map, half a wave.  Fewer
+// spread an implant's metal over more workgroups, more keep the stream's bursts long.
+// 512x512x400 with no, one, two implants, us: 64 items 311 / 329 / 372, 32 items 303 / 325 /
+// 351, 16 items 332 / 363 / 368.
+constexpr int kTissueChunk = 32;
 
 template <int NM>
 __device__ __forceinline__ void tissue_store1(const TissueArgs &a, long long v, float h) {
@@ -215,17 +220,17 @@ __global__ __launch_bounds__(kTissueBlock) void tissue_map(TissueArgs a, long lo
     __shared__ int count;
     __shared__ double sw[9];
     const int tid = threadIdx.x;
-    // Wave-sized chunks of 64 items are dealt round the workgroups, so an implant (whose
-    // metal sits in neighbouring rows) is spread over many of them.
+    // Chunks of items are dealt round the workgroups, so an implant (whose metal sits in
+    // neighbouring rows) is spread over many of them.
     const long long stride = (long long)gridDim.x * kTissueBlock;
     auto item = [&](long long b0, int e) {                   // e = u * kTissueBlock + thread
-        return b0 + ((long long)(e >> 6) * gridDim.x + blockIdx.x) * 64 + (e & 63);
+        return b0 + ((long long)(e / kTissueChunk) * gridDim.x + blockIdx.x) * kTissueChunk + e % kTissueChunk;
     };
     if (tid == 0) count = 0;
     if (R == 4 && tid < 9) sw[tid] = a.w[tid];
     lds_barrier();
     const long long whole = n / V;                           // items of V voxels; one more if n % V
-    for (long long b0 = 0; b0 + blockIdx.x * 64LL < nitems; b0 += kItems * stride) {
+    for (long long b0 = 0; b0 + blockIdx.x * (long long)kTissueChunk < nitems; b0 += kItems * stride) {
         float h[kItems][V];
         unsigned which[kItems];
 #pragma unroll
@@ -320,8 +325,8 @@ extern "C" int pvd_tissue_map(const pvd_tissue_params *p, const float *ct, int n
     const bool vec = (r4 ? n >= 4 : n2 % 4 == 0) && aligned(ct, 16) && (!corrected || aligned(corrected, 16)) &&
                      (!density || aligned(density, 16)) && (!class_bits || aligned(class_bits, 4));
     const long long items = vec ? (n + 3) / 4 : n;
-    // (a workgroup per 64 items at most, so that small volumes spread as well)
-    const long long g = std::min<long long>((items + 63) / 64, kTissueGrid);
+    // (a workgroup per chunk at most, so that small volumes spread as well)
+    const long long g = std::min<long long>((items + kTissueChunk - 1) / kTissueChunk, kTissueGrid);
     const dim3 grid((unsigned)g), block(kTissueBlock);
     if (a.nmat <= 16) {
         if (vec && r4) hipLaunchKernelGGL((tissue_map<true, 4, 16>), grid, block, 0, st, a, items, n);

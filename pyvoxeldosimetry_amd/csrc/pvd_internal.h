@@ -452,6 +452,9 @@ hipError_t pvd_fft_xy3_set_lds(size_t bytes);
 
 // Record an error message for pvd_last_error() and return `code` (pvd_api.hip).
 int pvd_set_error(int code, const char *fmt, ...);
+// Outputs larger than this (the MI355X's last-level cache) are stored non-temporally by the
+// passes that only stream: cached, they would evict each other and what else is in use.
+#define PVD_STREAM_BYTES (256LL << 20)
 // Map a HIP error to PVD_ENOMEM / PVD_EHIP with a message.
 int pvd_hip_error(hipError_t e, const char *what);
 

@@ -177,7 +177,10 @@ struct StagedArgs {
 // a branch per output): a workgroup now keeps a lane's z positions over kRsPlanes output
 // planes and gives each wave whole rows, about 12 instructions an output.
 // 251x251x196 -> 512x512x400 150 -> 126 us (94 at the copy rate), 400x300x350 -> half 32.6
-// -> 29.7; eight planes a workgroup with 64 VGPRs 170.
+// -> 29.7; eight planes a workgroup with 64 VGPRs 170.  NT: outputs that do not fit the
+// last-level cache are stored past it (124 -> 101 us; 333x333x333 outputs, 148 MB, would
+// take 54 instead of 43).
+template <bool NT>
 __global__ __launch_bounds__(kRsBlock) void resample_linear(StagedArgs q) {
     extern __shared__ float rs_lds[];
     __shared__ float s_wy[kRsRows];
@@ -274,7 +277,9 @@ __global__ __launch_bounds__(kRsBlock) void resample_linear(StagedArgs q) {
                 const float e0 = fmaf(fy, p1[c] - p[c], p[c]);
                 const float e1 = fmaf(fy, p1[c + 1] - p[c + 1], p[c + 1]);
                 const float x = fmaf(kf[u], e1 - e0, e0);
-                o[64 * u] = a.scale * (ko[u] < 0 ? 0.0f : x);
+                const float y = a.scale * (ko[u] < 0 ? 0.0f : x);
+                if (NT) __builtin_nontemporal_store(y, o + 64 * u);
+                else o[64 * u] = y;
             }
         }
         lds_barrier();       // S is read
@@ -432,7 +437,9 @@ hipError_t launch_linear(const ResampleArgs &a, hipStream_t st) {
     const long long per = (long long)q.njt * q.nkc;
     while (q.ti > 1 && per * ((a.m[0] + q.ti - 1) / q.ti) < 2048) q.ti /= 2;
     q.tiles = per * ((a.m[0] + q.ti - 1) / q.ti);
-    return launch_staged(resample_linear, q, 0, st);
+    const long long bytes = 4LL * a.m[0] * a.m[1] * a.m[2];
+    return bytes > PVD_STREAM_BYTES ? launch_staged(resample_linear<true>, q, 0, st)
+                                    : launch_staged(resample_linear<false>, q, 0, st);
 }
 
 hipError_t launch_cubic(const ResampleArgs &a, hipStream_t st) {

@@ -41,6 +41,15 @@ __device__ __forceinline__ void bspline3_weights(float t, float w[4]) {
     w[3] = t3 * (1.0f / 6.0f);
 }
 
+// An output: stored past the last-level cache where the whole output is larger than it.
+// 512x512x400 linear 124 -> 98 us, 512x512x512 nearest 285 -> 206, cubic 309 -> 273; 333x333x333
+// (148 MB) would take 54 us instead of 43.
+template <bool NT>
+__device__ __forceinline__ void put(float *p, float v) {
+    if (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+
 // continuous index -> (lower neighbour, weight of the upper one); false if outside
 __device__ __forceinline__ bool axis_pos(double c, int n, int &i0, float &f) {
     if (!(c >= -0.5 && c < n - 0.5)) return false;
@@ -55,6 +64,7 @@ __device__ __forceinline__ bool axis_pos(double c, int n, int &i0, float &f) {
 // to the 8 XCDs round-robin, so block b works on row chunk (b % 8) * G/8 + b / 8:
 // each XCD walks a contiguous band of rows and neighbouring output rows find
 // their shared input rows in that XCD's L2.
+template <bool NT>
 __global__ __launch_bounds__(256) void resample_kernel(ResampleArgs a) {
     const int rows = a.m[0] * a.m[1];
     const int G = gridDim.x;
@@ -101,7 +111,7 @@ __global__ __launch_bounds__(256) void resample_kernel(ResampleArgs a) {
                         v = fmaf(wxy[r], s, v);
                     }
                 }
-                orow[k] = a.scale * v;
+                put<NT>(orow + k, a.scale * v);
             }
             continue;
         }
@@ -114,7 +124,7 @@ __global__ __launch_bounds__(256) void resample_kernel(ResampleArgs a) {
                 float f2;
                 float v = 0.0f;
                 if (axis_pos(k * a.ratio[2], a.n[2], b2, f2)) v = p[min(max(b2 + (f2 >= 0.5f), 0), a.n[2] - 1)];
-                orow[k] = a.scale * v;
+                put<NT>(orow + k, a.scale * v);
             }
             continue;
         }
@@ -138,7 +148,7 @@ __global__ __launch_bounds__(256) void resample_kernel(ResampleArgs a) {
                 const float e1 = fmaf(f1, c11 - c10, c10);
                 v = fmaf(f0, e1 - e0, e0);
             }
-            orow[k] = a.scale * v;
+            put<NT>(orow + k, a.scale * v);
         }
     }
 }
@@ -177,9 +187,7 @@ struct StagedArgs {
 // a branch per output): a workgroup now keeps a lane's z positions over kRsPlanes output
 // planes and gives each wave whole rows, about 12 instructions an output.
 // 251x251x196 -> 512x512x400 150 -> 126 us (94 at the copy rate), 400x300x350 -> half 32.6
-// -> 29.7; eight planes a workgroup with 64 VGPRs 170.  NT: outputs that do not fit the
-// last-level cache are stored past it (124 -> 101 us; 333x333x333 outputs, 148 MB, would
-// take 54 instead of 43).
+// -> 29.7; eight planes a workgroup with 64 VGPRs 170.
 template <bool NT>
 __global__ __launch_bounds__(kRsBlock) void resample_linear(StagedArgs q) {
     extern __shared__ float rs_lds[];
@@ -277,9 +285,7 @@ __global__ __launch_bounds__(kRsBlock) void resample_linear(StagedArgs q) {
                 const float e0 = fmaf(fy, p1[c] - p[c], p[c]);
                 const float e1 = fmaf(fy, p1[c + 1] - p[c + 1], p[c + 1]);
                 const float x = fmaf(kf[u], e1 - e0, e0);
-                const float y = a.scale * (ko[u] < 0 ? 0.0f : x);
-                if (NT) __builtin_nontemporal_store(y, o + 64 * u);
-                else o[64 * u] = y;
+                put<NT>(o + 64 * u, a.scale * (ko[u] < 0 ? 0.0f : x));
             }
         }
         lds_barrier();       // S is read
@@ -289,6 +295,7 @@ __global__ __launch_bounds__(kRsBlock) void resample_linear(StagedArgs q) {
 // Cubic: T[j][z] = S interpolated along y, then 4 values of T an output; an output plane per
 // workgroup.  (The linear kernel's form held 135 VGPRs here and took 120x250x250 @3.3 ->
 // 1.5 mm from 181 to 255 us.)
+template <bool NT>
 __global__ __launch_bounds__(kRsBlock) void resample_cubic(StagedArgs q) {
     constexpr int W = 4, B = 3;          // neighbours, and the furthest of them past the base index
     extern __shared__ float rs_lds[];
@@ -390,7 +397,7 @@ __global__ __launch_bounds__(kRsBlock) void resample_cubic(StagedArgs q) {
                 const float *p = T + jj * q.span;
                 x = fmaf(wz[3], p[z[3]], fmaf(wz[2], p[z[2]], fmaf(wz[1], p[z[1]], wz[0] * p[z[0]])));
             }
-            orow[(long long)jj * a.m[2] + k] = a.scale * x;
+            put<NT>(orow + (long long)jj * a.m[2] + k, a.scale * x);
         }
     }
 }
@@ -407,6 +414,8 @@ int staged_extent(double ratio, int cnt, int past) {
 // inputs, gather / staged us: linear 102 / 97 at 2.04, 38 / 52 at 3.0; cubic 225 / 110 at
 // 3.0, 99 / 72 at 4.5, 32 / 34 at 8.3.
 constexpr double kStagedLinear = 2.5, kStagedCubic = 8.0;
+
+bool streamed(const ResampleArgs &a) { return 4LL * a.m[0] * a.m[1] * a.m[2] > PVD_STREAM_BYTES; }
 
 template <typename Kernel>
 hipError_t launch_staged(Kernel kernel, const StagedArgs &q, int tj, hipStream_t st) {
@@ -437,9 +446,8 @@ hipError_t launch_linear(const ResampleArgs &a, hipStream_t st) {
     const long long per = (long long)q.njt * q.nkc;
     while (q.ti > 1 && per * ((a.m[0] + q.ti - 1) / q.ti) < 2048) q.ti /= 2;
     q.tiles = per * ((a.m[0] + q.ti - 1) / q.ti);
-    const long long bytes = 4LL * a.m[0] * a.m[1] * a.m[2];
-    return bytes > PVD_STREAM_BYTES ? launch_staged(resample_linear<true>, q, 0, st)
-                                    : launch_staged(resample_linear<false>, q, 0, st);
+    return streamed(a) ? launch_staged(resample_linear<true>, q, 0, st)
+                       : launch_staged(resample_linear<false>, q, 0, st);
 }
 
 hipError_t launch_cubic(const ResampleArgs &a, hipStream_t st) {
@@ -462,7 +470,8 @@ hipError_t launch_cubic(const ResampleArgs &a, hipStream_t st) {
     q.njt = (a.m[1] + q.tj - 1) / q.tj;
     q.nkc = (a.m[2] + q.kt - 1) / q.kt;
     q.tiles = (long long)a.m[0] * q.njt * q.nkc;
-    return launch_staged(resample_cubic, q, q.tj, st);
+    return streamed(a) ? launch_staged(resample_cubic<true>, q, q.tj, st)
+                       : launch_staged(resample_cubic<false>, q, q.tj, st);
 }
 
 // Cubic B-spline prefilter: c[i] = sum_k sqrt(3) z^|k| w[i + k], z = sqrt(3) - 2, as one
@@ -623,7 +632,8 @@ extern "C" int pvd_resample(const float *in, int n0, int n1, int n2, const doubl
     } else if (interp == PVD_INTERP_CUBIC && a.ratio[2] <= kStagedCubic && a.ratio[1] <= kStagedCubic) {
         e = launch_cubic(a, (hipStream_t)stream);
     } else {
-        hipLaunchKernelGGL(resample_kernel, dim3((unsigned)g), dim3(256), 0, (hipStream_t)stream, a);
+        if (streamed(a)) hipLaunchKernelGGL(resample_kernel<true>, dim3((unsigned)g), dim3(256), 0, (hipStream_t)stream, a);
+        else hipLaunchKernelGGL(resample_kernel<false>, dim3((unsigned)g), dim3(256), 0, (hipStream_t)stream, a);
         e = hipGetLastError();
     }
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch resample");

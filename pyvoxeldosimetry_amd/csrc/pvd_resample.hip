@@ -1,8 +1,8 @@
 // Grid-to-grid resampling (nearest / trilinear / cubic B-spline) for the activity
 // <-> kernel resolution round trip of the dose path.  Linear and cubic interpolation
 // are separable: a workgroup interpolates the input along x once into LDS and writes a
-// tile of output rows from it (resample_linear, resample_cubic); nearest, and outputs much coarser than
-// the input, gather each output's neighbours (resample_kernel).  Coordinates are formed
+// tile of output rows from it (resample_linear, resample_cubic); nearest, and outputs much
+// coarser than the input, gather each output's neighbours (resample_kernel).  Coordinates are formed
 // in FP64 so that equal spacings map every output voxel exactly onto an input voxel.
 // The cubic B-spline coefficients come from a separable mirror-boundary prefilter
 // (two launches: x, then y and z).
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(256) void resample_kernel(ResampleArgs a) {
 // The gather form above issues 8 (linear) or 64 (cubic) loads per output and is bound
 // by them; here a tile costs W loads per input element it spans, so the cost follows
 // the input samples per output and the pass goes to the HBM stores.  Gather -> staged:
-// 251x251x196 -> 512x512x400 linear 321 -> 126 us (94 at the copy rate), cubic 2139 ->
+// 251x251x196 -> 512x512x400 linear 321 -> 98 us (88 at the copy rate), cubic 2139 ->
 // 209; 301x301x233 -> 206x206x160 linear 51 -> 25 us, cubic 283 -> 41 (22).
 constexpr int kRsBlock = 256;      // threads
 constexpr int kRsU = 5;            // linear: columns per lane in flight in step 1

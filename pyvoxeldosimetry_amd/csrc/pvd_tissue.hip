@@ -112,7 +112,7 @@ __device__ __forceinline__ void classify(const TissueArgs &a, float v, unsigned 
 // Lanes whose voxels hold metal do not fill them in place (81 dependent load rounds for
 // radius 4, while a rod along z puts 40 such lanes into one wave): they list their items in
 // LDS, and the workgroup fills the listed items together, a wave per item.  512x512x400 with
-// a plate and a rod of 22,000 metal voxels: 502 -> 352 us (305 without implants: 4.5 TB/s,
+// a plate and a rod of 22,000 metal voxels: 502 -> 338 us (294 without implants: 4.6 TB/s,
 // the copy rate is 5.0); 511x300x401 599 -> 235, 200^3 with one plate 260 -> 35.  A volume
 // that is two thirds metal takes longer than before (401x30x50: 167 -> 225 us): a wave per
 // item has less in flight than a lane per item.

@@ -99,6 +99,9 @@ int pvd_cnn_input_layer(const float *activity, const float *density, const float
  * not needed by pvd_cnn_layer_grad).  x and y 16-byte aligned, y not x. */
 int pvd_cnn_train_layer(const void *x, int cin, const void *w, const float *bias, void *y, unsigned *mask, int n0,
                         int n1, int n2, void *stream);
+/* The same on the listed blocks only (NULL: the whole volume), y and mask alike. */
+int pvd_cnn_train_layer_blocks(const void *x, int cin, const void *w, const float *bias, void *y, unsigned *mask,
+                               int n0, int n1, int n2, const int *blocks, const int *nblocks, void *stream);
 
 /* The blocks within the network's 6-voxel receptive field of the region dp >= frac *
  * (*dose_max): block_list receives their indices (in no fixed order) and *nblocks their

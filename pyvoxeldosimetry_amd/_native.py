@@ -92,6 +92,7 @@ SIGNATURES = {
     "pvd_cnn_conv_fwd": (_I, [_P, _I, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _P, _P, _P]),
     "pvd_cnn_input_layer": (_I, [_P, _P, _P, _P, _P, ctypes.c_longlong, _P, _P, _P, _I, _I, _I, _P, _P, _P]),
     "pvd_cnn_train_layer": (_I, [_P, _I, _P, _P, _P, _P, _I, _I, _I, _P]),
+    "pvd_cnn_train_layer_blocks": (_I, [_P, _I, _P, _P, _P, _P, _I, _I, _I, _P, _P, _P]),
     "pvd_cnn_grad_parts": (ctypes.c_size_t, [_I, _I, _I]),
     "pvd_cnn_out_grad_parts": (ctypes.c_size_t, [_I, _I, _I]),
     "pvd_cnn_layer_grad": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),

@@ -71,7 +71,8 @@ constexpr size_t fwd_lds_bytes() {
            (size_t)(FWD_THREADS / 64) * FWD_STAGE;
 }
 
-template <int CIN, int EPI>
+// MASK (a residual layer in training): a.mask instead of a.act.
+template <int CIN, int EPI, bool MASK = false>
 __global__ __launch_bounds__(FWD_THREADS) void cnn_conv_fwd(ConvArgs a) {
     extern __shared__ uint4 lds_u4[];
     char *lds = reinterpret_cast<char *>(lds_u4);
@@ -200,7 +201,16 @@ __global__ __launch_bounds__(FWD_THREADS) void cnn_conv_fwd(ConvArgs a) {
             // stores).  One wave reads only what it wrote, in program order.
             uint16_t *sy = reinterpret_cast<uint16_t *>(stg);
             const uint4 *src = reinterpret_cast<const uint4 *>(stg);
-            if (a.act) {                         // training: the activations first
+            if constexpr (MASK) {
+                // a voxel's 32 channels are a half wave: one ballot has the words of two voxels
+                uint32_t word = 0;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const unsigned long long on = __ballot(f2bf(fmaxf(acc[i] + bco, 0.0f)) != 0);
+                    if (m == i) word = (uint32_t)(kh ? on >> 32 : on);
+                }
+                if (m < 16) a.mask[vrow + mfma_row(m, lane)] = word;
+            } else if (a.act) {                  // the activations first
 #pragma unroll
                 for (int i = 0; i < 16; ++i) sy[mfma_row(i, lane) * 32 + co] = f2bf(fmaxf(acc[i] + bco, 0.0f));
                 uint4 *dst = reinterpret_cast<uint4 *>(a.act + vrow * 32);
@@ -1538,16 +1548,16 @@ int num_cus() {
     return g_num_cus;
 }
 
-template <int CIN, int EPI>
+template <int CIN, int EPI, bool MASK = false>
 hipError_t launch_fwd(const ConvArgs &a, int blocks, hipStream_t st) {
     static bool attr = false;
     if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_fwd<CIN, EPI>,
+        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_fwd<CIN, EPI, MASK>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)fwd_lds_bytes<CIN>());
         if (e != hipSuccess) return e;
         attr = true;
     }
-    hipLaunchKernelGGL((cnn_conv_fwd<CIN, EPI>), dim3(blocks), dim3(FWD_THREADS), fwd_lds_bytes<CIN>(), st, a);
+    hipLaunchKernelGGL((cnn_conv_fwd<CIN, EPI, MASK>), dim3(blocks), dim3(FWD_THREADS), fwd_lds_bytes<CIN>(), st, a);
     return hipGetLastError();
 }
 
@@ -1762,15 +1772,24 @@ int pvd_cnn_input_layer(const float *activity, const float *density, const float
 
 int pvd_cnn_train_layer(const void *x, int cin, const void *w, const float *bias, void *y, unsigned *mask, int n0,
                         int n1, int n2, void *stream) {
+    return pvd_cnn_train_layer_blocks(x, cin, w, bias, y, mask, n0, n1, n2, nullptr, nullptr, stream);
+}
+
+int pvd_cnn_train_layer_blocks(const void *x, int cin, const void *w, const float *bias, void *y, unsigned *mask,
+                               int n0, int n1, int n2, const int *blocks, const int *nblocks, void *stream) {
+    if ((blocks == nullptr) != (nblocks == nullptr)) return pvd_set_error(PVD_EINVAL, "blocks and nblocks go together");
     if (int rc = check_grid(n0, n1, n2)) return rc;
     if (!x || !w || !y || !mask) return pvd_set_error(PVD_EINVAL, "null argument");
     if (cin != 4 && cin != 32) return pvd_set_error(PVD_EINVAL, "cin must be 4 or 32 (got %d)", cin);
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15)
         return pvd_set_error(PVD_EINVAL, "x and y must be 16-byte aligned");
     ConvArgs a{(const uint16_t *)x, (const uint16_t *)w, bias, (const uint16_t *)x, (uint16_t *)y, nullptr, nullptr,
-               n0, n1, n2, nullptr, nullptr, mask};
+               n0, n1, n2, blocks, nblocks, mask};
+    const long long total = (long long)((n0 + FWD_BX - 1) / FWD_BX) * ((n1 + FWD_BY - 1) / FWD_BY) * (n2 >> 5);
+    const int grid = (int)(total < num_cus() ? total : num_cus());
     hipStream_t st = (hipStream_t)stream;
-    const hipError_t e = cin == 4 ? launch_io<true>(a, 0, true, st) : launch_layer(a, st);
+    const hipError_t e = cin == 4 ? launch_io<true>(a, grid, !blocks, st)
+                         : blocks ? launch_fwd<32, PVD_CNN_EPI_RESID_RELU, true>(a, grid, st) : launch_layer(a, st);
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch CNN training layer");
 }
 

@@ -157,22 +157,24 @@ class ResidualCNN:
         """x: BF16 [n, 16] inputs, or (inference) ``maps``: activity, density and plain dose,
         FP32, the device maxima of activity and plain dose that scale them, and the pitch
         of the maps' rows in floats; returns the FP32 correction r [n] (workspace tensor).
-        ``keep_activations=False`` (inference) skips the ReLU masks backward needs (a
-        whole-volume forward writes them).
+        ``keep_activations=False`` (inference) skips the ReLU masks backward needs.
         ``blocks``: (block list, count) device tensors from ``pvd_cnn_region_blocks``:
-        every layer runs on those blocks only, and r is defined on the region they cover."""
+        every layer runs on those blocks only, and r is defined on the region they cover
+        (training: a loss mask within that region has the whole volume's gradients)."""
+        if keep_activations and maps is not None:
+            raise ValueError("maps are for inference (keep_activations=False): backward reads the packed input")
         ws = self._workspace(shape)
         h = ws["h"]
+        bl, bn = blocks if blocks is not None else (None, None)
         # the input's channels 4..15 are zero (pvd_cnn_pack): the four-channel input layer
-        if keep_activations and blocks is None:
+        if keep_activations:
             for l in range(5):
-                nat.check(self.lib.pvd_cnn_train_layer(_p(x if l == 0 else h[l - 1]), 4 if l == 0 else 32,
-                                                       _p(self.w_bf16(l)), _p(self.bias(l)), _p(h[l]), _p(ws["mask"][l]),
-                                                       shape[0], shape[1], shape[2], self._stream()),
-                          "pvd_cnn_train_layer")
+                nat.check(self.lib.pvd_cnn_train_layer_blocks(_p(x if l == 0 else h[l - 1]), 4 if l == 0 else 32,
+                                                              _p(self.w_bf16(l)), _p(self.bias(l)), _p(h[l]),
+                                                              _p(ws["mask"][l]), shape[0], shape[1], shape[2], _p(bl),
+                                                              _p(bn), self._stream()), "pvd_cnn_train_layer_blocks")
         else:
             if maps is not None:
-                bl, bn = blocks if blocks is not None else (None, None)
                 nat.check(self.lib.pvd_cnn_input_layer(*(_p(t) for t in maps[:5]), maps[5], _p(self.w_bf16(0)),
                                                        _p(self.bias(0)), _p(h[0]), *shape, _p(bl), _p(bn),
                                                        self._stream()), "pvd_cnn_input_layer")

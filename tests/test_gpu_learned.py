@@ -860,3 +860,59 @@ def test_monte_carlo_maps_histories_alike(shape, histories, every):
         again = mc.edep(act, rho, 2.0, histories, seed=5)
         assert float((e - again).abs().max()) <= 1e-12 * float(e.max())
         assert float(e.min()) >= 0.0
+
+
+@pytest.mark.parametrize("shape", [(9, 18, 64), (40, 33, 96), (24, 70, 32)])
+def test_training_on_a_region_list_has_the_whole_volume_gradients(shape):
+    """Forward on the blocks around a region and a loss within it, on a workspace that has seen
+    no other forward and on one that holds another input's: every gradient is the whole
+    volume's bit for bit (outside the blocks dL/dh is zero, and both forms of a layer round
+    alike)."""
+    import ctypes
+    import torch
+    from pyvoxeldosimetry_amd import _native as nat
+    from pyvoxeldosimetry_amd.learned.cnn import ResidualCNN
+    _say("cnn region training", shape)
+    lib = nat.load()
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    n = int(np.prod(shape))
+
+    def network():
+        net = ResidualCNN(seed=3)
+        a, b = net.offsets[5]
+        g = torch.Generator().manual_seed(4)
+        net.master[a:b].view(27, 32, 32)[:, 0] = (torch.randn((27, 32), generator=g) * 0.05).cuda()
+        net.bf16.copy_(net.master.to(torch.bfloat16))
+        return net
+
+    def inputs(seed):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        x = torch.zeros((n, 16), device="cuda", dtype=torch.bfloat16)
+        x[:, :3] = torch.rand((n, 3), device="cuda", generator=g).to(torch.bfloat16)
+        where = torch.zeros(shape, device="cuda")
+        where[:3, 2:5, 3:9] = 1.0                       # the region: its blocks leave part of the volume out
+        return x, where.reshape(-1), 1.0 + 0.2 * torch.rand(n, device="cuda", generator=g)
+
+    def gradients(net, x, mask, dt, blocks):
+        net.forward(x, shape, blocks=blocks)
+        net.loss_and_grad(torch.ones_like(dt), dt, mask, shape)
+        net.backward(x, shape)
+        return net.grad.clone()
+
+    region, whole = network(), network()
+    for seed in (1, 2):
+        x, mask, dt = inputs(seed)
+        nb = int(lib.pvd_cnn_region_block_count(*shape))
+        flags, blist = (torch.empty(nb, dtype=torch.int32, device="cuda") for _ in range(2))
+        count, top = torch.empty(1, dtype=torch.int32, device="cuda"), torch.ones(1, device="cuda")
+        torch.cuda.synchronize()
+        nat.check(lib.pvd_cnn_region_blocks(p(mask), *shape, p(top), ctypes.c_float(0.5), p(flags), p(blist), p(count),
+                                            None), "pvd_cnn_region_blocks")
+        torch.cuda.synchronize()
+        assert 0 < int(count) < nb
+        want = gradients(whole, x, mask, dt, None)
+        got = gradients(region, x, mask, dt, (blist, count))
+        assert all(want[a:a + 27 * 32 * 3].any() for a, _ in whole.offsets)
+        assert torch.equal(got, want)
+    with pytest.raises(ValueError):                     # no packed input, which backward reads
+        region.forward(None, shape, maps=(mask, mask, mask, top, top, shape[2]))

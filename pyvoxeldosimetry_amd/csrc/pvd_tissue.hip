@@ -50,16 +50,14 @@ __device__ __forceinline__ double fill_source(float c, float metal) {
     return (double)c;
 }
 
-// Smoothed values of V consecutive voxels of one z-row (x, y, z0 .. z0+V-1),
-// for the voxels flagged in `which`.  For each of the (2r+1)^2 (dx, dy) rows the
-// lane issues all V+2r reflected z-loads of that row before using them, so a
-// metal voxel costs (2r+1)^2 load round trips, shared by the V voxels.  R is
-// the radius when known at compile time (the window then lives in registers),
-// or -1 for a run-time radius.
-template <int V, int R>
+// Smoothed values of V consecutive voxels of one z-row (x, y, z0 .. z0+V-1), for the voxels
+// flagged in `which`, at the run-time radius.  For each of the (2r+1)^2 (dx, dy) rows the lane
+// issues all V+2r reflected z-loads of that row before using them, so a metal voxel costs
+// (2r+1)^2 load round trips, shared by the V voxels.
+template <int V>
 __device__ void metal_fill_row(const TissueArgs &a, int x, int y, int z0, unsigned which, float *h) {
-    const int r = R >= 0 ? R : a.radius, side = 2 * r + 1;
-    constexpr int W = V + 2 * (R >= 0 ? R : PVD_TISSUE_MAX_RADIUS);
+    const int r = a.radius, side = 2 * r + 1;
+    constexpr int W = V + 2 * PVD_TISSUE_MAX_RADIUS;
     double acc[V];
 #pragma unroll
     for (int k = 0; k < V; ++k) acc[k] = 0.0;
@@ -71,17 +69,12 @@ __device__ void metal_fill_row(const TissueArgs &a, int x, int y, int z0, unsign
             float win[W];
 #pragma unroll
             for (int j = 0; j < W; ++j)
-                if (R >= 0 || j < V + 2 * r) win[j] = row[reflect(z0 - r + j, a.n2)];
+                if (j < V + 2 * r) win[j] = row[reflect(z0 - r + j, a.n2)];
 #pragma unroll
             for (int k = 0; k < V; ++k) {
                 if (!(which & (1u << k))) continue;
                 double s = 0.0;
-                if constexpr (R >= 0) {
-#pragma unroll
-                    for (int dz = 0; dz < 2 * R + 1; ++dz) s += a.w[dz] * fill_source(win[k + dz], a.metal);
-                } else {
-                    for (int dz = 0; dz < side; ++dz) s += a.w[dz] * fill_source(win[k + dz], a.metal);
-                }
+                for (int dz = 0; dz < side; ++dz) s += a.w[dz] * fill_source(win[k + dz], a.metal);
                 acc[k] += wxy * s;
             }
         }
@@ -112,10 +105,10 @@ __device__ __forceinline__ void classify(const TissueArgs &a, float v, unsigned 
 // Lanes whose voxels hold metal do not fill them in place (81 dependent load rounds for
 // radius 4, while a rod along z puts 40 such lanes into one wave): they list their items in
 // LDS, and the workgroup fills the listed items together, a wave per item.  512x512x400 with
-// a plate and a rod of 22,000 metal voxels: 502 -> 338 us (294 without implants: 4.6 TB/s,
-// the copy rate is 5.0); 511x300x401 599 -> 235, 200^3 with one plate 260 -> 35.  A volume
-// that is two thirds metal takes longer than before (401x30x50: 167 -> 225 us): a wave per
-// item has less in flight than a lane per item.
+// a plate and a rod of 22,000 metal voxels: 505 -> 329 us (294 without implants: 4.6 TB/s,
+// the copy rate is 5.0); 511x300x401 580 -> 181, 200^3 with two implants 233 -> 37.  Volumes
+// within the last-level cache and without metal pay for the list: 200^3 23.1 -> 28.1, 256x256x200
+// 36.8 -> 39.5.
 constexpr int kItems = 4;
 constexpr int kTissueGrid = 2048;       // workgroups (at most)
 constexpr int kTissueBlock = 512;
@@ -124,6 +117,16 @@ constexpr int kTissueBlock = 512;
 // 512x512x400 with no, one, two implants, us: 64 items 311 / 329 / 372, 32 items 303 / 325 /
 // 351, 16 items 332 / 363 / 368.
 constexpr int kTissueChunk = 32;
+// Chunks a workgroup has before there are more than kTissueFew workgroups (a CU each): a
+// chunk each costs 64^3 12.1 us without metal, this rule 4.2 (100^3 13.4 -> 6.8, 128^3 14.6 ->
+// 11.1).  With two implants 64^3 18.8 -> 15.1, 128^3 19.0 -> 20.6; 32 chunks 26.4 there.
+constexpr int kTissuePer = 16, kTissueFew = 256;
+// A workgroup with at least kTissueDense items of metal, kTissuePerSpan or more of them to each
+// span of kSpan voxels that holds any, fills whole spans: a third of the instructions an item
+// where most items are listed.  200^3, single items -> spans: its first two thirds metal 2640 ->
+// 486 us, random 30 % 3175 -> 725, random 10 % (4 items a span) 1557 -> 700; random 2 % (1.5)
+// would take 500 instead of 453.
+constexpr int kTissueDense = 16, kTissuePerSpan = 3;
 
 template <int NM>
 __device__ __forceinline__ void tissue_store1(const TissueArgs &a, long long v, float h) {
@@ -183,6 +186,14 @@ __device__ __forceinline__ unsigned metal_of(const TissueArgs &a, const float *h
     return which;
 }
 
+// The lane, opaque: what the fills derive from it (rows, columns, weights' places) is computed
+// where it is used and not kept in registers over the streaming loop.
+__device__ __forceinline__ int fill_lane() {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+
 // Fill of the cnt <= V voxels of item i by a wave, radius 4 (sw: the nine weights in LDS):
 // lane (g, j) sums wxy * source over the rows (dx, dy) g, g + G, ... at z = z0 - 4 + j (W
 // consecutive floats of a row per group: coalesced), the groups are added, and the outputs
@@ -190,7 +201,7 @@ __device__ __forceinline__ unsigned metal_of(const TissueArgs &a, const float *h
 template <int V, int NM>
 __device__ __forceinline__ void metal_fill_wave(const TissueArgs &a, const double *sw, long long i, int cnt) {
     constexpr int R = 4, W = V + 2 * R, G = 64 / W, ROWS = 81, PER = (ROWS + G - 1) / G;
-    const int lane = threadIdx.x & 63, g = lane / W, j = lane - g * W;
+    const int lane = fill_lane(), g = lane / W, j = lane - g * W;
     auto fold = [](int k, int n) { return k < 0 || k >= n ? reflect(k, n) : k; };
     long long xy = i * V / a.n2;
     int z0 = (int)(i * V - xy * a.n2);
@@ -225,12 +236,50 @@ __device__ __forceinline__ void metal_fill_wave(const TissueArgs &a, const doubl
     }
 }
 
-template <bool VEC, int R, int NM, bool NT = false>
-__global__ __launch_bounds__(kTissueBlock) void tissue_map(TissueArgs a, long long nitems, long long n) {
+// Fill of `run` <= kSpan consecutive voxels of a z-row by a wave, radius 4: a lane per column
+// z0 - 4 + lane sums it over the 81 rows.  Voxels without metal keep their value.  (The offsets
+// of a plane's nine rows lie in lanes 0..8: as uniform addresses they took the scalar registers
+// of the streaming loop's tables, 511x300x401 without metal 150 -> 161 us.)
+constexpr int kSpan = 48;                // a third of a chunk's voxels at most, with 8 more columns
+template <int NM>
+__device__ __forceinline__ void metal_fill_span(const TissueArgs &a, const double *sw, int x, int y, int z0, int run) {
+    constexpr int R = 4;
+    const int lane = fill_lane();
+    auto fold = [](int k, int n) { return k < 0 || k >= n ? reflect(k, n) : k; };
+    const int z = fold(z0 - R + lane, a.n2);
+    const long long yo = (long long)fold(y + min(lane, 2 * R) - R, a.n1) * a.n2;
+    double sum = 0.0;
+#pragma unroll 1
+    for (int dx = 0; dx <= 2 * R; ++dx) {
+        const float *col = a.ct + (long long)fold(x + dx - R, a.n0) * a.n1 * a.n2 + z;
+        float c[2 * R + 1];
+#pragma unroll
+        for (int dy = 0; dy <= 2 * R; ++dy) c[dy] = col[__shfl(yo, dy)];
+        double row = 0.0;
+#pragma unroll
+        for (int dy = 0; dy <= 2 * R; ++dy) row += sw[dy] * fill_source(c[dy], a.metal);
+        sum += sw[dx] * row;
+    }
+    double out = 0.0;
+#pragma unroll
+    for (int dz = 0; dz <= 2 * R; ++dz) out += sw[dz] * __shfl(sum, (lane + dz) & 63);
+    if (lane < run) {
+        const long long v = ((long long)x * a.n1 + y) * a.n2 + z0 + lane;
+        const float c = a.ct[v];
+        tissue_store1<NM>(a, v, c > a.metal ? (float)out : c);
+    }
+}
+
+// (More than 16 materials: held to 128 registers, two workgroups a CU; 200^3 51 -> 37 us.)
+template <bool VEC, int NM, bool NT = false>
+__global__ __launch_bounds__(kTissueBlock) __attribute__((amdgpu_waves_per_eu(NM == 32 ? 4 : 1))) void tissue_map(TissueArgs a, long long nitems, long long n) {
     constexpr int V = VEC ? 4 : 1;
     __shared__ unsigned short list[kItems * kTissueBlock];
     __shared__ int count;
     __shared__ double sw[9];
+    constexpr int kChunks = kItems * kTissueBlock / kTissueChunk;
+    constexpr int kUnits = (kTissueChunk * V + kSpan - 1) / kSpan;
+    __shared__ unsigned flags[kChunks];
     const int tid = threadIdx.x;
     // Chunks of items are dealt round the workgroups, so an implant (whose metal sits in
     // neighbouring rows) is spread over many of them.
@@ -239,7 +288,7 @@ __global__ __launch_bounds__(kTissueBlock) void tissue_map(TissueArgs a, long lo
         return b0 + ((long long)(e / kTissueChunk) * gridDim.x + blockIdx.x) * kTissueChunk + e % kTissueChunk;
     };
     if (tid == 0) count = 0;
-    if (R == 4 && tid < 9) sw[tid] = a.w[tid];
+    if (tid < 9) sw[tid] = a.w[tid];
     lds_barrier();
     const long long whole = n / V;                           // items of V voxels; one more if n % V
     for (long long b0 = 0; b0 + blockIdx.x * (long long)kTissueChunk < nitems; b0 += kItems * stride) {
@@ -254,33 +303,88 @@ __global__ __launch_bounds__(kTissueBlock) void tissue_map(TissueArgs a, long lo
             const long long i = item(b0, u * kTissueBlock + tid);
             // (without artefact handling the metal threshold is infinite); the last n % V
             // voxels go through the list as well
-            which[u] = i < whole ? metal_of<V>(a, h[u]) : (R == 4 && i < nitems) ? 1u : 0u;
+            which[u] = i < whole ? metal_of<V>(a, h[u]) : i < nitems ? 1u : 0u;
             mine += which[u] ? 1 : 0;
             if (i < whole && !which[u]) tissue_store<V, NM, NT>(a, i, h[u]);
         }
-        if constexpr (R == 4) {
-            int at = mine ? atomicAdd(&count, mine) : 0;
+        int at = mine ? atomicAdd(&count, mine) : 0;
 #pragma unroll
-            for (int u = 0; u < kItems; ++u)
-                if (which[u]) list[at++] = (unsigned short)(u * kTissueBlock + tid);
+        for (int u = 0; u < kItems; ++u)
+            if (which[u]) list[at++] = (unsigned short)(u * kTissueBlock + tid);
+        lds_barrier();
+        const int m = count;
+        lds_barrier();
+        if (m == 0) continue;                            // uniform
+        if (tid == 0) count = 0;
+        bool spans = false;
+        if (m >= kTissueDense) {
+            static_assert(kTissueChunk == 32 && kChunks == 64, "a word of flags per chunk, a lane per word");
+            if (tid < kChunks) flags[tid] = 0u;
             lds_barrier();
-            const int m = count;
+            for (int k = tid; k < m; k += kTissueBlock) atomicOr(&flags[list[k] >> 5], 1u << (list[k] & 31));
             lds_barrier();
-            if (m == 0) continue;                            // uniform
-            if (tid == 0) count = 0;
+            const unsigned f = flags[tid & 63];
+            constexpr unsigned part = kUnits == 1 ? ~0u : (1u << (kSpan / V) % 32) - 1u;
+            int units = 0;                               // spans that hold metal
+#pragma unroll
+            for (int q = 0; q < kUnits; ++q) units += __popcll(__ballot(((f >> (q * (kSpan / V))) & part) != 0u));
+            spans = m >= kTissuePerSpan * units;
+        }
+        if (!spans) {
             for (int k = tid >> 6; k < m; k += kTissueBlock / 64) {
                 const long long i = item(b0, list[k]);
                 metal_fill_wave<V, NM>(a, sw, i, (int)min((long long)V, n - i * V));
             }
-            lds_barrier();                                   // list and count are free again
         } else {
-#pragma unroll
-            for (int u = 0; u < kItems; ++u)
-                if (which[u]) {
-                    const long long i = item(b0, u * kTissueBlock + tid), v0 = i * V, xy = v0 / a.n2;
-                    metal_fill_row<V, R>(a, (int)(xy / a.n1), (int)(xy % a.n1), (int)(v0 - xy * a.n2), which[u], h[u]);
-                    tissue_store<V, NM, NT>(a, i, h[u]);
+            for (int u = tid >> 6; u < kChunks * kUnits; u += kTissueBlock / 64) {
+                const int c = u / kUnits;
+                const unsigned on = flags[c];
+                const long long v0 = item(b0, c * kTissueChunk) * V;
+                int p = (u - c * kUnits) * kSpan;
+                const int end = (int)min((long long)min(p + kSpan, kTissueChunk * V), n - v0);
+                while (p < end) {
+                    const unsigned rest = on >> (p / V);
+                    if (!rest) break;
+                    if (!(rest & 1u)) {                  // to the next item with metal
+                        p = (p / V + __ffs(rest) - 1) * V;
+                        continue;
+                    }
+                    const long long xy = (v0 + p) / a.n2;
+                    const int z0 = (int)(v0 + p - xy * a.n2), x = (int)(xy / a.n1);
+                    const int run = min(end - p, a.n2 - z0);
+                    metal_fill_span<NM>(a, sw, x, (int)(xy - (long long)x * a.n1), z0, run);
+                    p += run;
                 }
+            }
+        }
+        lds_barrier();                                   // list and count are free again
+    }
+}
+
+// Any other radius: a lane holding metal fills it in place (VEC: n2 % 4 == 0, so an item lies in
+// one z-row).  Workgroups of 256 threads over consecutive items: the window of a run-time radius
+// takes 140-156 registers, which leave one workgroup of 512 on a CU (512x512x200 at sigma 0.6
+// with no, two implants 191, 308 us; in workgroups of 512 with the chunks above 511, 708).
+constexpr int kRowBlock = 256, kRowGrid = 4096;
+template <bool VEC, int NM>
+__global__ __launch_bounds__(kRowBlock) void tissue_map_rows(TissueArgs a, long long nitems) {
+    constexpr int V = VEC ? 4 : 1;
+    const long long stride = (long long)gridDim.x * kRowBlock;
+    for (long long i0 = blockIdx.x * (long long)kRowBlock + threadIdx.x; i0 < nitems; i0 += kItems * stride) {
+        float h[kItems][V];
+#pragma unroll
+        for (int u = 0; u < kItems; ++u)
+            if (i0 + u * stride < nitems) tissue_load<V>(a, i0 + u * stride, h[u]);
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) {
+            const long long i = i0 + u * stride;
+            if (i >= nitems) continue;
+            const unsigned which = metal_of<V>(a, h[u]);
+            if (which) {
+                const long long v0 = i * V, xy = v0 / a.n2;
+                metal_fill_row<V>(a, (int)(xy / a.n1), (int)(xy % a.n1), (int)(v0 % a.n2), which, h[u]);
+            }
+            tissue_store<V, NM, false>(a, i, h[u]);
         }
     }
 }
@@ -337,22 +441,21 @@ extern "C" int pvd_tissue_map(const pvd_tissue_params *p, const float *ct, int n
     // (other radii fill in place, four voxels of one z-row at a time)
     const bool vec = (r4 ? n >= 4 : n2 % 4 == 0) && aligned(ct, 16) && (!corrected || aligned(corrected, 16)) &&
                      (!density || aligned(density, 16)) && (!class_bits || aligned(class_bits, 4));
-    const long long items = vec ? (n + 3) / 4 : n;
-    // (a workgroup per chunk at most, so that small volumes spread as well)
-    const long long g = std::min<long long>((items + kTissueChunk - 1) / kTissueChunk, kTissueGrid);
-    const dim3 grid((unsigned)g), block(kTissueBlock);
-    if (a.nmat <= 16) {
-        if (vec && r4 && nt) hipLaunchKernelGGL((tissue_map<true, 4, 16, true>), grid, block, 0, st, a, items, n);
-        else if (vec && r4) hipLaunchKernelGGL((tissue_map<true, 4, 16>), grid, block, 0, st, a, items, n);
-        else if (vec) hipLaunchKernelGGL((tissue_map<true, -1, 16>), grid, block, 0, st, a, items, n);
-        else if (r4) hipLaunchKernelGGL((tissue_map<false, 4, 16>), grid, block, 0, st, a, items, n);
-        else hipLaunchKernelGGL((tissue_map<false, -1, 16>), grid, block, 0, st, a, items, n);
+    const bool few = a.nmat <= 16;
+    if (r4) {
+        const long long items = vec ? (n + 3) / 4 : n, chunks = (items + kTissueChunk - 1) / kTissueChunk;
+        const long long g = std::min<long long>(
+            {chunks, kTissueGrid, std::max<long long>(kTissueFew, (chunks + kTissuePer - 1) / kTissuePer)});
+        const auto kernel = vec ? nt ? few ? tissue_map<true, 16, true> : tissue_map<true, 32, true>
+                                     : few ? tissue_map<true, 16> : tissue_map<true, 32>
+                                : few ? tissue_map<false, 16> : tissue_map<false, 32>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)g), dim3(kTissueBlock), 0, st, a, items, n);
     } else {
-        if (vec && r4 && nt) hipLaunchKernelGGL((tissue_map<true, 4, 32, true>), grid, block, 0, st, a, items, n);
-        else if (vec && r4) hipLaunchKernelGGL((tissue_map<true, 4, 32>), grid, block, 0, st, a, items, n);
-        else if (vec) hipLaunchKernelGGL((tissue_map<true, -1, 32>), grid, block, 0, st, a, items, n);
-        else if (r4) hipLaunchKernelGGL((tissue_map<false, 4, 32>), grid, block, 0, st, a, items, n);
-        else hipLaunchKernelGGL((tissue_map<false, -1, 32>), grid, block, 0, st, a, items, n);
+        const long long items = vec ? n / 4 : n;
+        const long long g = std::min<long long>((items + kRowBlock - 1) / kRowBlock, kRowGrid);
+        const auto kernel = vec ? few ? tissue_map_rows<true, 16> : tissue_map_rows<true, 32>
+                                : few ? tissue_map_rows<false, 16> : tissue_map_rows<false, 32>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)g), dim3(kRowBlock), 0, st, a, items);
     }
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return pvd_hip_error(e, "launch tissue map");
     return PVD_OK;

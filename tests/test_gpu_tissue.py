@@ -153,3 +153,35 @@ def test_tissue_map_of_an_unaligned_view():
     tc = TissueComposition()
     for a, b in zip(tc.map(view), tc.map(view.clone())):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("shape", [(3, 5, 7), (20, 33, 31), (17, 16, 200), (9, 40, 50), (1, 1, 300), (40, 64, 2), (33, 64, 64)])
+@pytest.mark.parametrize("pattern", ["slab", "random", "all", "block"])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_tissue_map_mostly_metal(shape, pattern, aligned):
+    """Workgroups that fill spans of consecutive voxels (many metal items) beside those that
+    fill single items: spans cut by z-rows, chunks and the volume's end, windows wider than the
+    volume; the oracle's fill, tolerances as above."""
+    import torch
+    _say("tissue dense metal", shape, pattern, aligned)
+    rng = np.random.default_rng(sum(shape))
+    ct = rng.normal(40.0, 300.0, size=shape).astype(np.float32)
+    if pattern == "slab":
+        ct[: (2 * shape[0] + 2) // 3] = 2900.0
+    elif pattern == "random":
+        ct[rng.random(shape) < 0.6] = 2900.0
+    elif pattern == "all":
+        ct[:] = 3000.0
+        ct[-1, -1, -1] = -700.0
+    else:                                                      # dense and sparse metal in one volume
+        ct[: shape[0] // 2 + 1, : shape[1] // 2 + 1] = 2900.0
+        ct[rng.random(shape) < 0.01] = 2500.0
+    if aligned:
+        _check(ct)
+        return
+    from pyvoxeldosimetry_amd.tissue import TissueComposition
+    flat = torch.zeros(ct.size + 1, device="cuda")
+    view = flat[1:].view(shape)
+    view.copy_(torch.from_numpy(ct))
+    corr = TissueComposition().map(view)[0].cpu().numpy()
+    np.testing.assert_allclose(corr, ot.handle_artifacts(ct), rtol=1e-6, atol=5e-4)

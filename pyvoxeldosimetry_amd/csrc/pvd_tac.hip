@@ -1,13 +1,17 @@
 // Voxelwise time-activity-curve fits: one thread per voxel, FP64
 // Levenberg-Marquardt with analytic Jacobians (the reference runs
 // scipy.optimize.curve_fit voxel by voxel, time_integration/curve_fitting.py).
-// The normal equations are accumulated on the fly (no Jacobian storage), so a
-// thread holds the T samples, the system and the parameters in registers.  The kernel is
+// The normal equations are accumulated on the fly (no Jacobian storage).  The kernel is
 // compiled per model and per sample count (4, 8 or 16 at most), so that every loop is
-// unrolled and nothing is indexed at run time.  Bound by the FP64 vector instructions
-// (256x256x200 voxels, mono-exponential, 4 samples: 1995 -> 585 us, about 1700 instructions
-// a voxel; with one run-time-indexed kernel for all models, each trial point evaluated
-// twice and seven divisions a step before; NUKFIT f2 15.7 -> 4.7 ms, f3a at 100^3 141 -> 82).
+// unrolled and nothing is indexed at run time; a thread holds the samples, the system and
+// the parameters in registers, except the four- and five-parameter models with 9 to 16
+// samples, which spill (388 to 1236 bytes a lane, one wave per SIMD).  Bound by the FP64
+// vector instructions (256x256x200 voxels, mono-exponential, 4 samples: 1995 -> 585 us,
+// about 1700 instructions a voxel; with one run-time-indexed kernel for all models, each
+// trial point evaluated twice and seven divisions a step before; NUKFIT f2 15.7 -> 4.7 ms,
+// f3a at 100^3 141 -> 82 us).  The larger models at 48^3, us, run-time-indexed -> now: f4a 6
+// samples 3772 -> 2586, 12 samples 5186 -> 3756, 16 samples 6786 -> 4637; f4b 5628 -> 3367
+// at 8, 7041 -> 4539 at 16; tri-exponential 5781 -> 3568 at 8, 10528 -> 6813 at 16.
 #include "pvd_internal.h"
 #include "../../include/pvd_tac.h"
 
@@ -301,8 +305,10 @@ __global__ __launch_bounds__(256) void tac_fit_kernel(TacArgs a) {
             for (int i = 0; i < NT; ++i) y[i] -= y0;
             y[0] = 0.0;
         }
-        bool ok = NP <= q.n_times;
-        if (ok) ok = lm<MODEL, NT>(a, y, p);
+        bool ok = false;
+        if constexpr (NP <= NT) {                  // (else n_times <= NT < NP: no form can fit)
+            if (NP <= q.n_times) ok = lm<MODEL, NT>(a, y, p);
+        }
 #pragma unroll
         for (int k = 0; k < NP; ++k) ok = ok && isfinite(p[k]);
         if (!ok) {

@@ -123,3 +123,57 @@ def test_sample_counts_of_the_compiled_forms(T):
     pe, acce = tac.fit_basic(times, y, 64.1)
     np.testing.assert_allclose(p.reshape(2, -1), pe, rtol=2e-5, atol=1e-9)
     np.testing.assert_allclose(acc.reshape(-1), acce, rtol=5e-5)
+
+
+@pytest.mark.parametrize("T", [4, 6, 8, 9, 16])
+@pytest.mark.parametrize("model,name,centre", [("nukfit", "f3", [3.0, 0.02, 0.3]), ("nukfit", "f3a", [3.0, 0.6, 0.1]),
+                                               ("nukfit", "f4a", [3.0, 0.15, 1.0, 0.01]),
+                                               ("nukfit", "f4b", [4.0, 0.02, 2.0, 0.15, 0.8]),
+                                               ("nukfit", "f4c", [3.0, 0.02, 1.0, 0.1, 0.8]),
+                                               ("lmfit", "bi-exponential", [3.0, 80.0, 6.0]),
+                                               ("lmfit", "tri-exponential", [4.0, 90.0, 2.0, 15.0, 2.0])])
+def test_models_of_three_to_five_parameters_at_each_sample_count(T, model, name, centre):
+    """Every compiled form of the larger models, through the C ABI: noise-free curves whose
+    parameters lie within 10 % of the start are fitted and recovered.  The same iteration in
+    FP64 numpy recovers them within 8e-6 (FP32 samples) and the curve within 7e-8 of its
+    largest value; five FP32 parameters of a few units add 6e-7: tolerances 2e-5 and 2e-6.
+    Fewer samples than parameters: fail_params and status 0."""
+    import ctypes
+    import torch
+    from pyvoxeldosimetry_amd import _native as nat
+    _say("tac larger models", name, T)
+    lib = nat.load()
+    rng = np.random.default_rng(T)
+    n, k = 260, len(centre)                         # one past a block
+    hl = 64.1
+    f = tac.models(hl, np.log(2) / hl)[model == "lmfit"][name][0]
+    t = np.geomspace(0.5, 160.0, T)
+    truth = np.array(centre) * rng.uniform(0.9, 1.1, (n, k))
+    y = np.array([f(t, *p) for p in truth]).astype(np.float32)
+    q = nat.TacParams()
+    q.model = {"f3": 2, "f3a": 3, "f4a": 4, "f4b": 5, "f4c": 6, "bi-exponential": 8, "tri-exponential": 9}[name]
+    q.n_times, q.lambda_phys, q.max_iter, q.tol, q.auc_mode = T, np.log(2) / hl, 3333, 1.49012e-8, 1
+    for i in range(T):
+        q.t[i], q.w[i] = t[i], 1.0
+    for i in range(k):
+        q.p0[i], q.fail_params[i] = centre[i], 0.25 * centre[i]
+    maps = [torch.from_numpy(np.ascontiguousarray(y[:, i])).cuda() for i in range(T)]
+    params, auc = torch.empty((k, n), device="cuda"), torch.empty(n, device="cuda")
+    status = torch.full((n,), 7, dtype=torch.uint8, device="cuda")
+    ptr = lambda x: ctypes.c_void_p(x.data_ptr())  # noqa: E731
+    torch.cuda.synchronize()
+    nat.check(lib.pvd_tac_fit(ctypes.byref(q), (ctypes.c_void_p * T)(*[m.data_ptr() for m in maps]), n, ptr(params),
+                              ptr(auc), ptr(status), None), "pvd_tac_fit")
+    torch.cuda.synchronize()
+    p, s, a = params.cpu().double().numpy(), status.cpu().numpy(), auc.cpu().numpy()
+    if T < k:
+        assert not s.any()
+        np.testing.assert_allclose(p, np.tile(0.25 * np.array(centre)[:, None], n), rtol=1e-6)
+    else:
+        assert (s == 1).all()
+        np.testing.assert_allclose(p.T, truth, rtol=2e-5)
+    got = np.array([f(t, *p[:, i]) for i in range(n)])
+    if T >= k:
+        assert (np.abs(got - y).max(1) <= 2e-6 * np.abs(y).max(1)).all()
+    scale = np.array([tac.trapezoid(np.abs(g), t) for g in got])
+    np.testing.assert_array_less(np.abs(a - np.array([tac.trapezoid(g, t) for g in got])), 1e-5 * scale + 1e-30)

@@ -180,7 +180,12 @@ struct StagedArgs {
     int njt, nkc;                  // tiles along y and z
     int span, rows;                // LDS extents: input columns, input rows
     long long tiles;
+    long long first;               // tile of this launch's first workgroup
 };
+
+// Workgroups of a launch (at most): a launch has fewer than 2^32 threads, so larger outputs take
+// several.
+constexpr long long kRsGrid = 1 << 21;
 
 // Linear: an output takes the bilinear product of y and z from 2 x 2 values of S.  The
 // wave issue rate bound the tile-per-output-plane form (an FP64 coordinate, a row lookup and
@@ -198,7 +203,7 @@ __global__ __launch_bounds__(kRsBlock) void resample_linear(StagedArgs q) {
     constexpr int NW = kRsBlock / 64;
     // XCD-contiguous bands of tiles (neighbouring tiles share input rows in one L2)
     const long long G = gridDim.x;
-    const long long t = (long long)(blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
+    const long long t = q.first + (long long)(blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
     if (t >= q.tiles) return;
     const int kc = (int)(t % q.nkc);
     const long long ij = t / q.nkc;
@@ -305,7 +310,7 @@ __global__ __launch_bounds__(kRsBlock) void resample_cubic(StagedArgs q) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     // XCD-contiguous bands of tiles (neighbouring tiles share input rows in one L2)
     const long long G = gridDim.x;
-    const long long t = (long long)(blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
+    const long long t = q.first + (long long)(blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
     if (t >= q.tiles) return;
     const int kc = (int)(t % q.nkc);
     const long long ij = t / q.nkc;
@@ -418,12 +423,16 @@ constexpr double kStagedLinear = 2.5, kStagedCubic = 8.0;
 bool streamed(const ResampleArgs &a) { return 4LL * a.m[0] * a.m[1] * a.m[2] > PVD_STREAM_BYTES; }
 
 template <typename Kernel>
-hipError_t launch_staged(Kernel kernel, const StagedArgs &q, int tj, hipStream_t st) {
+hipError_t launch_staged(Kernel kernel, StagedArgs &q, int tj, hipStream_t st) {
     const size_t lds = sizeof(float) * q.span * (size_t)(q.rows + tj);
-    const long long grid = (q.tiles + 7) / 8 * 8;
-    if (grid > 0x7fffffffLL || q.span > kRsSpan || lds > 48 * 1024) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kRsBlock), lds, st, q);
-    return hipGetLastError();
+    if (q.span > kRsSpan || lds > 48 * 1024) return hipErrorInvalidValue;
+    hipError_t e = hipSuccess;
+    for (q.first = 0; q.first < q.tiles && e == hipSuccess; q.first += kRsGrid) {
+        const long long grid = (std::min(q.tiles - q.first, kRsGrid) + 7) / 8 * 8;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kRsBlock), lds, st, q);
+        e = hipGetLastError();
+    }
+    return e;
 }
 
 hipError_t launch_linear(const ResampleArgs &a, hipStream_t st) {
@@ -526,9 +535,10 @@ constexpr int kBsZ = 27;           // outputs per unit along z (odd: neighbourin
 constexpr int kBsCols = 17 * kBsZ + 2 * kBsK;      // columns of a z tile (at most): 487
 
 __global__ __launch_bounds__(256) void bspline_x(const float *__restrict__ src, float *__restrict__ dst, int n0,
-                                                 long long plane, long long gx) {
-    const long long p = blockIdx.x % gx * 256LL + threadIdx.x;
-    const int x0 = (int)(blockIdx.x / gx) * kBsX;
+                                                 long long plane, long long gx, long long first) {
+    const long long b = first + blockIdx.x;
+    const long long p = b % gx * 256LL + threadIdx.x;
+    const int x0 = (int)(b / gx) * kBsX;
     const long long pc = p < plane ? p : plane - 1;
     float c[kBsX];
     bs_line([&](int i) { return src[(long long)mirror_index(min(x0 + i - kBsK, n0 - 1 + kBsK), n0) * plane + pc]; }, c);
@@ -585,7 +595,6 @@ extern "C" int pvd_bspline_prefilter(const float *in, int n0, int n1, int n2, fl
     if (coef == in || tmp == in || coef == tmp) return pvd_set_error(PVD_EINVAL, "coef, tmp and in must differ");
     const long long plane = (long long)n1 * n2;
     const long long gx = (plane + 255) / 256, blocks_x = gx * ((n0 + (long long)kBsX - 1) / kBsX);
-    if (blocks_x > 0x7fffffffLL) return pvd_set_error(PVD_ENOTSUP, "grid too large");
     const int nyt = (n1 + kBsY - 1) / kBsY;
     // z tiles of equal width, a multiple of the unit; a thread per column
     const int nt = (n2 + kBsCols - 2 * kBsK - 1) / (kBsCols - 2 * kBsK);
@@ -593,12 +602,16 @@ extern "C" int pvd_bspline_prefilter(const float *in, int n0, int n1, int n2, fl
     const int block = (std::max(zt + 2 * kBsK, kBsY * (zt / kBsZ)) + 63) / 64 * 64;
     const int ld = zt + 2 * kBsK + 1;
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(bspline_x, dim3((unsigned)blocks_x), dim3(256), 0, st, in, tmp, n0, plane, gx);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return pvd_hip_error(e, "launch B-spline prefilter");
+    hipError_t e = hipSuccess;
+    for (long long first = 0; first < blocks_x; first += kRsGrid) {
+        hipLaunchKernelGGL(bspline_x, dim3((unsigned)std::min(blocks_x - first, kRsGrid)), dim3(256), 0, st, in, tmp, n0,
+                           plane, gx, first);
+        e = hipGetLastError();
+        if (e != hipSuccess) return pvd_hip_error(e, "launch B-spline prefilter");
+    }
     const int nzt = (n2 + zt - 1) / zt;
     const long long tiles = (long long)n0 * nyt * nzt;
-    hipLaunchKernelGGL(bspline_yz, dim3((unsigned)std::min<long long>(tiles, 0x7fffffffLL)), dim3(block),
+    hipLaunchKernelGGL(bspline_yz, dim3((unsigned)std::min(tiles, kRsGrid)), dim3(block),
                        sizeof(float) * kBsY * ld, st, (const float *)tmp, coef, n1, n2, zt, ld, nzt, nyt, tiles);
     e = hipGetLastError();
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch B-spline prefilter");

@@ -166,3 +166,54 @@ def test_linear_tiles_of_several_planes(shape, ratio):
     got = resample(img, (1.0, 1.0, 1.0), ratio, "linear", output_shape=out_shape, scale=1.0)
     exp = ors.resample(img, (1.0, 1.0, 1.0), ratio, "linear", shape=out_shape)
     np.testing.assert_allclose(got, exp, rtol=0, atol=1e-6 * np.abs(img).max())
+
+
+@pytest.mark.parametrize("mode,size,out_size", [("linear", 1500, (24000, 24001)), ("cubic", 1500, (12000, 12001))])
+def test_outputs_of_more_workgroups_than_one_launch_takes(mode, size, out_size):
+    """A flat output whose tiles have 2^32 threads or more (17e6 and more workgroups of 256): the
+    image is an outer product, so every output is the product of two one-dimensional results.
+    FP32 interpolation along three axes on either side: 4e-6 of the largest product."""
+    import torch
+    from pyvoxeldosimetry_amd.resample import resample_device
+    _say("resample beyond a launch", mode, out_size)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    g, h = (torch.randn(size, device="cuda", generator=gen) for _ in range(2))
+    ratio = (size / out_size[0], size / out_size[1], 1.0)
+    image = (g[:, None] * h[None, :]).reshape(size, size, 1).contiguous()
+    out = torch.full((*out_size, 1), float("nan"), device="cuda")
+    resample_device(image, (1.0,) * 3, ratio, mode, (*out_size, 1), out=out)
+    G = resample_device(g.reshape(size, 1, 1), (1.0,) * 3, ratio, mode, (out_size[0], 1, 1)).reshape(-1)
+    H = resample_device(h.reshape(1, size, 1), (1.0,) * 3, ratio, mode, (1, out_size[1], 1)).reshape(-1)
+    tol = 4e-6 * float(G.abs().max() * H.abs().max())
+    for i in range(0, out_size[0], 1000):
+        d = (out[i:i + 1000, :, 0] - G[i:i + 1000, None] * H[None, :]).abs().max()
+        assert float(d) <= tol, (i, float(d))              # (a NaN that was left fails)
+
+
+def test_prefilter_of_more_workgroups_than_one_launch_takes():
+    """A line of 540e6 voxels (either launch beyond 2^32 threads): every coefficient is written
+    and those at both ends and around the launches' seam are a short line's (15 samples and
+    more from its cuts; three FP32 recursions over other windows: 4e-6)."""
+    import ctypes
+    import torch
+    from pyvoxeldosimetry_amd import _native as nat
+    _say("prefilter beyond a launch")
+    lib = nat.load()
+    n = 540_000_001
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+
+    def prefilter(x):
+        coef, tmp = torch.full_like(x, float("nan")), torch.empty_like(x)
+        torch.cuda.synchronize()
+        nat.check(lib.pvd_bspline_prefilter(p(x), x.numel(), 1, 1, p(coef), p(tmp), None), "pvd_bspline_prefilter")
+        torch.cuda.synchronize()
+        return coef
+
+    x = torch.rand(n, device="cuda", generator=torch.Generator(device="cuda").manual_seed(4))
+    coef = prefilter(x)
+    assert not bool(torch.isnan(coef).any())
+    seam = (1 << 21) * 32
+    for a in (0, seam - 2048, 8 * seam - 2048, n - 4096):
+        part = prefilter(x[a:a + 4096].clone())
+        lo, hi = (0 if a == 0 else 64), (4096 if a + 4096 == n else 4032)
+        assert float((part[lo:hi] - coef[a + lo:a + hi]).abs().max()) <= 4e-6

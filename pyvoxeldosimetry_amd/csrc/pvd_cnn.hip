@@ -1365,30 +1365,34 @@ __global__ __launch_bounds__(256) void cnn_adam(float *p, const float *g, float 
 // on cols / 256 blocks: the 2048 x 32 bias partials of a 128^3 layer took about 460 us and
 // the 256 x 27648 weight partials 61 us; both now take 4-6 us.)
 constexpr int RED_COLS = 32, RED_GROUPS = 32;
+constexpr int RED_GRID = 1 << 20;      // workgroups (at most; a launch has fewer than 2^32 threads)
 __global__ __launch_bounds__(RED_COLS * RED_GROUPS) void reduce_rows(const float *__restrict__ part, int rows, int cols,
                                                                      float *__restrict__ out, int accumulate,
                                                                      int pitch) {
     __shared__ float red[RED_GROUPS][RED_COLS + 1];
     const int l = threadIdx.x & (RED_COLS - 1), g = threadIdx.x / RED_COLS;
-    const int c = blockIdx.x * RED_COLS + l;
-    const float *p = part + (c < cols ? c : cols - 1);
-    float s = 0.0f;
-    for (int r0 = g; r0 < rows; r0 += 8 * RED_GROUPS) {
-        float v[8];
+    for (long long b = blockIdx.x; b * RED_COLS < cols; b += gridDim.x) {
+        const long long c = b * RED_COLS + l;
+        const float *p = part + (c < cols ? c : cols - 1);
+        float s = 0.0f;
+        for (long long r0 = g; r0 < rows; r0 += 8 * RED_GROUPS) {
+            float v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = p[(size_t)min(r0 + u * RED_GROUPS, rows - 1) * cols];
+            for (int u = 0; u < 8; ++u) v[u] = p[(size_t)min(r0 + u * RED_GROUPS, rows - 1LL) * cols];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) s += r0 + u * RED_GROUPS < rows ? v[u] : 0.0f;
-    }
-    red[g][l] = s;
-    __syncthreads();
+            for (int u = 0; u < 8; ++u) s += r0 + u * RED_GROUPS < rows ? v[u] : 0.0f;
+        }
+        red[g][l] = s;
+        __syncthreads();
 #pragma unroll
-    for (int h = RED_GROUPS / 2; h > 0; h >>= 1) {
-        if (g < h) red[g][l] += red[g + h][l];
+        for (int h = RED_GROUPS / 2; h > 0; h >>= 1) {
+            if (g < h) red[g][l] += red[g + h][l];
+            __syncthreads();
+        }
+        float *o = out + (size_t)b * pitch + l;                  // `pitch` floats per 32 columns
+        if (g == 0 && c < cols) *o = accumulate ? *o + red[0][l] : red[0][l];
         __syncthreads();
     }
-    float *o = out + (size_t)blockIdx.x * pitch + l;         // `pitch` floats per 32 columns
-    if (g == 0 && c < cols) *o = accumulate ? *o + red[0][l] : red[0][l];
 }
 
 __global__ __launch_bounds__(256) void cnn_pack(const float *__restrict__ a, const float *__restrict__ d,
@@ -1855,7 +1859,7 @@ int pvd_cnn_wgrad(const void *x, int cin, const void *dz, float *dw, float *work
     hipError_t e = cin == 16 ? launch_wgrad<16>(a, blocks, st) : launch_wgrad<32>(a, blocks, st);
     if (e != hipSuccess) return pvd_hip_error(e, "launch weight gradient");
     const int cols = 27 * 32 * cin;
-    hipLaunchKernelGGL(reduce_rows, dim3((cols + RED_COLS - 1) / RED_COLS), dim3(RED_COLS * RED_GROUPS), 0, st,
+    hipLaunchKernelGGL(reduce_rows, dim3(std::min((cols - 1) / RED_COLS + 1, RED_GRID)), dim3(RED_COLS * RED_GROUPS), 0, st,
                        (const float *)work, blocks, cols, dw, 0, RED_COLS);
     e = hipGetLastError();
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch reduction");
@@ -2023,7 +2027,7 @@ size_t pvd_cnn_region_block_count(int n0, int n1, int n2) {
 
 int pvd_reduce_rows(const float *part, int rows, int cols, float *out, int accumulate, void *stream) {
     if (!part || !out || rows < 1 || cols < 1) return pvd_set_error(PVD_EINVAL, "bad argument");
-    hipLaunchKernelGGL(reduce_rows, dim3((cols + RED_COLS - 1) / RED_COLS), dim3(RED_COLS * RED_GROUPS), 0,
+    hipLaunchKernelGGL(reduce_rows, dim3(std::min((cols - 1) / RED_COLS + 1, RED_GRID)), dim3(RED_COLS * RED_GROUPS), 0,
                        (hipStream_t)stream, part, rows, cols, out, accumulate, RED_COLS);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? PVD_OK : pvd_hip_error(e, "launch reduction");

@@ -916,3 +916,28 @@ def test_training_on_a_region_list_has_the_whole_volume_gradients(shape):
         assert torch.equal(got, want)
     with pytest.raises(ValueError):                     # no packed input, which backward reads
         region.forward(None, shape, maps=(mask, mask, mask, top, top, shape[2]))
+
+
+@pytest.mark.parametrize("rows,cols", [(2, 140_000_003), ((1 << 31) - 1, 1)])
+def test_reduce_rows_of_the_largest_extents(rows, cols):
+    """More columns than one launch has threads for, and a row count at the end of its type
+    (zeros but for both ends and both sides of 2^30): exact."""
+    import ctypes
+    import torch
+    from pyvoxeldosimetry_amd import _native as nat
+    _say("reduce_rows extents", rows, cols)
+    lib = nat.load()
+    if cols > 1:
+        part = torch.arange(rows * cols, device="cuda", dtype=torch.int32).remainder_(1021).float().reshape(rows, cols)
+        want = part.sum(0)
+    else:
+        part = torch.zeros((rows, cols), device="cuda")
+        at = torch.tensor([0, 1, (1 << 30) - 1, 1 << 30, rows - 300, rows - 2, rows - 1], device="cuda")
+        part[at, 0] = 1.0
+        want = torch.tensor([float(at.numel())], device="cuda")
+    out = torch.full((cols,), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    nat.check(lib.pvd_reduce_rows(ctypes.c_void_p(part.data_ptr()), rows, cols, ctypes.c_void_p(out.data_ptr()), 0, None),
+              "pvd_reduce_rows")
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)

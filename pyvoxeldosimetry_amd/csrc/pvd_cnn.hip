@@ -1554,13 +1554,8 @@ int num_cus() {
 
 template <int CIN, int EPI, bool MASK = false>
 hipError_t launch_fwd(const ConvArgs &a, int blocks, hipStream_t st) {
-    static bool attr = false;
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_fwd<CIN, EPI, MASK>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)fwd_lds_bytes<CIN>());
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
+    static pvd_device_once once;
+    if (hipError_t e = pvd_lds_limit(once, cnn_conv_fwd<CIN, EPI, MASK>, fwd_lds_bytes<CIN>()); e != hipSuccess) return e;
     hipLaunchKernelGGL((cnn_conv_fwd<CIN, EPI, MASK>), dim3(blocks), dim3(FWD_THREADS), fwd_lds_bytes<CIN>(), st, a);
     return hipGetLastError();
 }
@@ -1593,13 +1588,8 @@ void out_grad_plan(MarchArgs *q, int n0, int n1, int n2) {
 
 template <int MODE>
 hipError_t launch_march(MarchArgs &q, hipStream_t st) {
-    static bool attr = false;
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_march<MODE>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)MR_LDS);
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
+    static pvd_device_once once;
+    if (hipError_t e = pvd_lds_limit(once, cnn_conv_march<MODE>, MR_LDS); e != hipSuccess) return e;
     march_plan(&q, q.c.n0, q.c.n1, q.c.n2);
     const long long grid = ((long long)q.nby * q.nbz * q.nseg + 7) / 8 * 8;
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
@@ -1615,14 +1605,9 @@ hipError_t launch_layer(const ConvArgs &a, hipStream_t st) {
 
 template <int BX, int BY, bool MAPS>
 hipError_t launch_in_as(const ConvArgs &a, const InMaps &mp, int blocks, hipStream_t st) {
-    static bool attr = false;
+    static pvd_device_once once;
     constexpr size_t lds = in_lds_bytes<BX, BY>();
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_in<BX, BY, MAPS>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
+    if (hipError_t e = pvd_lds_limit(once, cnn_conv_in<BX, BY, MAPS>, lds); e != hipSuccess) return e;
     hipLaunchKernelGGL((cnn_conv_in<BX, BY, MAPS>), dim3(blocks), dim3(FWD_THREADS), lds, st, a, mp);
     return hipGetLastError();
 }
@@ -1634,26 +1619,16 @@ hipError_t launch_in(const ConvArgs &a, const InMaps *mp, int blocks, hipStream_
 
 template <int BX, int BY>
 hipError_t launch_out(const ConvArgs &a, int blocks, hipStream_t st) {
-    static bool attr = false;
+    static pvd_device_once once;
     constexpr size_t lds = out_lds_bytes<BX, BY>();
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_out<BX, BY>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
+    if (hipError_t e = pvd_lds_limit(once, cnn_conv_out<BX, BY>, lds); e != hipSuccess) return e;
     hipLaunchKernelGGL((cnn_conv_out<BX, BY>), dim3(blocks), dim3(FWD_THREADS), lds, st, a);
     return hipGetLastError();
 }
 
 hipError_t launch_out_march(const ConvArgs &a, hipStream_t st) {
-    static bool attr = false;
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void *)cnn_conv_out_march,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)OM_LDS);
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
+    static pvd_device_once once;
+    if (hipError_t e = pvd_lds_limit(once, cnn_conv_out_march, OM_LDS); e != hipSuccess) return e;
     // two workgroups a CU (77 KB of LDS each), segments of at least 4 planes
     const int nby = (a.n1 + OM_Y - 1) / OM_Y, nbz = a.n2 >> 5;
     const long long cols = (long long)nby * nbz;
@@ -1679,13 +1654,8 @@ hipError_t launch_io(const ConvArgs &a, int grid, bool whole, hipStream_t st, co
 
 template <int CIN>
 hipError_t launch_wgrad(const WgradArgs &a, int blocks, hipStream_t st) {
-    static bool attr = false;
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void *)cnn_wgrad<CIN>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)wg_lds<CIN>());
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
+    static pvd_device_once once;
+    if (hipError_t e = pvd_lds_limit(once, cnn_wgrad<CIN>, wg_lds<CIN>()); e != hipSuccess) return e;
     hipLaunchKernelGGL((cnn_wgrad<CIN>), dim3(blocks), dim3(WG_THREADS), wg_lds<CIN>(), st, a);
     return hipGetLastError();
 }
@@ -1887,13 +1857,8 @@ int pvd_cnn_out_wgrad(const void *x, const void *dr, float *dw, float *work, int
     if (int rc = check_grid(n0, n1, n2)) return rc;
     if (!x || !dr || !dw || !work) return pvd_set_error(PVD_EINVAL, "null argument");
     if (reinterpret_cast<uintptr_t>(x) & 15) return pvd_set_error(PVD_EINVAL, "x must be 16-byte aligned");
-    static bool attr = false;
-    if (!attr) {
-        const hipError_t e = hipFuncSetAttribute((const void *)cnn_out_wgrad,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)OW_LDS);
-        if (e != hipSuccess) return pvd_hip_error(e, "set LDS limit");
-        attr = true;
-    }
+    static pvd_device_once once;
+    if (hipError_t e = pvd_lds_limit(once, cnn_out_wgrad, OW_LDS); e != hipSuccess) return pvd_hip_error(e, "set LDS limit");
     const long long total = (long long)n0 * ((n1 + OW_Y - 1) / OW_Y) * (n2 >> 5);
     if (total > 0x7fffffffLL) return pvd_set_error(PVD_ENOTSUP, "grid too large");
     // (32 partial sums of this layer fit where pvd_cnn_wgrad_work_floats has one workgroup's)

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "../../include/pvd.h"
+#include "pvd_once.h"
 
 #define PVD_MAXSTAGE 16
 
@@ -449,6 +450,17 @@ hipError_t pvd_fft_z_set_lds(size_t bytes);
 hipError_t pvd_fft_xy1_set_lds(size_t bytes);
 hipError_t pvd_fft_xy2_set_lds(size_t bytes);
 hipError_t pvd_fft_xy3_set_lds(size_t bytes);
+
+// Dynamic LDS limit of a kernel, set at its first launch on each device.
+template <typename K>
+inline hipError_t pvd_lds_limit(pvd_device_once &once, K *kernel, size_t bytes) {
+    int dev = 0;
+    if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+    return once.run(dev, [&] {
+        return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)bytes);
+    });
+}
 
 // Record an error message for pvd_last_error() and return `code` (pvd_api.hip).
 int pvd_set_error(int code, const char *fmt, ...);

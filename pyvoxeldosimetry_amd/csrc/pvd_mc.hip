@@ -436,14 +436,9 @@ hipError_t launch_mc(const MCArgs &a, const float *act, const float *dens, doubl
                      int per_src, int kinds, long long nvox, hipStream_t st) {
     const size_t lds = TILE ? sizeof(double) * (size_t)nvox : 0;
     if (TILE) {
-        static bool attr = false;
-        if (!attr) {
-            const int most = (int)(sizeof(double) * kMcTileVoxels);
-            const hipError_t e = hipFuncSetAttribute((const void *)pvd_mc_kernel<TILE, I>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, most);
-            if (e != hipSuccess) return e;
-            attr = true;
-        }
+        static pvd_device_once once;
+        const hipError_t e = pvd_lds_limit(once, pvd_mc_kernel<TILE, I>, sizeof(double) * kMcTileVoxels);
+        if (e != hipSuccess) return e;
     }
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess ||

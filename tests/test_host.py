@@ -234,3 +234,37 @@ def test_subregion_box_centres_on_the_maximum_and_stays_inside():
     assert subregion_box(a, 64) == (slice(0, 64), slice(16, 80), slice(6, 70))
     with pytest.raises(ValueError):
         subregion_box(torch.zeros((32, 80, 70)), 64)
+
+
+def test_kernel_limits_are_set_once_on_each_device(tmp_path):
+    """A kernel's LDS limit belongs to the device it was set on: set at the first call on every
+    device, again after a failure, and behind no process-wide flag."""
+    import re
+    import shutil
+    import subprocess
+    csrc = os.path.join(ROOT, "pyvoxeldosimetry_amd", "csrc")
+    for f in sorted(os.listdir(csrc)):
+        with open(os.path.join(csrc, f)) as h:
+            assert not re.search(r"static\s+bool\s+\w+\s*=\s*false", h.read()), f
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    src = tmp_path / "once.cpp"
+    src.write_text("""
+#include <cstdio>
+#include "pvd_once.h"
+int main() {
+    static pvd_device_once once;
+    int runs[70] = {};
+    for (int turn = 0; turn < 3; ++turn)
+        for (int dev = 0; dev < 70; ++dev) {
+            const int e = once.run(dev, [&] { ++runs[dev]; return dev == 5 && turn == 0 ? 9 : 0; });
+            if (e != (dev == 5 && turn == 0 ? 9 : 0)) return 1;
+        }
+    for (int dev = 0; dev < 70; ++dev)
+        if (runs[dev] != (dev == 5 ? 2 : dev < 64 ? 1 : 3)) return 2;
+    return 0;
+}
+""")
+    exe = tmp_path / "once"
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-I", csrc, str(src), "-o", str(exe)], check=True)
+    subprocess.run([str(exe)], check=True)

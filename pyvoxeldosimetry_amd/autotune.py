@@ -8,7 +8,9 @@ tile size of each pass (8 / 16 / 32 lines per workgroup, z then y then x), the
 largest Stockham radix (16 or 8) and the LDS Stockham stages in place of the
 register-resident transforms, keeping a change only when it is at least 2 %
 faster.  Each candidate is timed with HIP events on synthetic input;
-the winner is cached in a JSON file keyed by shape, kernel, mode and device.
+the winner is cached in a JSON file keyed by shape, kernel, mode and device.  Entries
+from before the plans chose small tiles and whole planes for small volumes (without "own")
+are not used: their explicit tiles would keep such a volume off both; it is tuned again.
 """
 from __future__ import annotations
 
@@ -57,6 +59,11 @@ def _load_cache():
         return {}
 
 
+def _usable(entry):
+    """A cache entry written under the present layout rules, else None."""
+    return entry if isinstance(entry, dict) and "own" in entry else None
+
+
 def _save_cache(c):
     try:
         os.makedirs(os.path.dirname(_CACHE_PATH), exist_ok=True)
@@ -90,10 +97,10 @@ def tuned_plan(shape, kernel_shape, mode, kernel_dev, max_candidates: int = 6, s
     key = json.dumps([list(shape), list(kernel_shape), mode, torch.cuda.get_device_name(dev)])
     with _lock:
         cache = _load_cache()
-        hit = cache.get(key)
+        hit = _usable(cache.get(key))
     if hit is not None:
         fft = hit["algo"] == "fft"
-        walked = fft and not hit.get("own", False)     # tiles and radix found by the walk
+        walked = fft and not hit["own"]                # tiles and radix found by the walk
         plan = ConvPlan(shape, kernel_shape, mode=mode, algo=hit["algo"], fft_n=hit.get("fft_n") if fft else None,
                         tile=hit.get("tile") if walked else None, max_radix=hit.get("max_radix", 0) if walked else 0,
                         stockham=bool(hit.get("stockham", False)) and fft, device=dev)

@@ -268,3 +268,47 @@ int main() {
     exe = tmp_path / "once"
     subprocess.run(["g++", "-std=c++17", "-Wall", "-I", csrc, str(src), "-o", str(exe)], check=True)
     subprocess.run([str(exe)], check=True)
+
+
+def test_autotune_cache_entry_of_earlier_rules_does_not_pin_the_tiles(tmp_path, monkeypatch):
+    """An entry without "own" (explicit 16-line tiles, which keep a small volume off its whole
+    planes) is tuned again; one with it makes the plan it describes."""
+    import json
+    import torch
+    from pyvoxeldosimetry_amd import autotune
+    made = []
+
+    class Plan:
+        def __init__(self, shape, kernel_shape, **kw):
+            made.append(kw)
+            self.tile, self.max_radix, self.fft_n = (16, 16, 8), 8, kw.get("fft_n")
+
+        def set_kernel(self, k):
+            pass
+
+        def close(self):
+            pass
+
+    monkeypatch.setattr(autotune, "ConvPlan", Plan)
+    monkeypatch.setattr(autotune, "describe_plan", lambda *a, **k: {"fft_n": [80, 80, 80]})
+    monkeypatch.setattr(autotune, "time_plan", lambda p: 1.0)
+    monkeypatch.setattr(autotune, "_CACHE_PATH", str(tmp_path / "cache.json"))
+    monkeypatch.setattr(torch.cuda, "get_device_name", lambda d=None: "gpu")
+    kernel = torch.zeros((21, 21, 21))
+    key = json.dumps([[64, 64, 64], [21, 21, 21], "linear", "gpu"])
+    old = {"algo": "fft", "fft_n": [80, 80, 80], "ms": 1.0, "tile": [16, 16, 16], "max_radix": 16, "stockham": False}
+    for entry in (old, "damaged"):
+        made.clear()
+        (tmp_path / "cache.json").write_text(json.dumps({key: entry}))
+        autotune.tuned_plan((64, 64, 64), (21, 21, 21), "linear", kernel)
+        assert len(made) > 1 and not made[0].get("tile")
+        stored = json.loads((tmp_path / "cache.json").read_text())[key]
+        assert stored["own"] is True
+        made.clear()                                          # the next call: the stored plan, its own tiles
+        autotune.tuned_plan((64, 64, 64), (21, 21, 21), "linear", kernel)
+        assert len(made) == 1 and made[0]["tile"] is None and made[0]["max_radix"] == 0
+    stored.update(own=False, tile=[16, 8, 16], max_radix=16)
+    (tmp_path / "cache.json").write_text(json.dumps({key: stored}))
+    made.clear()
+    autotune.tuned_plan((64, 64, 64), (21, 21, 21), "linear", kernel)
+    assert len(made) == 1 and made[0]["tile"] == [16, 8, 16] and made[0]["max_radix"] == 16

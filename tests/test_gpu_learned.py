@@ -941,3 +941,35 @@ def test_reduce_rows_of_the_largest_extents(rows, cols):
               "pvd_reduce_rows")
     torch.cuda.synchronize()
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("nuclide", ["Y90", "Lu177"])
+@pytest.mark.parametrize("photons", [True, False])
+def test_monte_carlo_map_totals_and_both_tallies(nuclide, photons):
+    """The deposit map sums to the deposited energy, and the maps tallied in LDS (21^3) and in
+    memory (the same grid with three more planes along z, in which no electron can turn back)
+    agree voxel by voxel: the same histories, FP64 sums in another order (1e-12 of the maximum).
+    A map's terms are FP32 products (2^-24 each): totals to 1e-6."""
+    import torch
+    from pyvoxeldosimetry_amd.learned.mc import MonteCarlo
+    _say("mc tallies", nuclide, photons)
+    g = torch.Generator().manual_seed(8)
+    act, rho = torch.zeros((21, 21, 24)), 0.8 + 0.4 * torch.rand((21, 21, 24), generator=g)
+    act[6:15, 6:15, 6:15] = torch.rand((9, 9, 9), generator=g)      # 6 voxels of 4 mm from every face
+    maps = {}
+    for nz, histories in ((21, 37), (24, 37)):
+        mc = MonteCarlo(nuclide, photons=photons, photon_every=3)
+        e = mc.edep(act[..., :nz].contiguous().cuda(), rho[..., :nz].contiguous().cuda(), 4.0, histories, seed=7)
+        emitted, deposited, escaped = mc.last_totals.tolist()
+        assert float(e.sum()) == pytest.approx(deposited, rel=1e-6)
+        assert deposited + escaped == pytest.approx(emitted, rel=1e-6)
+        maps[nz] = e
+    diff = (maps[24][..., :21] - maps[21]).abs().max()
+    assert float(diff) <= 1e-12 * float(maps[21].max())
+    assert photons or float(maps[24][..., 21:].abs().max()) == 0.0
+    # a grid beyond the LDS tally whose electrons leave it on every side
+    mc = MonteCarlo(nuclide, photons=photons)
+    e = mc.edep(torch.rand((30, 25, 27), generator=g).cuda(), None, 0.7, 5, seed=2)
+    emitted, deposited, escaped = mc.last_totals.tolist()
+    assert escaped > 0 and float(e.sum()) == pytest.approx(deposited, rel=1e-6)
+    assert deposited + escaped == pytest.approx(emitted, rel=1e-5)

@@ -217,3 +217,30 @@ def test_prefilter_of_more_workgroups_than_one_launch_takes():
         part = prefilter(x[a:a + 4096].clone())
         lo, hi = (0 if a == 0 else 64), (4096 if a + 4096 == n else 4032)
         assert float((part[lo:hi] - coef[a + lo:a + hi]).abs().max()) <= 4e-6
+
+
+@pytest.mark.parametrize("mode", ["nearest", "linear", "cubic"])
+@pytest.mark.parametrize("m", [(410, 411, 409), (405, 406, 407)])
+def test_outputs_on_either_side_of_the_streaming_threshold(mode, m):
+    """Outputs above and below 256 MB (stored past the last-level cache, and through it): the
+    image is an outer product, so every output is the product of three one-dimensional
+    results.  FP32 interpolation along three axes on either side: 6e-6 of the largest
+    product (nearest: two roundings)."""
+    import torch
+    from pyvoxeldosimetry_amd.resample import resample_device
+    _say("streamed resample", mode, m)
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    n = (61, 70, 83)
+    f = [torch.randn(k, device="cuda", generator=gen) for k in n]
+    ratio = tuple(a / b for a, b in zip(n, m))
+    image = (f[0][:, None, None] * f[1][None, :, None] * f[2][None, None, :]).contiguous()
+    out = torch.full(m, float("nan"), device="cuda")
+    resample_device(image, (1.0,) * 3, ratio, mode, m, out=out)
+    one = []
+    for a in range(3):
+        shape, size, r = [1, 1, 1], [1, 1, 1], [1.0, 1.0, 1.0]
+        shape[a], size[a], r[a] = n[a], m[a], ratio[a]
+        one.append(resample_device(f[a].reshape(shape), (1.0,) * 3, r, mode, tuple(size)).reshape(-1))
+    want = one[0][:, None, None] * one[1][None, :, None] * one[2][None, None, :]
+    top = float(want.abs().max())
+    assert float((out - want).abs().max()) <= (2.0 ** -22 if mode == "nearest" else 6e-6) * top

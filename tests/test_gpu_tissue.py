@@ -185,3 +185,31 @@ def test_tissue_map_mostly_metal(shape, pattern, aligned):
     view.copy_(torch.from_numpy(ct))
     corr = TissueComposition().map(view)[0].cpu().numpy()
     np.testing.assert_allclose(corr, ot.handle_artifacts(ct), rtol=1e-6, atol=5e-4)
+
+
+def test_tissue_map_beyond_the_streaming_threshold():
+    """Outputs above 256 MB (stored past the last-level cache) against the two halves of the
+    volume with five planes more each, whose outputs are below it: bit for bit without metal,
+    the fills' FP64 sums in another order within the tolerance above."""
+    import torch
+    from pyvoxeldosimetry_amd.tissue import TissueComposition
+    _say("tissue streamed")
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    shape = (313, 317, 315)                                  # 31e6 voxels, n % 4 = 3
+    ct = torch.randn(shape, device="cuda", generator=gen) * 300.0
+    ct[100:200, 150:156, 100:104] = 3000.0
+    ct[:, 40, 50] = 2800.0
+    ct[torch.rand(shape, device="cuda", generator=gen) < 1e-4] = 2500.0
+    ct[-1, -1, -1] = 2600.0
+    tc = TissueComposition()
+    full = tc.map(ct)
+    for part, keep in ((slice(0, 162), slice(0, 157)), (slice(152, 313), slice(157, 313))):
+        half = tc.map(ct[part].contiguous())
+        lo = keep.start - part.start
+        c, b, d = (t[lo:lo + keep.stop - keep.start] for t in half)
+        C, B, D = (t[keep] for t in full)
+        metal = ct[keep] > 2000.0
+        same = C == c
+        assert bool((same | metal).all())
+        assert float(((C - c).abs() - 1e-6 * c.abs()).max()) <= 5e-4
+        assert torch.equal(B[same], b[same]) and torch.equal(D[same], d[same])

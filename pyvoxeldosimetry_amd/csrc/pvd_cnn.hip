@@ -1204,7 +1204,8 @@ __global__ __launch_bounds__(FWD_THREADS) void cnn_out_grad(MarchArgs q) {
             uint32_t f[4];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const uint32_t v = ring[((p + tdx[c][j]) & 3) * OG_PLANE + toff[c][j]];
+                // (zeros past the last tap: an infinite dr times a zero weight is not 0)
+                const uint32_t v = c * 16 + kh * 8 + j < 27 ? ring[((p + tdx[c][j]) & 3) * OG_PLANE + toff[c][j]] : 0u;
                 f[j >> 1] = j & 1 ? f[j >> 1] | v << 16 : v;
             }
             acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[c], frag4(f[0], f[1], f[2], f[3]), acc, 0, 0, 0);

@@ -973,3 +973,34 @@ def test_monte_carlo_map_totals_and_both_tallies(nuclide, photons):
     emitted, deposited, escaped = mc.last_totals.tolist()
     assert escaped > 0 and float(e.sum()) == pytest.approx(deposited, rel=1e-6)
     assert deposited + escaped == pytest.approx(emitted, rel=1e-5)
+
+
+def test_output_layer_gradient_of_an_infinite_dr():
+    """One infinite dL/dr reaches the 27 voxels around it as an infinity of the weight's sign, and
+    nothing as a NaN."""
+    import ctypes
+    import torch
+    from pyvoxeldosimetry_amd import _native as nat
+    _say("cnn out grad infinity")
+    lib = nat.load()
+    shape, at = (5, 9, 64), (2, 4, 30)
+    n = int(np.prod(shape))
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    g = torch.Generator(device="cuda").manual_seed(1)
+    w = torch.zeros((27, 32, 32), device="cuda", dtype=torch.bfloat16)
+    w[:, 0] = (torch.rand((27, 32), device="cuda", generator=g) + 0.5).to(torch.bfloat16)
+    w[::2, 0] *= -1
+    dr = torch.zeros(shape, device="cuda", dtype=torch.bfloat16)
+    dr[at] = float("inf")
+    mask = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+    dh = torch.empty((*shape, 32), device="cuda")
+    dz = torch.empty((n, 32), device="cuda", dtype=torch.bfloat16)
+    part = torch.empty((int(lib.pvd_cnn_out_grad_parts(*shape)), 32), device="cuda")
+    torch.cuda.synchronize()
+    nat.check(lib.pvd_cnn_out_grad(p(dr), p(w), p(dh), p(mask), p(dz), p(part), *shape, None), "pvd_cnn_out_grad")
+    torch.cuda.synchronize()
+    want = torch.zeros_like(dh)
+    for t in range(27):                                    # dh[v] = sum_t dr[v + d(t)] w[26 - t]
+        v = tuple(a - (t // 3 ** (2 - i) % 3 - 1) for i, a in enumerate(at))
+        want[v] = float("inf") * w[26 - t, 0].float().sign()
+    assert torch.equal(dh, want)

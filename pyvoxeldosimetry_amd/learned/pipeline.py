@@ -245,7 +245,7 @@ class LearnedCorrector:
         if e < 32:
             raise ValueError("tile_z must be at least 32")
         halo = 6
-        act, rho = act.contiguous(), rho.contiguous()
+        act, rho, dp = act.contiguous(), rho.contiguous(), dp.contiguous()
         amax, dmax = self.input_maxima(act, dp)
         r = torch.empty(shape, dtype=torch.float32, device=self.device)
         for s0, s1, a, b in z_slabs(nz, e, halo):

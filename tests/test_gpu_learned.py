@@ -1004,3 +1004,23 @@ def test_output_layer_gradient_of_an_infinite_dr():
         v = tuple(a - (t // 3 ** (2 - i) % 3 - 1) for i, a in enumerate(at))
         want[v] = float("inf") * w[26 - t, 0].float().sign()
     assert torch.equal(dh, want)
+
+
+def test_tiled_network_of_strided_maps():
+    """The slab-wise network on views: activity, density and plain dose of any strides give the
+    correction of their contiguous copies."""
+    import torch
+    from pyvoxeldosimetry_amd.learned.pipeline import LearnedCorrector, synth_phantom
+    _say("tiled network of views")
+    corr = LearnedCorrector.pretrained("Y90", 2.0)
+    act, rho = synth_phantom(7, (32, 40, 77), corr.device)
+    dp = corr.plain(act, rho)
+    view = lambda t: t.permute(2, 0, 1).contiguous().permute(1, 2, 0)  # noqa: E731
+    for region in (False, True):
+        want = corr.network_tiled(act, rho, dp, 32, region)[0].reshape(act.shape)
+        where = dp >= corr.region_frac * dp.max() if region else torch.ones_like(dp, dtype=torch.bool)
+        for k in range(3):
+            maps = [view(t) if i == k else t for i, t in enumerate((act, rho, dp))]
+            assert not maps[k].is_contiguous()
+            got = corr.network_tiled(*maps, 32, region)[0].reshape(act.shape)
+            assert torch.equal(got[where], want[where]), (region, k)

@@ -1367,32 +1367,32 @@ __global__ __launch_bounds__(256) void cnn_adam(float *p, const float *g, float 
 // the 256 x 27648 weight partials 61 us; both now take 4-6 us.)
 constexpr int RED_COLS = 32, RED_GROUPS = 32;
 constexpr int RED_GRID = 1 << 20;      // workgroups (at most; a launch has fewer than 2^32 threads)
-__global__ __launch_bounds__(RED_COLS * RED_GROUPS) void reduce_rows(const float *__restrict__ part, int rows, int cols,
-                                                                     float *__restrict__ out, int accumulate,
-                                                                     int pitch) {
+__global__ __launch_bounds__(RED_COLS * RED_GROUPS) void reduce_rows(const float *__restrict__ part, unsigned rows,
+                                                                     unsigned cols, float *__restrict__ out,
+                                                                     int accumulate, int pitch) {
     __shared__ float red[RED_GROUPS][RED_COLS + 1];
-    const int l = threadIdx.x & (RED_COLS - 1), g = threadIdx.x / RED_COLS;
-    for (long long b = blockIdx.x; b * RED_COLS < cols; b += gridDim.x) {
-        const long long c = b * RED_COLS + l;
+    const unsigned l = threadIdx.x & (RED_COLS - 1), g = threadIdx.x / RED_COLS;
+    for (unsigned b = blockIdx.x; b * RED_COLS < cols; b += gridDim.x) {       // (rows, cols < 2^31)
+        const unsigned c = b * RED_COLS + l;
         const float *p = part + (c < cols ? c : cols - 1);
         float s = 0.0f;
-        for (long long r0 = g; r0 < rows; r0 += 8 * RED_GROUPS) {
+        for (unsigned r0 = g; r0 < rows; r0 += 8 * RED_GROUPS) {
             float v[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = p[(size_t)min(r0 + u * RED_GROUPS, rows - 1LL) * cols];
+            for (int u = 0; u < 8; ++u) v[u] = p[(size_t)min(r0 + u * RED_GROUPS, rows - 1) * cols];
 #pragma unroll
             for (int u = 0; u < 8; ++u) s += r0 + u * RED_GROUPS < rows ? v[u] : 0.0f;
         }
+        if (b != blockIdx.x) __syncthreads();                                  // red is free again
         red[g][l] = s;
         __syncthreads();
 #pragma unroll
         for (int h = RED_GROUPS / 2; h > 0; h >>= 1) {
-            if (g < h) red[g][l] += red[g + h][l];
+            if (g < (unsigned)h) red[g][l] += red[g + h][l];
             __syncthreads();
         }
         float *o = out + (size_t)b * pitch + l;                  // `pitch` floats per 32 columns
         if (g == 0 && c < cols) *o = accumulate ? *o + red[0][l] : red[0][l];
-        __syncthreads();
     }
 }
 

@@ -482,23 +482,25 @@ def cnn_measure(dev, steps: int, warmup: int, eval_seeds=None, eval_shape=(64, 6
     dp = corr.plain(act, rho)
     region_blocks = corr.region_blocks(dp, dp.max().reshape(1), corr.region_frac)[1].item()
     all_blocks = int(corr.lib.pvd_cnn_region_block_count(*shape))
-    x, _ = corr.pack(act, rho, corr.plain(act, rho))
+    # the network as `correct` runs it: the input layer from the FP32 maps
+    amax, dmax = corr.input_maxima(act, dp)
+    maps = (act, rho, dp, amax, dmax, shape[2])
     ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     reps = 20
-    corr.net.forward(x, shape, keep_activations=False)
+    corr.net.forward(None, shape, keep_activations=False, maps=maps)
     ev0.record()
     for _ in range(reps):
-        corr.net.forward(x, shape, keep_activations=False)
+        corr.net.forward(None, shape, keep_activations=False, maps=maps)
     ev1.record()
     torch.cuda.synchronize()
     ms_net = ev0.elapsed_time(ev1) / reps
     n = int(np.prod(shape))
     alg = 2.0 * 27 * (3 * 32 + 4 * 32 * 32 + 32 * 1) * n          # useful MACs x 2 (3 in, 32 hidden, 1 out)
     # as issued on the matrix cores: input layer 7 MFMAs (4 taps x 4 channels each) per 32
-    # voxels x 32 channels, residual layers 27 taps x 32 x 32, output layer 26 x 2 MFMAs of
-    # halo voxels x 32 tap columns per block of 256 voxels (SQ_INSTS_VALU_MFMA_MOPS_BF16
-    # gives the same per-voxel figures)
-    executed = (2.0 * 7 * 16 * 32 + 4 * 2.0 * 27 * 32 * 32 + 26 * 2 * 32768 / 256) * n
+    # voxels x 32 channels, residual layers 27 taps x 32 x 32, output layer 11 groups x 2 MFMAs
+    # of 32 halo voxels x 32 tap columns per 256 voxels of a plane, in segments of 16 planes
+    # with one more at either end
+    executed = (2.0 * 7 * 16 * 32 + 4 * 2.0 * 27 * 32 * 32 + 11 * 2 * 32768 / 256 * 18 / 16) * n
     ev = None if eval_seeds is None else evaluate(corr, eval_seeds, eval_shape, histories=histories)
     return {"corr": corr, "ms_plain": ms_plain, "ms_corr": ms_corr, "ms_net": ms_net, "alg_flops": alg,
             "executed_flops": executed, "eval": ev, "act": act, "ms_corr_region": ms_corr_region,
@@ -534,7 +536,7 @@ def bench_cnn(args):
                         "executed_TFLOPs": round(executed / (ms_net * 1e-3) / 1e12, 1),
                         "executed_frac": round(executed / (ms_net * 1e-3) / 1e12 / peak, 4),
                         "traffic": read_traffic("cnn_forward_6_launches", "cnn_forward_128cubed.md"),
-                        "kernel": "cnn_conv_fwd (6 launches)", "kernel_ms": round(ms_net, 5),
+                        "kernel": "cnn_conv_in, 4 cnn_conv_march, cnn_conv_out_march", "kernel_ms": round(ms_net, 5),
                         "algorithmic_flops": alg},
            "error_vs_monte_carlo_64cubed": m["eval"]}
     if not args.no_cpu:
@@ -680,7 +682,7 @@ def bench_resample(args):
            "roofline": {"bound": "hbm", "achieved": round(alg / (k_ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS,
                         "unit": "GB/s", "frac": round(alg / (k_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                         "traffic": read_traffic("resample_kernel_coarse_to_fine", "resample_512x512x400.md"),
-                        "kernel": "resample_kernel (coarse -> fine)", "kernel_ms": round(k_ms, 5),
+                        "kernel": "resample_linear (coarse -> fine)", "kernel_ms": round(k_ms, 5),
                         "algorithmic_bytes": alg}}
     if not args.no_cpu:
         from oracle import resample as ors

@@ -42,7 +42,7 @@ __device__ __forceinline__ void bspline3_weights(float t, float w[4]) {
 }
 
 // An output: stored past the last-level cache where the whole output is larger than it.
-// 512x512x400 linear 124 -> 98 us, 512x512x512 nearest 285 -> 206, cubic 309 -> 273; 333x333x333
+// 512x512x400 linear 124 -> 83-98 us, 512x512x512 nearest 285 -> 206, cubic 309 -> 273; 333x333x333
 // (148 MB) would take 54 us instead of 43.
 template <bool NT>
 __device__ __forceinline__ void put(float *p, float v) {
@@ -163,8 +163,8 @@ __global__ __launch_bounds__(256) void resample_kernel(ResampleArgs a) {
 // The gather form above issues 8 (linear) or 64 (cubic) loads per output and is bound
 // by them; here a tile costs W loads per input element it spans, so the cost follows
 // the input samples per output and the pass goes to the HBM stores.  Gather -> staged:
-// 251x251x196 -> 512x512x400 linear 321 -> 98 us (88 at the copy rate), cubic 2139 ->
-// 209; 301x301x233 -> 206x206x160 linear 51 -> 25 us, cubic 283 -> 41 (22).
+// 251x251x196 -> 512x512x400 linear 321 -> 83-98 us by box (88 at the copy rate), cubic 2139
+// -> 209; 301x301x233 -> 206x206x160 linear 51 -> 25 us, cubic 283 -> 41 (22).
 constexpr int kRsBlock = 256;      // threads
 constexpr int kRsU = 5;            // linear: columns per lane in flight in step 1
 constexpr int kRsSpan = 64 * kRsU; // input columns of a tile (at most)
@@ -191,8 +191,8 @@ constexpr long long kRsGrid = 1 << 21;
 // wave issue rate bound the tile-per-output-plane form (an FP64 coordinate, a row lookup and
 // a branch per output): a workgroup now keeps a lane's z positions over kRsPlanes output
 // planes and gives each wave whole rows, about 12 instructions an output.
-// 251x251x196 -> 512x512x400 150 -> 126 us (94 at the copy rate), 400x300x350 -> half 32.6
-// -> 29.7; eight planes a workgroup with 64 VGPRs 170.
+// 251x251x196 -> 512x512x400, through the cache, 150 -> 124 us (past it 83-98), 400x300x350 ->
+// half 32.6 -> 29.7; eight planes a workgroup with 64 VGPRs 170.
 template <bool NT>
 __global__ __launch_bounds__(kRsBlock) void resample_linear(StagedArgs q) {
     extern __shared__ float rs_lds[];

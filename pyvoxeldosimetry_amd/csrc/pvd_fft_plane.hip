@@ -177,8 +177,15 @@ __device__ __forceinline__ plane_ctx plane_context(const pvd_vol_d &v, float2 *s
     return c;
 }
 
-constexpr int kPlTp = 32;      // threads per line pair of the loads and the epilogue
 constexpr int kPlB = 4;        // elements per line in flight per thread
+
+// log2 of the threads per line pair of the loads and the epilogue: one round of kPlB elements a
+// thread, a wave at most.  (32 for every length left most of them idle on short lines and took
+// long ones round after round: 15x115x12, T = 3 44.5 -> 29.0 us, 295x22x527 96.0 -> 90.1, 817
+// volumes 2.4 % on average; a volume of a few hundred voxels pays 0.4 us.)
+__device__ __forceinline__ int pair_threads(int len) {
+    return len <= 16 ? 2 : len <= 32 ? 3 : len <= 64 ? 4 : len <= 128 ? 5 : 6;
+}
 
 template <int G>
 __global__ __launch_bounds__(1024) void pvd_fft_plane_zy(pvd_vol_d v) {
@@ -190,11 +197,12 @@ __global__ __launch_bounds__(1024) void pvd_fft_plane_zy(pvd_vol_d v) {
     load_twiddles(twz, az);
     load_twiddles(twy, ay);
     const long long p0 = (long long)blockIdx.x * G * c.Ny * Nz;        // the first plane's first voxel
-    for (int w = threadIdx.x; w < npair * kPlTp; w += blockDim.x) {
-        const int q = w / kPlTp, t = w % kPlTp;
+    const int ltp = pair_threads(c.Pz), tp = 1 << ltp;
+    for (int w = threadIdx.x; w < npair << ltp; w += blockDim.x) {
+        const int q = w >> ltp, t = w & (tp - 1);
         const bool h1 = 2 * q + 1 < c.nreal;
         const uint32_t o0 = (uint32_t)(2 * q * Nz);
-        for (int z0 = t; z0 < c.Pz; z0 += kPlTp * kPlB) {
+        for (int z0 = t; z0 < c.Pz; z0 += tp * kPlB) {
             float2 a[kPlB];
             for (int tt = 0; tt < v.T; ++tt) {
                 const float *m = v.act[tt] + p0;
@@ -202,7 +210,7 @@ __global__ __launch_bounds__(1024) void pvd_fft_plane_zy(pvd_vol_d v) {
                 float xa[kPlB], xb[kPlB];                            // issued together, masked afterwards
 #pragma unroll
                 for (int u = 0; u < kPlB; ++u) {
-                    const int z = z0 + kPlTp * u;
+                    const int z = z0 + tp * u;
                     xa[u] = at(m, (z < Nz ? o0 + z : 0u) * 4u);
                     xb[u] = at(m, ((z < Nz && h1) ? o0 + Nz + z : 0u) * 4u);
                 }
@@ -214,7 +222,7 @@ __global__ __launch_bounds__(1024) void pvd_fft_plane_zy(pvd_vol_d v) {
             }
 #pragma unroll
             for (int u = 0; u < kPlB; ++u) {
-                const int z = z0 + kPlTp * u;
+                const int z = z0 + tp * u;
                 if (z < c.Pz) s[z * c.ldz + q] = make_float2(z < Nz ? a[u].x : 0.f, z < Nz && h1 ? a[u].y : 0.f);
             }
         }
@@ -248,21 +256,22 @@ __global__ __launch_bounds__(1024) void pvd_fft_plane_yz(pvd_vol_d v) {
     const long long p0 = (long long)blockIdx.x * G * c.Ny * Nz;
     const bool has_dens = v.dens != nullptr;
     const float sc = v.scale;
-    for (int w = threadIdx.x; w < npair * kPlTp; w += blockDim.x) {
-        const int q = w / kPlTp, t = w % kPlTp;
+    const int ltp = pair_threads(Nz), tp = 1 << ltp;
+    for (int w = threadIdx.x; w < npair << ltp; w += blockDim.x) {
+        const int q = w >> ltp, t = w & (tp - 1);
         const bool h1 = 2 * q + 1 < c.nreal;
         const long long o0 = p0 + 2LL * q * Nz;
-        for (int z0 = t; z0 < Nz; z0 += kPlTp * kPlB) {
+        for (int z0 = t; z0 < Nz; z0 += tp * kPlB) {
             float2 d[kPlB];
 #pragma unroll
             for (int u = 0; u < kPlB; ++u) {
-                const int o = z0 + kPlTp * u;
+                const int o = z0 + tp * u;
                 d[u].x = (has_dens && o < Nz) ? gmem(v.dens)[o0 + o] : 1.f;
                 d[u].y = (has_dens && o < Nz && h1) ? gmem(v.dens)[o0 + Nz + o] : 1.f;
             }
 #pragma unroll
             for (int u = 0; u < kPlB; ++u) {
-                const int o = z0 + kPlTp * u;
+                const int o = z0 + tp * u;
                 if (o >= Nz) continue;
                 float2 val = s[wrap_add(o, az.off, c.Pz) * c.ldz + q];
                 if (o < az.foldn) {

@@ -350,10 +350,19 @@ bool x_offsets_fit(long long Nx, long long Px, long long Py, long long Hp, long 
 // lies between z lines of 64 points at 1772 waves (75.6 -> 69.3 with 8) and of 125 points
 // at 2500 (89.3, 90.5 with 8).  In a batch of sixteen 64^3 volumes 16 lines take 103 us and
 // small tiles 131, of four 74 and 65.
-constexpr double kFewWaves = 2048;
+// A tile of few elements is one wavefront with little to do: halving it gains nothing and
+// narrows the rows it reads.  x and y tiles of at most 128 elements stay whole, of at most 320
+// where the pass has 256 waves (of 500 random volumes 24 were up to 10 % slower with 4 columns
+// of 3 to 20 points than with 16, e.g. 15x181x134 31.7 -> 35.0 us; with this rule none by more than
+// 2.7 %, and the mean gain stays, 4.0 %).  For y the wave count that pays is kFewWavesY:
+// with 512 to 2048 waves of 16 columns 8 were 2 to 10 % slower (182x36x238 53.5 -> 61.4), below
+// 256 2 to 4 % faster, up to 10 %.
+constexpr double kFewWaves = 2048, kFewWavesY = 512;
 template <typename Tiles>
-int few_waves_tile(int n, int lines, int least, double share, Tiles tiles) {
-    while (lines > least && share * tiles(lines) * ((lines * n + 1023) / 1024) < kFewWaves) lines /= 2;
+int few_waves_tile(int n, int lines, int least, double few, bool wide_rows, double share, Tiles tiles) {
+    auto waves = [&](int l) { return share * tiles(l) * ((l * n + 1023) / 1024); };
+    const int elems = !wide_rows ? 0 : waves(lines) < 256 ? 128 : 320;
+    while (lines > least && lines * n > elems && waves(lines) < few) lines /= 2;
     return lines;
 }
 
@@ -361,9 +370,10 @@ int few_waves_tile(int n, int lines, int least, double share, Tiles tiles) {
 // and y transforms are Stockham stages whose tiles the plan chooses and a workgroup holds
 // the plane (two planes with an odd Ny, so that the line pairs stay those of the five
 // passes) at PVD_PLANE_PER elements a thread: 8192, 16 would spill.  Five passes -> plane
-// form, whole calls in us: 64^3 35.4 -> 27.7, 100^3 58.3 -> 47.3, 30x80x80 42.5 -> 35.2,
-// 512x64x64 65.2 -> 39.0, 400x63x100 77.4 -> 49.6, 500x126x126 122 -> 120.  The line on the
-// odd side: 31x63x126 (16 workgroups of 1024 threads) 46.9 -> 48.8, 200x63x125 64.7 -> 46.8.
+// form, whole calls in us (21^3 kernel, circular): 64^3 35.5 -> 26.3, 72x72x50 44.2 -> 36.2, 100^3
+// 56.3 -> 46.0, 512x64x64 64.3 -> 38.1, 400x63x100 76.5 -> 49.2, 500x126x126 121 -> 117; 817 random
+// volumes 10.6 % on average, the slowest of them 4 % slower.  The line on the odd side:
+// 31x63x126 (16 workgroups of 1024 threads) 46.9 -> 48.8 (13^3 kernel), 200x63x125 58.0 -> 47.0.
 void plane_layout(pvd_plan *p, bool regs) {
     const pvd_vol_d &v = p->vol;
     p->plane = launch_cfg();
@@ -397,7 +407,7 @@ int fft_layout(pvd_plan *p) {
     int lz, bz; size_t ldsz;
     pick_tile(Pz, p->tile[2], 1, &lz, &bz, &ldsz);
     if (p->prm.tile[2] == 0 && regs && !z_reg_code(Pz))
-        pick_tile(Pz, few_waves_tile(Pz, lz, 4, p->share[2], z_tiles), 1, &lz, &bz, &ldsz);
+        pick_tile(Pz, few_waves_tile(Pz, lz, 4, kFewWaves, false, p->share[2], z_tiles), 1, &lz, &bz, &ldsz);
     // z blocks are a power-of-two multiple of the lines per tile, so the z passes'
     // I/O phases (blockDim / lines threads per line pair) keep every thread busy
     // (at most 1024: both factors are powers of two)
@@ -407,7 +417,7 @@ int fft_layout(pvd_plan *p) {
     // y: whole 128-byte lines of 16 columns are worth more than waves (80x100x60 45.2 us, with
     // 8-column y tiles 46.8) except where they make one wavefront (64^3 37.4, with 8 35.7)
     if (p->prm.tile[1] == 0 && regs && !xy_two_step_len(Py) && tky * Py <= 1024)
-        pick_tile(Py, few_waves_tile(Py, tky, 8, p->share[1], y_tiles), 0, &tky, &by, &ldsy);
+        pick_tile(Py, few_waves_tile(Py, tky, 8, kFewWavesY, true, p->share[1], y_tiles), 0, &tky, &by, &ldsy);
     // x tile left to the plan: 8 columns for the fused two-step lengths 16 * B with
     // B >= 18 (the X pass holds a column's two transforms and its spectrum values in
     // registers there, and half-width tiles fit more workgroups per CU)
@@ -416,7 +426,7 @@ int fft_layout(pvd_plan *p) {
     int tkx, bx; size_t ldsx;
     pick_tile(Px, tile_x, 0, &tkx, &bx, &ldsx);
     if (p->prm.tile[0] == 0 && regs && !xy_two_step_len(Px))
-        pick_tile(Px, few_waves_tile(Px, tkx, 4, p->share[0], x_tiles), 0, &tkx, &bx, &ldsx);
+        pick_tile(Px, few_waves_tile(Px, tkx, 4, kFewWaves, true, p->share[0], x_tiles), 0, &tkx, &bx, &ldsx);
     // y/x register paths: 1 = the 256-point path (16-line tiles, no reference-mode fold;
     // checked again in the kernel); 2 = the two-step P = 16 * rb (rb in kXyRegB) in its
     // own kernel instances

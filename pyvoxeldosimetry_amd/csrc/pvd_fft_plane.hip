@@ -2,10 +2,10 @@
 // one launch each way.  A plane of a small volume (Ny * Pz/2 complex) fits the LDS of one
 // workgroup, so FZ + FY and IY + IZ keep it there: two launches and two round trips of the
 // half spectrum through memory less.  A small dose call is bound by the latency of its
-// launches, not by bytes or operations: 64^3 35.4 -> 27.7 us (ZY 10.7, X 9.2, YZ 9.6 in a
-// trace; the five passes 7.6, 6.2, 9.6, 6.0, 7.2), 512x64x64 65.2 -> 39.0.  Radix-16 stages
-// are left out: with the split or merge they spilled 45-150 VGPRs and cost more than the
-// launches (64^3 37.8).
+// launches, not by bytes or operations: 64^3 35.5 -> 26.3 us (three launches of 9 to 10 us in a
+// trace, the five passes 6 to 10 each), 512x64x64 64.3 -> 38.1.  Radix-16 stages are left out:
+// with the split or merge they spilled 45-150 VGPRs and cost more than the launches (64^3
+// 37.8 then).
 //   ZY  load the T weighted maps, z transform of the line pairs, split, y transform, store
 //   YZ  load, inverse y transform (roll / fold), merge, inverse z transform, epilogue
 // The stages are the Stockham stages of fft_lines (same radices, twiddles and order of the

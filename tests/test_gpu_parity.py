@@ -565,3 +565,27 @@ def test_plane_passes_give_the_bits_of_the_five_passes(shape, kshape, mode):
     assert_parity(got, scale * ref / dens.astype(np.float64), what=f"plane {shape} {mode}")
     plan.close()
     five.close()
+
+
+@pytest.mark.parametrize("nz", [15, 16, 18, 32, 35, 63, 64, 70, 126, 128, 135, 256, 270])
+@pytest.mark.parametrize("ny,mode", [(6, "linear"), (7, "reference")])
+def test_plane_passes_of_short_and_long_lines(nz, ny, mode):
+    """The threads per line pair follow the line's length (steps at 16, 32, 64 and 128 points of
+    the padded and of the stored line): the bits of the five passes, and the oracle's dose."""
+    from pyvoxeldosimetry_amd import ConvPlan
+    _say("plane line lengths", nz, ny, mode)
+    shape, kshape = (5, ny, nz), (3, 3, 1)
+    rng = np.random.default_rng(nz)
+    a = rng.random(shape).astype(np.float32)
+    dens = rng.uniform(0.3, 1.9, shape).astype(np.float32)
+    k = rng.random(kshape)
+    plan = ConvPlan(shape, kshape, mode=mode, algo="fft")
+    plan.set_kernel(k)
+    five = ConvPlan(shape, kshape, mode=mode, algo="fft", tile=plan.tile, max_radix=plan.max_radix)
+    five.set_kernel(k)
+    got = plan.dose(dev_tensor(a), density=dev_tensor(dens)).cpu().numpy()
+    assert np.array_equal(got, five.dose(dev_tensor(a), density=dev_tensor(dens)).cpu().numpy())
+    ref = (conv.ref_conv if mode == "reference" else conv.linear_same)(a.astype(np.float64), k)
+    assert_parity(got, ref / dens.astype(np.float64), what=f"plane lines {shape} {mode}")
+    plan.close()
+    five.close()

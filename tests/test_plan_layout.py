@@ -143,3 +143,15 @@ def test_small_volumes_take_small_tiles_of_the_stockham_passes(shape, tile, radi
     assert (kept["tile"], kept["max_radix"]) == ((16, 16, 16), 16)
     old = describe_plan(shape, (11, 11, 11), "reference", algo="fft", stockham=True)
     assert (old["tile"], old["max_radix"]) == ((16, 16, 16), 16)
+
+
+@pytest.mark.parametrize("shape,k,mode,tile", [
+    ((182, 36, 238), 31, "reference", (16, 16, 16)),     # 1820 waves of y tiles: past the 512 that halving pays for
+    ((140, 59, 202), 7, "linear", (16, 16, 16)),
+    ((98, 43, 45), 3, "linear", (4, 8, 4)),              # 196 waves
+    ((15, 181, 134), 3, "linear", (16, 16, 16)),         # x columns of 16 points in 960 waves stay whole
+    ((8, 10, 12), 3, "linear", (8, 8, 4)),               # few waves: down to 128 elements
+])
+def test_tiles_that_halving_would_slow_down_stay_whole(shape, k, mode, tile):
+    d = describe_plan(shape, (k,) * 3, mode, algo="fft")
+    assert d["tile"] == tile, d

@@ -535,10 +535,10 @@ constexpr int kBsZ = 27;           // outputs per unit along z (odd: neighbourin
 constexpr int kBsCols = 17 * kBsZ + 2 * kBsK;      // columns of a z tile (at most): 487
 
 __global__ __launch_bounds__(256) void bspline_x(const float *__restrict__ src, float *__restrict__ dst, int n0,
-                                                 long long plane, long long gx, long long first) {
-    const long long b = first + blockIdx.x;
-    const long long p = b % gx * 256LL + threadIdx.x;
-    const int x0 = (int)(b / gx) * kBsX;
+                                                 long long plane, unsigned gx, unsigned first) {
+    const unsigned b = first + blockIdx.x, bx = b / gx;
+    const long long p = (b - bx * gx) * 256LL + threadIdx.x;
+    const int x0 = (int)bx * kBsX;
     const long long pc = p < plane ? p : plane - 1;
     float c[kBsX];
     bs_line([&](int i) { return src[(long long)mirror_index(min(x0 + i - kBsK, n0 - 1 + kBsK), n0) * plane + pc]; }, c);
@@ -595,6 +595,7 @@ extern "C" int pvd_bspline_prefilter(const float *in, int n0, int n1, int n2, fl
     if (coef == in || tmp == in || coef == tmp) return pvd_set_error(PVD_EINVAL, "coef, tmp and in must differ");
     const long long plane = (long long)n1 * n2;
     const long long gx = (plane + 255) / 256, blocks_x = gx * ((n0 + (long long)kBsX - 1) / kBsX);
+    if (blocks_x > 0xffffffffLL) return pvd_set_error(PVD_ENOTSUP, "grid too large");     // 4e12 bytes and more
     const int nyt = (n1 + kBsY - 1) / kBsY;
     // z tiles of equal width, a multiple of the unit; a thread per column
     const int nt = (n2 + kBsCols - 2 * kBsK - 1) / (kBsCols - 2 * kBsK);
@@ -605,7 +606,7 @@ extern "C" int pvd_bspline_prefilter(const float *in, int n0, int n1, int n2, fl
     hipError_t e = hipSuccess;
     for (long long first = 0; first < blocks_x; first += kRsGrid) {
         hipLaunchKernelGGL(bspline_x, dim3((unsigned)std::min(blocks_x - first, kRsGrid)), dim3(256), 0, st, in, tmp, n0,
-                           plane, gx, first);
+                           plane, (unsigned)gx, (unsigned)first);
         e = hipGetLastError();
         if (e != hipSuccess) return pvd_hip_error(e, "launch B-spline prefilter");
     }
